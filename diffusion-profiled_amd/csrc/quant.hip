@@ -165,6 +165,25 @@ __global__ __launch_bounds__(kQThreads) void cast_with_wprep_kernel(
   else cast_current_block<true>(x, n, partials, np, q, scale_out, blockIdx.x - wb, nb);
 }
 
+// The same two launches for one weight whose entry travels in the kernel arguments: an op
+// call has no device table to keep it in.
+template <bool kVec>
+__global__ __launch_bounds__(kQThreads) void amax_with_weight_kernel(
+    const uint16_t* __restrict__ x, int64_t n, uint32_t* __restrict__ partials, int nb,
+    const DpaWeightEntry e, uint32_t* __restrict__ wpart) {
+  if ((int)blockIdx.x < e.nblk) wprep_amax_tile(e, wpart, blockIdx.x);
+  else amax_partials_block<kVec>(x, n, partials, blockIdx.x - e.nblk, nb);
+}
+
+template <bool kVec>
+__global__ __launch_bounds__(kQThreads) void cast_with_weight_kernel(
+    const uint16_t* __restrict__ x, int64_t n, const uint32_t* __restrict__ partials, int np,
+    uint8_t* __restrict__ q, float* __restrict__ scale_out, int nb, const DpaWeightEntry e,
+    const uint32_t* __restrict__ wpart) {
+  if ((int)blockIdx.x < e.nblk) wprep_cast_tile(e, wpart, blockIdx.x);
+  else cast_current_block<kVec>(x, n, partials, np, q, scale_out, blockIdx.x - e.nblk, nb);
+}
+
 // Delayed scaling, one pass: q = cast(x, *prev_scale) and per-block amax of x. count (if
 // given) receives the number of partials, for a finalize in a later launch.
 template <bool kVec>
@@ -413,6 +432,65 @@ extern "C" int dpa_quantize_fp8_bf16_with_weight_prep(
   if (st != DPA_OK) return st;
   cast_with_wprep_kernel<<<(unsigned)(total_blocks + gc), kQThreads, 0, s>>>(
       xp, n, part, np, (uint8_t*)q, scale_out, gc, entries_dev, count, wpart, total_blocks);
+  return launch_status();
+}
+
+// Current scaling of the two operands of one FP8 product: x as dpa_quantize_fp8_bf16, and its
+// weight w [cout][taps][cin] (fp32, rounded to bf16 as it is read, or bf16) into wq and the
+// data-gradient copy wqt, as one entry of a weight preparation would be. Two launches: the
+// weight's blocks are the first of each. Quantizing a layer's x and w apart and transposing the
+// weight in the backward took seven (bf16 cast, 2 + 2 quantization, fragment or transpose
+// copies, the cast of the bf16 weight gradient), each ~4.5 us for a tensor of at most a few MB:
+// the 3x3 128 -> 128 conv at 32x32, batch 128, forward and both gradients: 129.1 -> 105.9 us.
+extern "C" int64_t dpa_quantize_with_weight_workspace_bytes(int cout, int taps, int cin) {
+  if (cout <= 0 || taps <= 0 || cin <= 0) return 0;
+  return (int64_t)kMaxPartials * 4 +
+         ceil_div(cout, kWpTile) * taps * ceil_div(cin, kWpTile) * 4;
+}
+
+extern "C" int dpa_quantize_fp8_bf16_with_weight(
+    const void* x, int64_t n, void* q, float* scale_out, const void* w, int flags, int cout,
+    int taps, int cin, void* wq, void* wqt, float* w_scale, void* workspace,
+    int64_t workspace_bytes, void* stream) {
+  if (!x || !q || !scale_out) return DPA_ERR_NULL;
+  if (n <= 0 || cout <= 0 || taps <= 0 || cin <= 0) return DPA_ERR_SIZE;
+  DpaWeightEntry e{};
+  e.w = (const float*)w;
+  e.q = wq;
+  e.qt = wqt;
+  e.scale_used = w_scale;
+  e.n = (int64_t)cout * taps * cin;
+  e.cout = cout; e.taps = taps; e.cin = cin;
+  e.flags = flags & (DPA_WP_BF16 | DPA_WP_FRAG);
+  const int wb = dpa_weight_prep_plan(&e, 1);
+  if (wb < 0) return wb;
+  if (!workspace ||
+      workspace_bytes < dpa_quantize_with_weight_workspace_bytes(cout, taps, cin))
+    return DPA_ERR_WORKSPACE;
+  if (!aligned(workspace, 4) || !aligned(scale_out, 4) || !aligned(w_scale, 4) ||
+      !aligned(x, 2) || !aligned(wqt, 8))
+    return DPA_ERR_ALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  const bool vec = aligned(x, 16) && aligned(q, 8);
+  const int np = vec ? grid_for(n, kAmaxBlocks) : 1;
+  const int gc = vec ? grid_for(n, kCastBlocks) : 1;
+  auto* xp = (const uint16_t*)x;
+  auto* part = (uint32_t*)workspace;
+  uint32_t* wpart = part + kMaxPartials;
+  if (vec)
+    amax_with_weight_kernel<true><<<(unsigned)(wb + np), kQThreads, 0, s>>>(xp, n, part, np, e,
+                                                                            wpart);
+  else
+    amax_with_weight_kernel<false><<<(unsigned)(wb + np), kQThreads, 0, s>>>(xp, n, part, np, e,
+                                                                             wpart);
+  const int st = launch_status();
+  if (st != DPA_OK) return st;
+  if (vec)
+    cast_with_weight_kernel<true><<<(unsigned)(wb + gc), kQThreads, 0, s>>>(
+        xp, n, part, np, (uint8_t*)q, scale_out, gc, e, wpart);
+  else
+    cast_with_weight_kernel<false><<<(unsigned)(wb + gc), kQThreads, 0, s>>>(
+        xp, n, part, np, (uint8_t*)q, scale_out, gc, e, wpart);
   return launch_status();
 }
 

@@ -81,14 +81,11 @@ __device__ __forceinline__ uint32_t wp_block_max(uint32_t v, uint32_t* red) {
   return r;
 }
 
-// Block b of the amax pass: the maximum of |bf16(w)| over its tile, into partials[b].
-__device__ __forceinline__ void wprep_amax_block(const DpaWeightEntry* __restrict__ e, int count,
-                                                 uint32_t* __restrict__ partials, int b) {
+// Block b of the amax pass, one of entry E's: the maximum of |bf16(w)| over its tile, into
+// partials[b].
+__device__ __forceinline__ void wprep_amax_tile(const DpaWeightEntry& E,
+                                                uint32_t* __restrict__ partials, int b) {
   __shared__ uint32_t red[kWpThreads / 64];
-  __shared__ int s_t;
-  if (threadIdx.x == 0) s_t = wp_entry_of(e, count, b);
-  __syncthreads();
-  const DpaWeightEntry& E = e[s_t];
   const WpTile T = wp_tile(E, b - E.blk0);
   us2 acc = {0, 0};
 #pragma unroll
@@ -101,16 +98,21 @@ __device__ __forceinline__ void wprep_amax_block(const DpaWeightEntry* __restric
   if (threadIdx.x == 0) partials[b] = m;
 }
 
-// Cast of one tile: q rows out directly (64 B per row), the transposed copy through an LDS
-// tile so that its rows (64 output channels of one input channel) leave as 64-B runs too.
-__device__ __forceinline__ void wprep_cast_block(const DpaWeightEntry* __restrict__ e, int count,
-                                                 const uint32_t* __restrict__ partials, int b) {
-  __shared__ uint32_t red[kWpThreads / 64];
-  __shared__ uint32_t tile[kWpTile][kWpTile / 4 + 1];  // [co row][ci / 4], padded
+__device__ __forceinline__ void wprep_amax_block(const DpaWeightEntry* __restrict__ e, int count,
+                                                 uint32_t* __restrict__ partials, int b) {
   __shared__ int s_t;
   if (threadIdx.x == 0) s_t = wp_entry_of(e, count, b);
   __syncthreads();
-  const DpaWeightEntry& E = e[s_t];
+  wprep_amax_tile(e[s_t], partials, b);
+}
+
+// Cast of one tile (block b, one of entry E's): q rows out directly (64 B per row), the
+// transposed copy through an LDS tile so that its rows (64 output channels of one input
+// channel) leave as 64-B runs too.
+__device__ __forceinline__ void wprep_cast_tile(const DpaWeightEntry& E,
+                                                const uint32_t* __restrict__ partials, int b) {
+  __shared__ uint32_t red[kWpThreads / 64];
+  __shared__ uint32_t tile[kWpTile][kWpTile / 4 + 1];  // [co row][ci / 4], padded
   const WpTile T = wp_tile(E, b - E.blk0);
   uint4 v[2];
   bool ok[2];
@@ -176,6 +178,14 @@ __device__ __forceinline__ void wprep_cast_block(const DpaWeightEntry* __restric
       for (int j = 0; j < 4 && co + j < E.cout; ++j) dst[j] = (uint8_t)(w >> (8 * j));
     }
   }
+}
+
+__device__ __forceinline__ void wprep_cast_block(const DpaWeightEntry* __restrict__ e, int count,
+                                                 const uint32_t* __restrict__ partials, int b) {
+  __shared__ int s_t;
+  if (threadIdx.x == 0) s_t = wp_entry_of(e, count, b);
+  __syncthreads();
+  wprep_cast_tile(e[s_t], partials, b);
 }
 
 }  // namespace dpa

@@ -141,6 +141,39 @@ def _quantize_impl(tensor: torch.Tensor, prev_scale: torch.Tensor | None) -> tup
     return quantized, scale
 
 
+def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool):
+    """Both operands of one FP8 product in two launches (dpa_quantize_fp8_bf16_with_weight):
+    (x e4m3, x scale, w e4m3, its data-gradient copy, w scale), the bytes and scales of
+    quantize_fp8 of x and of the bf16 weight. weight: fp32 or bf16, [Cout, Cin, k, k] or [N, K].
+    The weight's copies are the OHWI / [N][K] bytes and their [Cin][k][k][Cout] / [K][N]
+    transpose, or with ``frag`` the halo-patch conv's two fragment layouts (flat uint8)."""
+    if not _dense(x):
+        x = x.contiguous()
+    if weight.dtype not in (torch.float32, torch.bfloat16) or weight.data_ptr() % 16:
+        weight = weight.to(torch.bfloat16, copy=True)
+    weight = _nhwc(weight) if weight.ndim == 4 else weight.contiguous()
+    cout, cin = weight.shape[0], weight.shape[1]
+    taps = weight.shape[2] * weight.shape[3] if weight.ndim == 4 else 1
+    n, dev = x.numel(), x.device
+    xq = torch.empty_like(x, dtype=FP8_DTYPE, memory_format=torch.preserve_format)
+    xs = torch.empty((), device=dev, dtype=torch.float32)
+    ws = torch.empty((), device=dev, dtype=torch.float32)
+    if frag:
+        wq = torch.empty(weight.numel(), device=dev, dtype=torch.uint8)
+        wt = torch.empty(weight.numel(), device=dev, dtype=torch.uint8)
+    else:
+        wq = torch.empty(weight.shape, device=dev, dtype=FP8_DTYPE, memory_format=(
+            torch.channels_last if weight.ndim == 4 else torch.contiguous_format))
+        wt = torch.empty((cin, *weight.shape[2:], cout), device=dev, dtype=FP8_DTYPE)
+    ws_bytes = _lib.query("dpa_quantize_with_weight_workspace_bytes", cout, taps, cin)
+    workspace = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
+    flags = (1 if weight.dtype == torch.bfloat16 else 0) | (2 if frag else 0)   # DPA_WP_*
+    _lib.call("dpa_quantize_fp8_bf16_with_weight", x.data_ptr(), n, xq.data_ptr(), xs.data_ptr(),
+              weight.data_ptr(), flags, cout, taps, cin, wq.data_ptr(), wt.data_ptr(),
+              ws.data_ptr(), workspace.data_ptr(), ws_bytes, _stream(x))
+    return xq, xs, wq, wt, ws
+
+
 def quantize_fp8_delayed_window(tensor: torch.Tensor, prev_scale: torch.Tensor,
                                 window: torch.Tensor, window_pos: torch.Tensor,
                                 advance: bool) -> tuple[torch.Tensor, torch.Tensor]:
@@ -380,21 +413,15 @@ def conv2d_fp8_dgrad_general(
     wcout, cin, kh, kw = weight.shape
     assert wcout == cout and kh == kw
     height, width = input_hw
-    dx = torch.empty((batch, cin, height, width), device=dy.device, dtype=torch.bfloat16,
-                     memory_format=torch.channels_last)
-    geom = (batch, height, width, cin, cout, kh, kw, stride, padding)
     if split:
         if weight_t is None:
             weight_t = weight_transpose_fp8(weight)
         assert weight_t.numel() == weight.numel() and weight_t.is_contiguous()
-        ws_bytes = _lib.query("dpa_conv2d_dgrad_split_workspace_bytes", *geom)
-        workspace = _workspace(ws_bytes, dy.device)
-        _lib.call(
-            "dpa_conv2d_dgrad_fp8_wt_split",
-            dy.data_ptr(), weight_t.data_ptr(), dy_scale.data_ptr(), weight_scale.data_ptr(),
-            dx.data_ptr(), _ptr(workspace), ws_bytes, *geom, _stream(dy),
-        )
-    elif weight_t is None:
+        return conv2d_fp8_dgrad_wt(dy, weight_t.view(FP8_DTYPE).view(cin, kh, kw, cout), dy_scale,
+                                   weight_scale, input_hw, stride, padding)
+    dx = torch.empty((batch, cin, height, width), device=dy.device, dtype=torch.bfloat16,
+                     memory_format=torch.channels_last)
+    if weight_t is None:
         ws_bytes = _lib.query("dpa_conv2d_dgrad_workspace_bytes", cin, cout, kh, kw)
         workspace = torch.empty(ws_bytes, device=dy.device, dtype=torch.uint8)
         _lib.call(
@@ -410,6 +437,37 @@ def conv2d_fp8_dgrad_general(
             dy.data_ptr(), weight_t.data_ptr(), dy_scale.data_ptr(), weight_scale.data_ptr(),
             dx.data_ptr(), batch, height, width, cin, cout, kh, kw, stride, padding, _stream(dy),
         )
+    return dx
+
+
+def conv2d_fp8_dgrad_wt(
+    dy: torch.Tensor,
+    weight_t: torch.Tensor,
+    dy_scale: torch.Tensor,
+    weight_scale: torch.Tensor,
+    input_hw: tuple[int, int],
+    stride: int = 1,
+    padding: int = 1,
+) -> torch.Tensor:
+    """conv2d_fp8_dgrad_general on the transposed weight alone: [Cin, k, k, Cout] bytes."""
+    assert dy.dtype == FP8_DTYPE and weight_t.dtype == FP8_DTYPE and weight_t.is_contiguous()
+    torch_checks_scale(dy_scale, dy.device)
+    torch_checks_scale(weight_scale, dy.device)
+    dy = _nhwc(dy)
+    batch, cout, _, _ = dy.shape
+    cin, kh, kw, wcout = weight_t.shape
+    assert wcout == cout and kh == kw
+    height, width = input_hw
+    dx = torch.empty((batch, cin, height, width), device=dy.device, dtype=torch.bfloat16,
+                     memory_format=torch.channels_last)
+    geom = (batch, height, width, cin, cout, kh, kw, stride, padding)
+    ws_bytes = _lib.query("dpa_conv2d_dgrad_split_workspace_bytes", *geom)
+    workspace = _workspace(ws_bytes, dy.device)
+    _lib.call(
+        "dpa_conv2d_dgrad_fp8_wt_split",
+        dy.data_ptr(), weight_t.data_ptr(), dy_scale.data_ptr(), weight_scale.data_ptr(),
+        dx.data_ptr(), _ptr(workspace), ws_bytes, *geom, _stream(dy),
+    )
     return dx
 
 
@@ -597,6 +655,37 @@ def conv2d_bwd_weight_fp8(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
 # --------------------------------------------------------------------------------------
 # autograd boundary (diffusion/fp8_kernels.py:822-923)
 # --------------------------------------------------------------------------------------
+def _conv_current_fwd(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: int,
+                      padding: int) -> torch.Tensor:
+    """Current-scaling conv forward of a bf16 channels-last x and an fp32 or bf16 weight, saving
+    e4m3 x and the weight's data-gradient copy."""
+    assert x.dtype == torch.bfloat16 and x.is_cuda and x.ndim == 4, f"{x.dtype} {x.is_cuda} {x.ndim}"
+    assert weight.is_cuda and weight.ndim == 4, f"{weight.is_cuda} {weight.ndim}"
+    batch, cin, height, width = x.shape
+    cout, wcin, kh, kw = weight.shape
+    assert wcin == cin and kh == kw
+    frag = hconv_shape(batch, cin, cout, height, width, kh, stride, padding)
+    x_fp8, x_scale, w_fp8, w_t, w_scale = _ops.quantize_with_weight(x, weight, frag)
+    ctx.save_for_backward(x_fp8, w_t, x_scale, w_scale)
+    ctx.geom = (cin, height, width, kh, stride, padding)
+    ctx.dw_f32 = weight.dtype == torch.float32
+    return _ops.conv_fwd_prepared(x_fp8, w_fp8, x_scale, w_scale, cout, stride, padding)
+
+
+def _conv_current_bwd(ctx: Any, dy: torch.Tensor, need_dx: bool = True):
+    """(dx, dw) of ``_conv_current_fwd`` for a bf16 channels-last dy; dw in fp32 for an fp32
+    weight (the bf16-rounded values autograd's cast of a bf16 gradient would give)."""
+    x_fp8, w_t, x_scale, w_scale = ctx.saved_tensors
+    cin, height, width, k, stride, padding = ctx.geom
+    dy_fp8, dy_scale = quantize_fp8(dy)
+    dx = None
+    if need_dx:
+        dx = _ops.conv_dgrad_prepared(dy_fp8, w_t, dy_scale, w_scale, cin, height, width, k,
+                                      stride, padding)
+    dw = _ops.conv_wgrad(x_fp8, dy_fp8, x_scale, dy_scale, k, stride, padding, 0, ctx.dw_f32)
+    return dx, dw
+
+
 class Conv2dFP8Specialized(torch.autograd.Function):
     """FP8 3x3/stride-1/pad-1 conv with e4m3 saved activations; current or delayed scaling.
 
@@ -614,14 +703,14 @@ class Conv2dFP8Specialized(torch.autograd.Function):
         do_delayed: bool = False,
     ) -> torch.Tensor | tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         x = x.to(torch.bfloat16)
-        # the reference relies on the model having been converted to channels-last; a
-        # contiguous (OIHW) parameter is converted here instead of producing wrong results
-        weight = weight.to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
 
         assert x.is_contiguous(memory_format=torch.channels_last)
 
         ctx.do_delayed = do_delayed
         if do_delayed:
+            # the reference relies on the model having been converted to channels-last; a
+            # contiguous (OIHW) parameter is converted here instead of producing wrong results
+            weight = weight.to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
             assert hist_scales is not None
             assert dy_ptrs is not None
             x_scale, weight_scale = hist_scales
@@ -635,16 +724,15 @@ class Conv2dFP8Specialized(torch.autograd.Function):
             ctx.window_pos = window_pos
             ctx.save_for_backward(x_fp8, weight_fp8, x_scale, weight_scale, dy_scale_hist)
         else:
-            x_fp8, x_scale = quantize_fp8(x)
-            weight_fp8, weight_scale = quantize_fp8(weight)
-            ctx.save_for_backward(x_fp8, weight_fp8, x_scale, weight_scale)
+            # x and the weight in one launch pair, which also writes the weight's
+            # data-gradient copy: that is what the backward keeps of the weight
+            weight = _nhwc(weight)
+            fwd_shapes(x, weight, FP8_DTYPE)
+            return _conv_current_fwd(ctx, x, weight, 1, 1)
 
         out = conv2d_fwd_fp8_prequantized(x_fp8, weight_fp8, x_scale, weight_scale)
-
-        if do_delayed:
-            ctx.mark_non_differentiable(x_scale_curr, weight_scale_curr)
-            return out, x_scale_curr, weight_scale_curr
-        return out
+        ctx.mark_non_differentiable(x_scale_curr, weight_scale_curr)
+        return out, x_scale_curr, weight_scale_curr
 
     @staticmethod
     @custom_bwd(device_type="cuda")
@@ -654,14 +742,13 @@ class Conv2dFP8Specialized(torch.autograd.Function):
         if dy.dtype != torch.bfloat16:
             dy = dy.to(torch.bfloat16)
 
-        if ctx.do_delayed:
-            x_fp8, weight_fp8, x_scale, weight_scale, dy_scale = ctx.saved_tensors
-            dy_fp8, dy_scale_curr = quantize_fp8_delayed(dy, dy_scale)
-            window_idx = ctx.window_pos.unsqueeze(0)
-            ctx.dy_window.scatter_(0, window_idx, dy_scale_curr.unsqueeze(0))
-        else:
-            x_fp8, weight_fp8, x_scale, weight_scale = ctx.saved_tensors
-            dy_fp8, dy_scale = quantize_fp8(dy)
+        if not ctx.do_delayed:
+            dx, dw = _conv_current_bwd(ctx, dy)
+            return dx, dw, None, None, None
+        x_fp8, weight_fp8, x_scale, weight_scale, dy_scale = ctx.saved_tensors
+        dy_fp8, dy_scale_curr = quantize_fp8_delayed(dy, dy_scale)
+        window_idx = ctx.window_pos.unsqueeze(0)
+        ctx.dy_window.scatter_(0, window_idx, dy_scale_curr.unsqueeze(0))
 
         assert dy_fp8.is_contiguous(memory_format=torch.channels_last)
         assert weight_fp8.is_contiguous(memory_format=torch.channels_last)
@@ -735,27 +822,13 @@ class Conv2dFP8General(torch.autograd.Function):
     @custom_fwd(device_type="cuda")
     def forward(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: int, padding: int) -> torch.Tensor:
         x = x.to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
-        weight = weight.to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
-        x_fp8, x_scale = quantize_fp8(x)
-        w_fp8, w_scale = quantize_fp8(weight)
-        ctx.save_for_backward(x_fp8, w_fp8, x_scale, w_scale)
-        ctx.stride, ctx.padding = stride, padding
-        ctx.input_hw = (x.shape[2], x.shape[3])
-        return _ops.conv_fwd(x_fp8, w_fp8, x_scale, w_scale, stride, padding)
+        return _conv_current_fwd(ctx, x, weight, stride, padding)
 
     @staticmethod
     @custom_bwd(device_type="cuda")
     def backward(ctx: Any, dy: torch.Tensor) -> Any:
-        x_fp8, w_fp8, x_scale, w_scale = ctx.saved_tensors
         dy = dy.to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
-        dy_fp8, dy_scale = quantize_fp8(dy)
-        k = w_fp8.shape[2]
-        dx = None
-        if ctx.needs_input_grad[0]:
-            dx = _ops.conv_dgrad(dy_fp8, w_fp8, dy_scale, w_scale, ctx.input_hw[0],
-                                 ctx.input_hw[1], ctx.stride, ctx.padding)
-        dw = _ops.conv_wgrad(x_fp8, dy_fp8, x_scale, dy_scale, k, ctx.stride, ctx.padding, 0,
-                             False)
+        dx, dw = _conv_current_bwd(ctx, dy, ctx.needs_input_grad[0])
         return dx, dw, None, None
 
 
@@ -900,12 +973,12 @@ class LinearFP8Function(torch.autograd.Function):
         n, k = weight.shape
         assert x.shape[-1] == k
         x2 = x.to(torch.bfloat16).reshape(-1, k).contiguous()
-        w = weight.to(torch.bfloat16).contiguous()
-        xq, xs = quantize_fp8_tensor(x2)
-        wq, wsc = quantize_fp8_tensor(w)
+        assert x2.is_cuda and weight.is_cuda, f"{x2.is_cuda} {weight.is_cuda}"
+        xq, xs, wq, wt, wsc = _ops.quantize_with_weight(x2, weight, False)
         b32 = None if bias is None else bias.detach().float().contiguous()
         y = _ops.gemm(xq, wq, xs, wsc, b32)
-        ctx.save_for_backward(xq, wq, xs, wsc)
+        ctx.save_for_backward(xq, wt, xs, wsc)
+        ctx.dw_f32 = weight.dtype == torch.float32
         ctx.lead = lead
         ctx.has_bias = bias is not None
         return y.reshape(*lead, n)
@@ -913,15 +986,15 @@ class LinearFP8Function(torch.autograd.Function):
     @staticmethod
     @custom_bwd(device_type="cuda")
     def backward(ctx: Any, dy: torch.Tensor):
-        xq, wq, xs, wsc = ctx.saved_tensors
-        n, k = wq.shape
+        xq, wt, xs, wsc = ctx.saved_tensors
+        k, n = wt.shape
         dy2 = dy.to(torch.bfloat16).reshape(-1, n).contiguous()
         dyq, dys = quantize_fp8_tensor(dy2)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = _ops.gemm_dgrad(dyq, wq, dys, wsc).reshape(*ctx.lead, k)
+            dx = _ops.gemm_dgrad_wt(dyq, wt, dys, wsc).reshape(*ctx.lead, k)
         if ctx.needs_input_grad[1]:
-            dw = _ops.gemm_wgrad(xq, dyq, xs, dys, False)
+            dw = _ops.gemm_wgrad(xq, dyq, xs, dys, ctx.dw_f32)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = dy2.float().sum(0)
         return dx, dw, db
@@ -1027,10 +1100,10 @@ class Conv2dFP8GeneralPrepared(torch.autograd.Function):
         return dx, dw, None, None, None, None, None
 
 
-def _linear_dgrad_wt(dy: torch.Tensor, wq: torch.Tensor, wq_t: torch.Tensor, dy_scale, w_scale):
+def _linear_dgrad_wt(dy: torch.Tensor, wq_t: torch.Tensor, dy_scale, w_scale):
     """linear_fp8_dgrad_prequantized with the transposed weight [K][N] given."""
     m, n = dy.shape
-    k = wq.shape[1]
+    k = wq_t.shape[0]
     dx = torch.empty((m, k), device=dy.device, dtype=torch.bfloat16)
     geom = (m, 1, 1, k, n, 1, 1, 1, 0)
     ws_bytes = _lib.query("dpa_conv2d_dgrad_split_workspace_bytes", *geom)
@@ -1083,7 +1156,7 @@ class LinearFP8Prepared(torch.autograd.Function):
         dyq, dys = quantize_fp8_from_producer(dy2, dy) or quantize_fp8_tensor(dy2)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = _linear_dgrad_wt(dyq, wq, wq_t, dys, wsc).reshape(*ctx.lead, k)
+            dx = _linear_dgrad_wt(dyq, wq_t, dys, wsc).reshape(*ctx.lead, k)
         if ctx.needs_input_grad[1]:
             dw = linear_fp8_wgrad_prequantized(xq, dyq, xs, dys, out_f32=True)
         if ctx.has_bias and ctx.needs_input_grad[2]:

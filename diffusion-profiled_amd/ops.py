@@ -14,9 +14,13 @@ Namespace ``dpa_fp8``:
 =================  ====================================================================
 ``quantize``        current scaling: (e4m3 q, fp32 scale)  (fp8_kernels.py:559-601)
 ``quantize_delayed``  cast with prev_scale, return the current scale  (:518-556)
+``quantize_with_weight``  x and its layer's weight in one launch pair, the weight in both
+                    layouts its products read
 ``conv_fwd``        e4m3 conv forward, any supported (k, stride, pad)  (:604-639)
 ``conv_dgrad``      e4m3 conv data gradient  (:671-709)
 ``conv_wgrad``      e4m3 conv weight gradient  (:723-808)
+``conv_fwd_prepared``, ``conv_dgrad_prepared``, ``gemm_dgrad_wt``  the products on the weight
+                    copies of ``quantize_with_weight``
 ``gemm``            e4m3 GEMM x @ w^T (the FP8 linear; no reference kernel)
 ``gemm_dgrad``      its data gradient dy @ w
 ``gemm_wgrad``      its weight gradient dy^T @ x
@@ -68,6 +72,30 @@ def _quantize_delayed_fake(tensor, prev_scale):
     return _quantize_fake(tensor)
 
 
+@torch.library.custom_op("dpa_fp8::quantize_with_weight", mutates_args=(), device_types="cuda")
+def quantize_with_weight(x: torch.Tensor, weight: torch.Tensor, frag: bool
+                         ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(e4m3 x, x scale, e4m3 w, its data-gradient copy, w scale), the weight's copies in the
+    halo-patch conv's fragment layouts (flat uint8) with ``frag``."""
+    return K._quantize_with_weight_impl(x, weight, frag)
+
+
+@quantize_with_weight.register_fake
+def _quantize_with_weight_fake(x, weight, frag):
+    xq, xs = _quantize_fake(x)
+    ws = x.new_empty((), dtype=torch.float32)
+    if frag:
+        wq = weight.new_empty((weight.numel(),), dtype=torch.uint8)
+        return xq, xs, wq, torch.empty_like(wq), ws
+    cout, cin = weight.shape[0], weight.shape[1]
+    if weight.ndim == 4:
+        wq = _empty_cl(weight.shape, weight.device, K.FP8_DTYPE)
+    else:
+        wq = weight.new_empty((cout, cin), dtype=K.FP8_DTYPE)
+    wt = weight.new_empty((cin, *weight.shape[2:], cout), dtype=K.FP8_DTYPE)
+    return xq, xs, wq, wt, ws
+
+
 # ---- convolution ---------------------------------------------------------------------
 @torch.library.custom_op("dpa_fp8::conv_fwd", mutates_args=(), device_types="cuda")
 def conv_fwd(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor,
@@ -111,6 +139,41 @@ def _conv_wgrad_fake(x, dy, x_scale, dy_scale, kernel_size, stride, padding, spl
                      torch.float32 if out_f32 else _BF16)
 
 
+@torch.library.custom_op("dpa_fp8::conv_fwd_prepared", mutates_args=(), device_types="cuda")
+def conv_fwd_prepared(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor,
+                      weight_scale: torch.Tensor, cout: int, stride: int,
+                      padding: int) -> torch.Tensor:
+    """conv_fwd with the weight as quantize_with_weight left it."""
+    if weight.dtype == torch.uint8:
+        return K.conv2d_fp8_fwd_wf(x, weight, x_scale, weight_scale, cout)
+    return K.conv2d_fp8_fwd_general(x, weight, x_scale, weight_scale, stride, padding)
+
+
+@conv_fwd_prepared.register_fake
+def _conv_fwd_prepared_fake(x, weight, x_scale, weight_scale, cout, stride, padding):
+    batch, _, height, width = x.shape
+    k = 3 if weight.dtype == torch.uint8 else weight.shape[2]
+    oh, ow = K._out_hw(height, width, k, stride, padding)
+    return _empty_cl((batch, cout, oh, ow), x.device)
+
+
+@torch.library.custom_op("dpa_fp8::conv_dgrad_prepared", mutates_args=(), device_types="cuda")
+def conv_dgrad_prepared(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torch.Tensor,
+                        weight_scale: torch.Tensor, cin: int, height: int, width: int, k: int,
+                        stride: int, padding: int) -> torch.Tensor:
+    """conv_dgrad with the weight's data-gradient copy of quantize_with_weight."""
+    if weight_t.dtype == torch.uint8:
+        return K.conv2d_fp8_dgrad_wf(dy, weight_t, dy_scale, weight_scale, cin)
+    return K.conv2d_fp8_dgrad_wt(dy, weight_t, dy_scale, weight_scale, (height, width), stride,
+                                 padding)
+
+
+@conv_dgrad_prepared.register_fake
+def _conv_dgrad_prepared_fake(dy, weight_t, dy_scale, weight_scale, cin, height, width, k,
+                              stride, padding):
+    return _empty_cl((dy.shape[0], cin, height, width), dy.device)
+
+
 # ---- GEMM (the FP8 linear) -------------------------------------------------------------
 @torch.library.custom_op("dpa_fp8::gemm", mutates_args=(), device_types="cuda")
 def gemm(a: torch.Tensor, b: torch.Tensor, a_scale: torch.Tensor, b_scale: torch.Tensor,
@@ -132,6 +195,18 @@ def gemm_dgrad(dy: torch.Tensor, weight: torch.Tensor, dy_scale: torch.Tensor,
 @gemm_dgrad.register_fake
 def _gemm_dgrad_fake(dy, weight, dy_scale, weight_scale):
     return dy.new_empty((dy.shape[0], weight.shape[1]), dtype=_BF16)
+
+
+@torch.library.custom_op("dpa_fp8::gemm_dgrad_wt", mutates_args=(), device_types="cuda")
+def gemm_dgrad_wt(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torch.Tensor,
+                  weight_scale: torch.Tensor) -> torch.Tensor:
+    """gemm_dgrad with the transposed e4m3 weight [K][N] of quantize_with_weight."""
+    return K._linear_dgrad_wt(dy, weight_t, dy_scale, weight_scale)
+
+
+@gemm_dgrad_wt.register_fake
+def _gemm_dgrad_wt_fake(dy, weight_t, dy_scale, weight_scale):
+    return dy.new_empty((dy.shape[0], weight_t.shape[0]), dtype=_BF16)
 
 
 @torch.library.custom_op("dpa_fp8::gemm_wgrad", mutates_args=(), device_types="cuda")

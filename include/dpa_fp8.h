@@ -442,6 +442,15 @@ int dpa_quantize_fp8_bf16_with_weight_prep(const void* x, int64_t n, void* q, fl
                                            const DpaWeightEntry* entries_dev, int count,
                                            int total_blocks, void* wp_workspace,
                                            int64_t wp_workspace_bytes, void* stream);
+/* Current scaling of x and of one weight w [cout][taps][cin] in two launches: x as
+ * dpa_quantize_fp8_bf16, w as a DpaWeightEntry of its own (flags: DPA_WP_BF16 | DPA_WP_FRAG;
+ * wq, wqt, w_scale: the entry's q, qt (NULL: none, else 8-B aligned), scale_used). The same bytes and scales
+ * as the two calls apart. */
+int64_t dpa_quantize_with_weight_workspace_bytes(int cout, int taps, int cin);
+int dpa_quantize_fp8_bf16_with_weight(const void* x, int64_t n, void* q, float* scale_out,
+                                      const void* w, int flags, int cout, int taps, int cin,
+                                      void* wq, void* wqt, float* w_scale, void* workspace,
+                                      int64_t workspace_bytes, void* stream);
 /* hist[i] = max over window i of len floats (torch.max; NaN if the window holds one);
  * windows_dev: device array of count window pointers. One launch for every window. */
 int dpa_window_max_grouped_f32(const float* const* windows_dev, int count, int64_t len,

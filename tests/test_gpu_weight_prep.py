@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import math
 
+import numpy as np
 import pytest
 import torch
 
@@ -250,3 +251,60 @@ def test_quantize_with_weight_prep_equals_the_two_calls(case):
         for i in range(len(ws)):
             assert torch.equal(fused.q[i].view(torch.uint8), sep.q[i].view(torch.uint8)), (rnd, i)
             assert torch.equal(fused.qt[i].view(torch.uint8), sep.qt[i].view(torch.uint8)), (rnd, i)
+
+
+@pytest.mark.parametrize("xshape,wshape,wdtype,stride", [
+    ((3, 128, 32, 32), (256, 128, 3, 3), torch.float32, 1),     # fragment layouts
+    ((2, 256, 16, 16), (128, 256, 3, 3), torch.bfloat16, 1),
+    ((5, 256, 6, 10), (128, 256, 3, 3), torch.float32, 2),      # OHWI bytes, their transpose
+    ((1, 128, 3, 3), (384, 128, 1, 1), torch.float16, 1),       # x of one workgroup
+    ((37, 256), (384, 256), torch.float32, 0),                  # a linear
+], ids=str)
+@pytest.mark.parametrize("aligned", [True, False], ids=["aligned", "offset"])
+def test_layer_quantizes_both_operands_as_the_separate_calls(xshape, wshape, wdtype, stride,
+                                                             aligned):
+    """The current-scaling conv and linear Functions against quantize_fp8 of x and of the bf16
+    weight and the prequantized products: the operands' bytes and scales, y, dx and dw are
+    equal (dw of an fp32 weight: the bf16 values in fp32). x 16-B aligned or not; the weight
+    contiguous, that is OIHW, not the order that the kernels read."""
+    g = torch.Generator().manual_seed(23)
+    n = int(np.prod(xshape))
+    x = (torch.randn(n + 1, generator=g) * 2).to(torch.bfloat16).cuda()[0 if aligned else 1:][:n]
+    w = (torch.randn(wshape, generator=g) * 0.05).to(wdtype).cuda().requires_grad_()
+    wb = w.detach().to(torch.bfloat16)
+    if stride:
+        b, c, h, wd = xshape
+        x = x.view(b, h, wd, c).permute(0, 3, 1, 2)
+        wb, pad = wb.contiguous(memory_format=torch.channels_last), wshape[2] // 2
+        frag = K.hconv_shape(b, c, wshape[0], h, wd, wshape[2], stride, pad)
+    else:
+        x, frag = x.view(xshape), False
+    x.requires_grad_()
+    xq, xs = K.quantize_fp8_tensor(x.detach())
+    wq, ws = K.quantize_fp8_tensor(wb)
+    oxq, oxs, owq, owt, ows = K._quantize_with_weight_impl(x.detach(), w.detach(), frag)
+    rq, rt = ((wq, K.weight_transpose_fp8(wq if stride else wq[:, :, None, None])) if not frag
+              else K.weight_frag_fp8(wq))
+    flat = lambda t: (t.permute(0, 2, 3, 1) if t.ndim == 4 and t.dtype != torch.uint8 else t) \
+        .contiguous().view(torch.uint8).flatten()                                # noqa: E731
+    assert float(oxs) == float(xs) and float(ows) == float(ws)
+    assert torch.equal(flat(oxq), flat(xq)) and torch.equal(flat(owq), flat(rq))
+    assert torch.equal(owt.contiguous().view(torch.uint8).flatten(),
+                       rt.contiguous().view(torch.uint8).flatten())
+
+    y = (K.conv2d_fp8(x, w, stride, pad) if stride else K.linear_fp8_autograd(x, w))
+    dy = (torch.randn(y.shape, generator=g) * 1e-2).to(torch.bfloat16).cuda()
+    if stride:
+        dy = dy.contiguous(memory_format=torch.channels_last)
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    dyq, dys = K.quantize_fp8_tensor(dy)
+    if stride:
+        ry = K.conv2d_fp8_fwd_general(xq, wq, xs, ws, stride, pad)
+        rdx = K.conv2d_fp8_dgrad_general(dyq, wq, dys, ws, xshape[2:], stride, pad)
+        rdw = K.conv2d_fp8_wgrad_general(xq, dyq, xs, dys, wshape[2], stride, pad)
+    else:
+        ry = K.linear_fp8_prequantized(xq, wq, xs, ws)
+        rdx = K.linear_fp8_dgrad_prequantized(dyq, wq, dys, ws)
+        rdw = K.linear_fp8_wgrad_prequantized(xq, dyq, xs, dys)
+    assert torch.equal(y, ry) and torch.equal(dx, rdx)
+    assert dw.dtype == wdtype and torch.equal(dw, rdw.to(wdtype))
