@@ -61,6 +61,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "dpa_weight_frag_fp8": (c_int, [c_void_p] * 3 + [c_int] * 4 + [c_void_p]),
     "dpa_conv2d_fwd_fp8_wf": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p]),
     "dpa_conv2d_dgrad_fp8_wf": (c_int, [c_void_p] * 5 + [c_int] * 5 + [c_void_p]),
+    "dpa_conv2d_fwd_fp8_frag": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p]),
+    "dpa_conv2d_dgrad_fp8_frag": (c_int, [c_void_p] * 5 + [c_int] * 5 + [c_void_p]),
+    "dpa_conv2d_frag_supported": (c_int, [c_int] * 5),
     "dpa_conv2d_wgrad_workspace_bytes": (c_int64, [c_int] * 10),
     "dpa_conv2d_wgrad_fp8": (
         c_int,

@@ -629,6 +629,10 @@ bool hconv_supported(int N, int H, int W, int C, int Cout);
 int hconv_run(const void* act, const void* wgt, const float* sa, const float* sb,
               const float* bias, void* out, int N, int H, int W, int C, int Cout, int flip,
               int wfrag, int num_cus, hipStream_t s);
+bool hconv_frag_supported(int N, int H, int W, int C, int Cout, int num_cus);
+int hconv_frag_run(const void* act, const void* wf, const float* sa, const float* sb,
+                   const float* bias, void* out, int N, int H, int W, int C, int Cout,
+                   int num_cus, hipStream_t s);
 int weight_frag_run(const void* w, void* out, int rows, int K, int T, int transpose,
                     hipStream_t s);
 
@@ -882,6 +886,32 @@ extern "C" int dpa_conv2d_dgrad_fp8_wf(const void* dyq, const void* wf_dgrad,
   if (!aligned(dyq, 16) || !aligned(wf_dgrad, 16) || !aligned(dx, 16)) return DPA_ERR_ALIGN;
   return hconv_run(dyq, wf_dgrad, dy_scale, w_scale, nullptr, dx, N, H, W, Cout, Cin, 0, 1,
                    num_cus(), (hipStream_t)stream);
+}
+
+// ---- the same on every image that one of the halo-patch kernel's tiles divides ----
+
+extern "C" int dpa_conv2d_frag_supported(int N, int H, int W, int Cin, int Cout) {
+  return hconv_frag_supported(N, H, W, Cin, Cout, num_cus()) ? 1 : 0;
+}
+
+extern "C" int dpa_conv2d_fwd_fp8_frag(const void* xq, const void* wf, const float* x_scale,
+                                       const float* w_scale, const float* bias, void* y, int N,
+                                       int H, int W, int Cin, int Cout, void* stream) {
+  if (!xq || !wf || !x_scale || !w_scale || !y) return DPA_ERR_NULL;
+  if (!hconv_frag_supported(N, H, W, Cin, Cout, num_cus())) return DPA_ERR_SHAPE;
+  if (!aligned(xq, 16) || !aligned(wf, 16) || !aligned(y, 16)) return DPA_ERR_ALIGN;
+  return hconv_frag_run(xq, wf, x_scale, w_scale, bias, y, N, H, W, Cin, Cout, num_cus(),
+                        (hipStream_t)stream);
+}
+
+extern "C" int dpa_conv2d_dgrad_fp8_frag(const void* dyq, const void* wf_dgrad,
+                                         const float* dy_scale, const float* w_scale, void* dx,
+                                         int N, int H, int W, int Cin, int Cout, void* stream) {
+  if (!dyq || !wf_dgrad || !dy_scale || !w_scale || !dx) return DPA_ERR_NULL;
+  if (!hconv_frag_supported(N, H, W, Cout, Cin, num_cus())) return DPA_ERR_SHAPE;
+  if (!aligned(dyq, 16) || !aligned(wf_dgrad, 16) || !aligned(dx, 16)) return DPA_ERR_ALIGN;
+  return hconv_frag_run(dyq, wf_dgrad, dy_scale, w_scale, nullptr, dx, N, H, W, Cout, Cin,
+                        num_cus(), (hipStream_t)stream);
 }
 
 extern "C" int dpa_gemm_fp8(const void* a, const void* b, const float* a_scale,

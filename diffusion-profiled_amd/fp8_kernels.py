@@ -527,6 +527,49 @@ def conv2d_fp8_dgrad_wf(dy: torch.Tensor, wf_dgrad: torch.Tensor, dy_scale: torc
     return dx
 
 
+def frag_shape(batch: int, cin: int, cout: int, height: int, width: int, k: int = 3,
+               stride: int = 1, padding: int = 1) -> bool:
+    """Shapes of conv2d_fp8_fwd_frag / _dgrad_frag: images that a tile of the halo-patch kernel
+    divides (dpa_conv2d_frag_supported)."""
+    tiled = ((width % 16 == 0 and height % 4 == 0) or (width % 8 == 0 and height % 8 == 0)
+             or (width == 4 and height == 4))
+    return (k == 3 and stride == 1 and padding == 1 and tiled and height > 0 and width > 0
+            and cin % 128 == 0 and cout % 128 == 0 and cin > 0 and cout > 0
+            and 0 < batch * height * width * max(cin, cout) < 2**31
+            and 9 * cin * cout < 2**31)
+
+
+def conv2d_fp8_fwd_frag(x: torch.Tensor, wf: torch.Tensor, x_scale: torch.Tensor,
+                        weight_scale: torch.Tensor, cout: int,
+                        bias: torch.Tensor | None = None) -> torch.Tensor:
+    """conv2d_fp8_fwd_wf for every frag_shape, on the tile that fills the GPU."""
+    assert x.dtype == FP8_DTYPE and wf.dtype == torch.uint8 and wf.is_contiguous()
+    x = _nhwc(x)
+    batch, cin, height, width = x.shape
+    assert wf.numel() == cout * 9 * cin and frag_shape(batch, cin, cout, height, width)
+    y = torch.empty((batch, cout, height, width), device=x.device, dtype=torch.bfloat16,
+                    memory_format=torch.channels_last)
+    _lib.call("dpa_conv2d_fwd_fp8_frag", x.data_ptr(), wf.data_ptr(), x_scale.data_ptr(),
+              weight_scale.data_ptr(), _ptr(bias), y.data_ptr(), batch, height, width, cin, cout,
+              _stream(x))
+    return y
+
+
+def conv2d_fp8_dgrad_frag(dy: torch.Tensor, wf_dgrad: torch.Tensor, dy_scale: torch.Tensor,
+                          weight_scale: torch.Tensor, cin: int) -> torch.Tensor:
+    """conv2d_fp8_dgrad_wf for every frag_shape, on the tile that fills the GPU."""
+    assert dy.dtype == FP8_DTYPE and wf_dgrad.dtype == torch.uint8 and wf_dgrad.is_contiguous()
+    dy = _nhwc(dy)
+    batch, cout, height, width = dy.shape
+    assert wf_dgrad.numel() == cout * 9 * cin and frag_shape(batch, cin, cout, height, width)
+    dx = torch.empty((batch, cin, height, width), device=dy.device, dtype=torch.bfloat16,
+                     memory_format=torch.channels_last)
+    _lib.call("dpa_conv2d_dgrad_fp8_frag", dy.data_ptr(), wf_dgrad.data_ptr(),
+              dy_scale.data_ptr(), weight_scale.data_ptr(), dx.data_ptr(), batch, height, width,
+              cin, cout, _stream(dy))
+    return dx
+
+
 def weight_transpose_fp8(weight: torch.Tensor) -> torch.Tensor:
     """[Cout][R][S][Cin] e4m3 bytes -> [Cin][R][S][Cout] (the data-gradient operand)."""
     assert weight.dtype == FP8_DTYPE
@@ -664,7 +707,7 @@ def _conv_current_fwd(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: i
     batch, cin, height, width = x.shape
     cout, wcin, kh, kw = weight.shape
     assert wcin == cin and kh == kw
-    frag = hconv_shape(batch, cin, cout, height, width, kh, stride, padding)
+    frag = frag_shape(batch, cin, cout, height, width, kh, stride, padding)
     x_fp8, x_scale, w_fp8, w_t, w_scale = _ops.quantize_with_weight(x, weight, frag)
     ctx.save_for_backward(x_fp8, w_t, x_scale, w_scale)
     ctx.geom = (cin, height, width, kh, stride, padding)
@@ -1036,7 +1079,7 @@ class Conv2dFP8DelayedPrepared(torch.autograd.Function):
         ctx.save_for_backward(x_fp8, wq, wq_t, x_scale, w_scale, dy_scale)
         if wq.dtype == torch.uint8:      # fragment layouts of the halo-patch kernel
             fwd_shapes(x_fp8, weight, FP8_DTYPE)
-            return conv2d_fp8_fwd_wf(x_fp8, wq, x_scale, w_scale, weight.shape[0])
+            return conv2d_fp8_fwd_frag(x_fp8, wq, x_scale, w_scale, weight.shape[0])
         return conv2d_fwd_fp8_prequantized(x_fp8, wq, x_scale, w_scale)
 
     @staticmethod
@@ -1051,7 +1094,7 @@ class Conv2dFP8DelayedPrepared(torch.autograd.Function):
                 dy = dy.to(torch.bfloat16)
             dy_fp8 = quantize_fp8_delayed_deferred(dy, dy_scale, ctx.parts[2], ctx.parts[3])
         if wq.dtype == torch.uint8:
-            dx = conv2d_fp8_dgrad_wf(dy_fp8, wq_t, dy_scale, w_scale, ctx.cin_cout[0])
+            dx = conv2d_fp8_dgrad_frag(dy_fp8, wq_t, dy_scale, w_scale, ctx.cin_cout[0])
         else:
             batch, cin, cout, height, width = xgrad_shapes(dy_fp8, wq, FP8_DTYPE)
             dx = conv2d_fp8_dgrad_general(dy_fp8, wq, dy_scale, w_scale, (height, width), 1, 1,
@@ -1077,7 +1120,7 @@ class Conv2dFP8GeneralPrepared(torch.autograd.Function):
         ctx.k, ctx.cin = weight.shape[2], weight.shape[1]
         if wq.dtype == torch.uint8:      # fragment layouts of the halo-patch kernel
             assert stride == 1 and padding == 1 and ctx.k == 3
-            return conv2d_fp8_fwd_wf(x_fp8, wq, x_scale, w_scale, weight.shape[0])
+            return conv2d_fp8_fwd_frag(x_fp8, wq, x_scale, w_scale, weight.shape[0])
         return conv2d_fp8_fwd_general(x_fp8, wq, x_scale, w_scale, stride, padding)
 
     @staticmethod
@@ -1091,7 +1134,7 @@ class Conv2dFP8GeneralPrepared(torch.autograd.Function):
         dx = None
         if ctx.needs_input_grad[0]:
             if wq.dtype == torch.uint8:
-                dx = conv2d_fp8_dgrad_wf(dy_fp8, wq_t, dy_scale, w_scale, ctx.cin)
+                dx = conv2d_fp8_dgrad_frag(dy_fp8, wq_t, dy_scale, w_scale, ctx.cin)
             else:
                 dx = conv2d_fp8_dgrad_general(dy_fp8, wq, dy_scale, w_scale, ctx.input_hw,
                                               ctx.stride, ctx.padding, weight_t=wq_t)

@@ -145,7 +145,7 @@ def conv_fwd_prepared(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tens
                       padding: int) -> torch.Tensor:
     """conv_fwd with the weight as quantize_with_weight left it."""
     if weight.dtype == torch.uint8:
-        return K.conv2d_fp8_fwd_wf(x, weight, x_scale, weight_scale, cout)
+        return K.conv2d_fp8_fwd_frag(x, weight, x_scale, weight_scale, cout)
     return K.conv2d_fp8_fwd_general(x, weight, x_scale, weight_scale, stride, padding)
 
 
@@ -163,7 +163,7 @@ def conv_dgrad_prepared(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torc
                         stride: int, padding: int) -> torch.Tensor:
     """conv_dgrad with the weight's data-gradient copy of quantize_with_weight."""
     if weight_t.dtype == torch.uint8:
-        return K.conv2d_fp8_dgrad_wf(dy, weight_t, dy_scale, weight_scale, cin)
+        return K.conv2d_fp8_dgrad_frag(dy, weight_t, dy_scale, weight_scale, cin)
     return K.conv2d_fp8_dgrad_wt(dy, weight_t, dy_scale, weight_scale, (height, width), stride,
                                  padding)
 

@@ -98,7 +98,7 @@ class _PreparedFP8Weight:
             self._fp8_mode = mode
             if x is not None and w.ndim == 4 and w.shape[2] == 3:
                 n, cin, h, wd = x.shape
-                self._fp8_frag = K.hconv_shape(n, cin, w.shape[0], h, wd)
+                self._fp8_frag = K.frag_shape(n, cin, w.shape[0], h, wd)
 
     def _prepared(self, mode: str):
         plan = self._fp8_plan
@@ -202,7 +202,9 @@ class Conv2dFP8(_PreparedFP8Weight, nn.Module):
             return out
         if self.conv_fp8_general(x, self.conv.weight):
             pw = self._prepared("current")
-            if pw is not None:
+            # (a weight prepared in the fragment layouts serves the shapes of their kernel)
+            if pw is not None and (not pw.frag or K.frag_shape(
+                    x.shape[0], x.shape[1], self.conv.weight.shape[0], *x.shape[2:])):
                 return K.Conv2dFP8GeneralPrepared.apply(x, self.conv.weight, pw.q, pw.qt,
                                                         pw.scale, 1, 1)
             self._note_fp8_mode("current", self.conv.weight, x)

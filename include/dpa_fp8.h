@@ -157,6 +157,18 @@ int dpa_conv2d_fwd_fp8_wf(const void* xq, const void* wf, const float* x_scale,
 int dpa_conv2d_dgrad_fp8_wf(const void* dyq, const void* wf_dgrad, const float* dy_scale,
                             const float* w_scale, void* dx, int N, int H, int W, int Cin,
                             int Cout, void* stream);
+/* The same products for every image that one of the halo-patch kernel's tiles divides (256
+ * pixels as 8 x 32 or 16 x 16, 128 as 8 x 16, 64 as 4 x 16, 8 x 8 or four images of 4 x 4 rows x
+ * columns; the launch takes the tile that fills the GPU): W % 16 == 0 and H % 4 == 0, W % 8 == 0
+ * and H % 8 == 0, or 4 x 4, and channels multiples of 128. dpa_conv2d_frag_supported: 1 where they do (else
+ * DPA_ERR_SHAPE). */
+int dpa_conv2d_frag_supported(int N, int H, int W, int Cin, int Cout);
+int dpa_conv2d_fwd_fp8_frag(const void* xq, const void* wf, const float* x_scale,
+                            const float* w_scale, const float* bias, void* y, int N, int H,
+                            int W, int Cin, int Cout, void* stream);
+int dpa_conv2d_dgrad_fp8_frag(const void* dyq, const void* wf_dgrad, const float* dy_scale,
+                              const float* w_scale, void* dx, int N, int H, int W, int Cin,
+                              int Cout, void* stream);
 
 /* Bytes of workspace dpa_conv2d_dgrad_fp8 needs (the transposed weight, Cout*R*S*Cin). */
 int64_t dpa_conv2d_dgrad_workspace_bytes(int Cin, int Cout, int R, int S);

@@ -212,3 +212,37 @@ def test_deferred_window_entries(lib):
     assert lib.dpa_quantize_fp8_delayed_deferred_bf16(ctypes.c_void_p(0x1008), 16, fake, fake, fake, 512, fake, nul) == -3
     assert lib.dpa_delayed_windows_finalize(nul, 3, nul) == -1
     assert lib.dpa_delayed_windows_finalize(fake, 0, nul) == -2
+
+
+def test_fragment_conv_shapes_agree_with_the_python_rule(lib):
+    """dpa_conv2d_frag_supported and fp8_kernels.frag_shape, which layers ask before their
+    weights are laid out, say the same over sizes around every tile's edges, and the entries
+    refuse what they refuse."""
+    K = dpa_mod("fp8_kernels")
+    sides = [1, 2, 4, 6, 8, 12, 16, 20, 24, 30, 32, 33, 40, 64]
+    seen = set()
+    for n in (1, 3, 128):
+        for h in sides:
+            for w in sides:
+                for cin, cout in ((128, 128), (256, 384), (96, 128), (128, 64)):
+                    ok = K.frag_shape(n, cin, cout, h, w)
+                    assert bool(lib.dpa_conv2d_frag_supported(n, h, w, cin, cout)) == ok, (n, h, w)
+                    seen.add(ok)
+    assert seen == {True, False}
+    assert not K.frag_shape(1 << 17, 128, 128, 16, 16)          # 32-bit offsets
+    assert not lib.dpa_conv2d_frag_supported(1 << 17, 16, 16, 128, 128)
+    assert not K.frag_shape(1, 128, 128, 16, 16, 3, 2, 1)
+    import ctypes
+    fake, nul, odd = ctypes.c_void_p(0x1000), None, ctypes.c_void_p(0x1008)
+    assert lib.dpa_conv2d_fwd_fp8_frag(fake, fake, fake, fake, nul, fake, 1, 6, 8, 128, 128, nul) == -4
+    assert lib.dpa_conv2d_fwd_fp8_frag(fake, nul, fake, fake, nul, fake, 1, 8, 8, 128, 128, nul) == -1
+    assert lib.dpa_conv2d_dgrad_fp8_frag(fake, fake, fake, fake, odd, 1, 8, 8, 128, 128, nul) == -3
+    # both operands of a layer: sizes, the weight's shape and alignment, the workspace
+    q = lib.dpa_quantize_fp8_bf16_with_weight
+    need = lib.dpa_quantize_with_weight_workspace_bytes(128, 9, 128)
+    assert need == 4096 + 4 * 36
+    assert q(nul, 16, fake, fake, fake, 0, 128, 9, 128, fake, fake, fake, fake, need, nul) == -1
+    assert q(fake, 0, fake, fake, fake, 0, 128, 9, 128, fake, fake, fake, fake, need, nul) == -2
+    assert q(fake, 16, fake, fake, fake, 2, 128, 9, 64, fake, fake, fake, fake, need, nul) == -4
+    assert q(fake, 16, fake, fake, odd, 0, 128, 9, 128, fake, fake, fake, fake, need, nul) == -3
+    assert q(fake, 16, fake, fake, fake, 0, 128, 9, 128, fake, fake, fake, fake, need - 4, nul) == -5

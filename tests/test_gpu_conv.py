@@ -344,3 +344,39 @@ def test_fragment_weight_entries_refuse_other_shapes():
     assert L.dpa_conv2d_fwd_fp8_wf(act, wgt, s, s, nul, out + 8, 2, 32, 32, 128, 128, nul) == -3
     assert L.dpa_weight_frag_fp8(wgt, act, nul, 100, 3, 3, 128, nul) == -4
     torch.cuda.synchronize()
+
+
+# tiles of 64 pixels (4 x 16, 8 x 8, four images of 4 x 4 with a ragged last tile), of 128 and
+# of 256 (chosen by the launch's size; a tile's columns not the whole image), odd and even
+# chunk counts, several tiles per workgroup
+FRAG_SHAPES = [(1, 128, 128, 8, 8), (5, 384, 256, 8, 8), (6, 256, 128, 4, 4), (3, 128, 256, 12, 48),
+               (2, 256, 128, 40, 24), (1, 128, 128, 64, 64), (36, 128, 256, 16, 32),
+               (70, 128, 256, 16, 16), (300, 128, 128, 8, 8), (9, 128, 128, 64, 64)]
+
+
+@pytest.mark.parametrize("shape", FRAG_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_fragment_weight_convs_on_every_tile(K, shape):
+    """conv2d_fp8_fwd_frag / _dgrad_frag against the exact oracle (the images that the oracle's
+    time allows) and the OHWI entries (all of them; fp32 sums in another order, so equal but
+    for bf16 rounding ties)."""
+    n, cin, cout, h, w = shape
+    xq, xs, wq, ws, dyq, dys = quantized_inputs(K, n, cin, cout, h, w, seed=sum(shape))
+    assert K.frag_shape(n, cin, cout, h, w)
+    wf, wt = K.weight_frag_fp8(wq)
+    bias = torch.linspace(-1, 1, cout, device="cuda")
+    y = K.conv2d_fp8_fwd_frag(xq, wf, xs, ws, cout)
+    yb = K.conv2d_fp8_fwd_frag(xq, wf, xs, ws, cout, bias)
+    dx = K.conv2d_fp8_dgrad_frag(dyq, wt, dys, ws, cin)
+    refs = (K.conv2d_fp8_fwd_general(xq, wq, xs, ws),
+            K.conv2d_fp8_fwd_general(xq, wq, xs, ws, bias=bias),
+            K.conv2d_fp8_dgrad_general(dyq, wq, dys, ws, (h, w)))
+    for got, ref in zip((y, yb, dx), refs):
+        assert got.shape == ref.shape and got.stride() == ref.stride()
+        # a rounding tie moves a value by one bf16 ulp, 2^-7 of it at most
+        assert bool(((got.float() - ref.float()).abs() <= 2**-7 * ref.float().abs() + 1e-30).all())
+        assert float((got != ref).float().mean()) < 1e-3
+    k = [0, n - 1] if n > 2 else list(range(n))
+    xb, wb, db = (nhwc_bits(t.cpu().view(torch.uint8)) for t in (xq[k], wq, dyq[k]))
+    assert_bf16_close(nhwc_bits(y[k].cpu()), O.conv2d_fwd(xb, wb, f32(xs), f32(ws)), f"fwd {shape}")
+    assert_bf16_close(nhwc_bits(dx[k].cpu()), O.conv2d_dgrad(db, wb, f32(dys), f32(ws), (h, w)),
+                      f"dgrad {shape}")
