@@ -83,36 +83,46 @@ struct GnArgs {
 // a 16-bit number, are >= floor(p * 2^16). Four elements per 64-bit hash halve the hash's vector
 // instructions against one per pair (its multiplies are done in 32-bit halves); 16 bits
 // still give a drop rate within 2^-16 of p.
-// Returns the keep bits of the 8 elements idx0 .. idx0 + 7 (idx0 a multiple of 8).
-__device__ __forceinline__ uint32_t drop_keep8(uint64_t seed, int64_t idx0, uint32_t keep_from) {
-  constexpr uint64_t kGolden = 0x9E3779B97F4A7C15ull;
-  const uint64_t z0 = seed + (uint64_t)(idx0 >> 2) * kGolden;
-  uint32_t bits = 0;
+// The decisions come as masks of bf16 pairs (0xffff: kept), to be and'ed into packed values:
+// four packed 16-bit instructions per pair instead of an extract, a compare and a select per
+// element. r >= k is sat(k - r) == 0 in 16 bits, and min(., 1) - 1 turns that into the mask.
+constexpr uint64_t kDropGolden = 0x9E3779B97F4A7C15ull;
+
+// hash input of element idx (a multiple of 4)
+__device__ __forceinline__ uint64_t drop_z(uint64_t seed, int64_t idx) {
+  return seed + (uint64_t)(idx >> 2) * kDropGolden;
+}
+
+__device__ __forceinline__ uint32_t drop_mask2(uint32_t r, uint32_t keep2) {
+  uint32_t m;
+  // (as instructions of its own: the compiler turns the form into compares and selects)
+  asm("v_pk_sub_u16 %0, %1, %2 clamp\n\tv_pk_min_u16 %0, %0, %3\n\tv_pk_sub_i16 %0, %0, %3"
+      : "=&v"(m)
+      : "v"(keep2), "v"(r), "v"(0x00010001u));
+  return m;
+}
+
+// Masks of the 8 elements whose hash input starts at z0; keep2: the threshold in both halves.
+__device__ __forceinline__ uint4 drop_mask8(uint64_t z0, uint32_t keep2) {
+  uint32_t m[4];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    uint64_t z = z0 + (uint64_t)i * kGolden;
+    uint64_t z = z0 + (uint64_t)i * kDropGolden;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z ^= z >> 31;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t r = (uint32_t)(z >> (16 * j)) & 0xffffu;
-      bits |= (uint32_t)(r >= keep_from) << (4 * i + j);
-    }
+    m[2 * i] = drop_mask2((uint32_t)z, keep2);
+    m[2 * i + 1] = drop_mask2((uint32_t)(z >> 32), keep2);
   }
-  return bits;
+  return uint4{m[0], m[1], m[2], m[3]};
 }
 
-// v * scale if bit e of the keep bits is set, else +0: the selection as a mask of the bit
-// (v_bfe_i32 gives 0 or all ones) and'ed into the product, so no per-element lane mask is
-// formed (in the backward, which keeps each pixel's keep bits for both passes, those masks
-// took 2 scalar registers per element and were spilled to vector lanes: ~700 v_readlane /
-// v_writelane per thread in the 1024-pixel form)
-__device__ __forceinline__ float drop_sel(float v, uint32_t keep, int e, float scale) {
-  uint32_t m;
-  // (as an instruction of its own: the compiler would turn the and back into a select)
-  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(m) : "v"(keep), "i"(e));
-  return __uint_as_float(__float_as_uint(v * scale) & m);
+__device__ __forceinline__ uint32_t drop_keep2(const GnArgs& p) {
+  return p.drop_keep | (p.drop_keep << 16);
+}
+
+__device__ __forceinline__ uint4 and4(uint4 a, uint4 b) {
+  return uint4{a.x & b.x, a.y & b.y, a.z & b.z, a.w & b.w};
 }
 
 // sigmoid(v) = 1 / (1 + e^-v) from the hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32,
@@ -157,7 +167,8 @@ __device__ __forceinline__ void slab_reduce(float (&v)[NV], float* red) {
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = red[gq * NV + k];
-#pragma unroll 1
+  // (with few values the reads of all waves are in flight at once)
+#pragma unroll(NV <= 2 ? kWaves : 1)
   for (int w = 1; w < kWaves; ++w) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] += red[(w * 8 + gq) * NV + k];
@@ -188,43 +199,88 @@ __device__ __forceinline__ void load8f(const float* src, float (&v)[8]) {
   }
 }
 
+// The same 8 floats as they are in memory, to be looked at later
+__device__ __forceinline__ void load8raw(const float* src, uint4 (&v)[2]) {
+  if ((reinterpret_cast<uintptr_t>(src) & 15) == 0) {
+    v[0] = reinterpret_cast<const uint4*>(src)[0];
+    v[1] = reinterpret_cast<const uint4*>(src)[1];
+  } else {
+    const uint32_t* s = reinterpret_cast<const uint32_t*>(src);
+    v[0] = uint4{s[0], s[1], s[2], s[3]};
+    v[1] = uint4{s[4], s[5], s[6], s[7]};
+  }
+}
+
+__device__ __forceinline__ void floats8(const uint4 (&v)[2], float (&f)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    f[4 * h] = __uint_as_float(v[h].x);
+    f[4 * h + 1] = __uint_as_float(v[h].y);
+    f[4 * h + 2] = __uint_as_float(v[h].z);
+    f[4 * h + 3] = __uint_as_float(v[h].w);
+  }
+}
+
 // FiLM scale/shift of channels ch..ch+7 of image n: fp32 [N][C] pairs, or the bf16 time
 // projection [N][2C] with scale bf16(w + 1) (the reference adds 1 in bf16) and shift b; no FiLM
-// gives 1 and 0.
-__device__ __forceinline__ bool load_film(const GnArgs& p, int n, int ch, float (&fsc)[8],
-                                          float (&fsh)[8]) {
-  if (p.fs) {
-    load8f(p.fs + (int64_t)n * p.C + ch, fsc);
-    load8f(p.fb + (int64_t)n * p.C + ch, fsh);
-    return true;
-  }
-  if (p.wb) {
-    const uint16_t* w = p.wb + (int64_t)n * 2 * p.C + ch;
-    float wf[8];
-    if ((reinterpret_cast<uintptr_t>(w) & 15) == 0) {  // (uniform: base alignment)
-      unpack8(*reinterpret_cast<const uint4*>(w), wf);
-      unpack8(*reinterpret_cast<const uint4*>(w + p.C), fsh);
-    } else {
+// gives 1 and 0. Loading and use are apart: a kernel issues these loads before its pixels'
+// (vector loads return in order: behind them, the first use would wait for every pixel) and
+// looks at them after.
+struct GnFilm {
+  uint4 s[2], b[2];
+  __device__ __forceinline__ void load(const GnArgs& p, int n, int ch) {
+    if (p.fs) {
+      load8raw(p.fs + (int64_t)n * p.C + ch, s);
+      load8raw(p.fb + (int64_t)n * p.C + ch, b);
+    } else if (p.wb) {
+      const uint16_t* w = p.wb + (int64_t)n * 2 * p.C + ch;
+      if ((reinterpret_cast<uintptr_t>(w) & 15) == 0) {  // (uniform: base alignment)
+        s[0] = *reinterpret_cast<const uint4*>(w);
+        b[0] = *reinterpret_cast<const uint4*>(w + p.C);
+      } else {
+        uint32_t t[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        wf[e] = bf16_bits_to_f32(w[e]);
-        fsh[e] = bf16_bits_to_f32(w[p.C + e]);
+        for (int e = 0; e < 4; ++e) {
+          t[e] = w[2 * e] | ((uint32_t)w[2 * e + 1] << 16);
+          t[4 + e] = w[p.C + 2 * e] | ((uint32_t)w[p.C + 2 * e + 1] << 16);
+        }
+        s[0] = uint4{t[0], t[1], t[2], t[3]};
+        b[0] = uint4{t[4], t[5], t[6], t[7]};
       }
     }
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const uint32_t pk = pack_bf16x2(wf[e] + 1.0f, wf[e + 1] + 1.0f);
-      fsc[e] = __uint_as_float(pk << 16);
-      fsc[e + 1] = __uint_as_float(pk & 0xffff0000u);
+  }
+  __device__ __forceinline__ bool get(const GnArgs& p, float (&fsc)[8], float (&fsh)[8]) const {
+    if (p.fs) {
+      floats8(s, fsc);
+      floats8(b, fsh);
+      return true;
     }
-    return true;
-  }
+    if (p.wb) {
+      float wf[8];
+      unpack8(s[0], wf);
+      unpack8(b[0], fsh);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    fsc[e] = 1.0f;
-    fsh[e] = 0.0f;
+      for (int e = 0; e < 8; e += 2) {
+        const uint32_t pk = pack_bf16x2(wf[e] + 1.0f, wf[e + 1] + 1.0f);
+        fsc[e] = __uint_as_float(pk << 16);
+        fsc[e + 1] = __uint_as_float(pk & 0xffff0000u);
+      }
+      return true;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      fsc[e] = 1.0f;
+      fsh[e] = 0.0f;
+    }
+    return false;
   }
-  return false;
+};
+
+__device__ __forceinline__ bool load_film(const GnArgs& p, int n, int ch, float (&fsc)[8],
+                                          float (&fsh)[8]) {
+  GnFilm f;
+  f.load(p, n, ch);
+  return f.get(p, fsc, fsh);
 }
 
 // Pixel loop of a pass: lane pl visits pixels pl, pl + PLN, ... in groups of U whose 16-B
@@ -601,11 +657,12 @@ __device__ __forceinline__ void unpack_x(const uint4 (&v)[NL][U], int u, float (
 struct GnQ {
   float s = 1.0f, r = 0.0f;
   us2 acc = {0, 0};
+  // (made before a kernel's pixels are loaded, set up after: see GnFilm)
   __device__ __forceinline__ explicit GnQ(const GnArgs& p) {
-    if (p.q) {
-      s = *p.q_scale;
-      r = quant_recip(s);
-    }
+    if (p.q) s = *p.q_scale;
+  }
+  __device__ __forceinline__ void setup(const GnArgs& p) {
+    if (p.q) r = quant_recip(s);
   }
   // the 8 bf16 values v of element offset off
   __device__ __forceinline__ void put(const GnArgs& p, int64_t off, uint4 v) {
@@ -692,16 +749,39 @@ __device__ __forceinline__ void finish_xb_amax(const GnArgs& p, us2 acc, uint32_
   store_amax_partial(acc, red, p.xb_part, nullptr, blk, gridDim.x * gridDim.y * gridDim.z);
 }
 
+// The channel constants of this thread's 8 channels (gamma, beta, FiLM) and, for the backward,
+// their groups' mean and rstd: loaded before a kernel's pixels, looked at after (see GnFilm).
+template <bool kFilm, bool kStats>
+struct GnChan {
+  uint4 g[2], b[2];
+  GnFilm film;
+  float mu[2], rs[2];
+  __device__ __forceinline__ GnChan(const GnArgs& p, int n, int ch) {
+    load8raw(p.gamma + ch, g);
+    load8raw(p.beta + ch, b);
+    if (kFilm) film.load(p, n, ch);
+    if (kStats) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int gi = n * p.G + (ch + 4 * h) / p.cpg;
+        mu[h] = p.mean[gi];
+        rs[h] = p.rstd[gi];
+      }
+    }
+  }
+};
+
 // The forward's per-channel affine of this thread's 8 channels: out = silu(x A + B) with
 // A = rstd gamma and B = beta - mean A, both times the FiLM scale (plus its shift in B) --
 // normalise, affine and FiLM in one fma per element.
 template <bool kFilm>
-__device__ __forceinline__ void fwd_affine(const GnArgs& p, int n, int ch, const float (&mu)[2],
-                                           const float (&rs)[2], float (&A)[8], float (&B)[8]) {
-  float fsc[8], fsh[8], gm[8], bt[8];
-  if (kFilm) load_film(p, n, ch, fsc, fsh);
-  load8f(p.gamma + ch, gm);
-  load8f(p.beta + ch, bt);
+__device__ __forceinline__ void fwd_affine(const GnArgs& p, const GnChan<kFilm, false>& k,
+                                           const float (&mu)[2], const float (&rs)[2],
+                                           float (&A)[8], float (&B)[8]) {
+  float gm[8], bt[8], fsc[8], fsh[8];
+  floats8(k.g, gm);
+  floats8(k.b, bt);
+  if (kFilm) k.film.get(p, fsc, fsh);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float a = rs[e >> 2] * gm[e];
@@ -714,17 +794,18 @@ __device__ __forceinline__ void fwd_affine(const GnArgs& p, int n, int ch, const
 // 8 outputs silu(f A + B) (dropout: kept ones times drop_scale, the rest 0), packed bf16
 template <bool kDrop>
 __device__ __forceinline__ uint4 fwd_out8(const float (&f)[8], const float (&A)[8],
-                                          const float (&B)[8], uint32_t keep, float drop_scale) {
+                                          const float (&B)[8], uint4 mask, float drop_scale) {
   float z[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float t = __builtin_fmaf(f[e], A[e], B[e]);
     float o = t * sigmoid_hw(t);
-    if (kDrop) o = (keep >> e) & 1u ? o * drop_scale : 0.0f;
+    if (kDrop) o = o * drop_scale;
     z[e] = o;
   }
-  return uint4{pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3]), pack_bf16x2(z[4], z[5]),
-               pack_bf16x2(z[6], z[7])};
+  const uint4 o = uint4{pack_bf16x2(z[0], z[1]), pack_bf16x2(z[2], z[3]), pack_bf16x2(z[4], z[5]),
+                        pack_bf16x2(z[6], z[7])};
+  return kDrop ? and4(o, mask) : o;
 }
 
 __device__ __forceinline__ int chunk_pixels(int HW, int chunk) {
@@ -812,6 +893,8 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_apply_kernel(const GnArgs
   const int gq = threadIdx.x & 7;
   const int pl = threadIdx.x >> 3;
   const int ch = c0 + gq * 8;
+  const GnChan<kFilm, false> kc(p, n, ch);
+  GnQ qo(p);
   const GnSrc<kF32, false> in(p, (int64_t)n * p.HW * p.C + ch);
   uint4 v[in.kN][kChU];
   bool ok[kChU];
@@ -855,10 +938,10 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_apply_kernel(const GnArgs
     rs[h] = st.y;
   }
   float A[8], B[8];
-  fwd_affine<kFilm>(p, n, ch, mu, rs, A, B);
+  fwd_affine<kFilm>(p, kc, mu, rs, A, B);
   uint16_t* ob = static_cast<uint16_t*>(p.out) + (int64_t)n * p.HW * p.C + ch;
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
-  GnQ qo(p);
+  qo.setup(p);
   us2 xacc = {0, 0};
 #pragma unroll
   for (int u = 0; u < kChU; ++u) {
@@ -868,8 +951,8 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_apply_kernel(const GnArgs
     if constexpr (kF32) {
       if (p.x_bf16 && ok[u]) xacc = absmax8(xacc, store_x_bf16(p, off, f));
     }
-    const uint32_t kb = kDrop ? drop_keep8(seed, off, p.drop_keep) : 0u;
-    const uint4 o = fwd_out8<kDrop>(f, A, B, kb, p.drop_scale);
+    const uint4 mk = kDrop ? drop_mask8(drop_z(seed, off), drop_keep2(p)) : uint4{};
+    const uint4 o = fwd_out8<kDrop>(f, A, B, mk, p.drop_scale);
     if (ok[u]) {
       if (p.q)
         qo.put(p, off, o);
@@ -905,41 +988,30 @@ __device__ __forceinline__ void bwd_terms(const float (&f)[8], const float (&d)[
   }
 }
 
-// dout of 8 channels, masked and scaled by the forward's dropout
+// dout of 8 channels, masked and scaled by the forward's dropout; z: its hash input
 template <bool kDrop>
-__device__ __forceinline__ void bwd_dout(uint4 v, uint64_t seed, int64_t off, const GnArgs& p,
-                                         float (&d)[8]) {
-  unpack8(v, d);
-  if (kDrop) {
-    const uint32_t kb = drop_keep8(seed, off, p.drop_keep);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) d[e] = (kb >> e) & 1u ? d[e] * p.drop_scale : 0.0f;
-  }
-}
-
-// the same with the keep bits already formed (the resident backward hashes once per pixel)
-template <bool kDrop>
-__device__ __forceinline__ void bwd_dout_kb(uint4 v, uint32_t kb, float drop_scale,
-                                            float (&d)[8]) {
+__device__ __forceinline__ void bwd_dout(uint4 v, uint64_t z, const GnArgs& p, float (&d)[8]) {
+  if (kDrop) v = and4(v, drop_mask8(z, drop_keep2(p)));
   unpack8(v, d);
   if (kDrop) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) d[e] = drop_sel(d[e], kb, e, drop_scale);
+    for (int e = 0; e < 8; ++e) d[e] = d[e] * p.drop_scale;
   }
 }
 
 template <bool kFilm>
-__device__ __forceinline__ void gn_bwd_setup(const GnArgs& p, int n, int ch, GnBwdSetup& st) {
+__device__ __forceinline__ void gn_bwd_setup(const GnArgs& p, const GnChan<kFilm, true>& k,
+                                             GnBwdSetup& st) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int g = (ch + 4 * h) / p.cpg;
-    st.mu[h] = p.mean[n * p.G + g];
-    st.rs[h] = p.rstd[n * p.G + g];
+    st.mu[h] = k.mu[h];
+    st.rs[h] = k.rs[h];
+    st.nmr[h] = -st.mu[h] * st.rs[h];
   }
-  load8f(p.gamma + ch, st.gm);
-  load8f(p.beta + ch, st.bt);
+  floats8(k.g, st.gm);
+  floats8(k.b, st.bt);
   if (kFilm) {
-    load_film(p, n, ch, st.fsc, st.fsh);
+    k.film.get(p, st.fsc, st.fsh);
   } else {  // compile-time identity: the FiLM terms fold away
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -947,8 +1019,6 @@ __device__ __forceinline__ void gn_bwd_setup(const GnArgs& p, int n, int ch, GnB
       st.fsh[e] = 0.0f;
     }
   }
-#pragma unroll
-  for (int h = 0; h < 2; ++h) st.nmr[h] = -st.mu[h] * st.rs[h];
 #pragma unroll
   for (int e = 0; e < 8; ++e) st.gC[e] = kFilm ? st.fsc[e] * st.gm[e] : st.gm[e];
 }
@@ -969,13 +1039,14 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_sums_kernel(const GnA
   const int ch = c0 + gq * 8;
   const int64_t base = (int64_t)n * p.HW * p.C + ch;
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
+  const GnChan<kFilm, true> kc(p, n, ch);
   const GnSrc<kF32, true> in(p, base);
   uint4 v[in.kN][kChU];
   bool ok[kChU];
   int pxs[kChU];
   chunk_load(in.src, in.stride, chunk * kChunkPx, pl, p.HW, v, ok, pxs);
   GnBwdSetup st;
-  gn_bwd_setup<kFilm>(p, n, ch, st);
+  gn_bwd_setup<kFilm>(p, kc, st);
   float acc[NS];
 #pragma unroll
   for (int k = 0; k < NS; ++k) acc[k] = 0.f;
@@ -983,7 +1054,7 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_sums_kernel(const GnA
   for (int u = 0; u < kChU; ++u) {
     float f[8], d[8], xh[8], g[8];
     unpack_x<kF32>(v, u, f);
-    bwd_dout<kDrop>(v[in.kN - 1][u], seed, base + (int64_t)pxs[u] * p.C, p, d);
+    bwd_dout<kDrop>(v[in.kN - 1][u], kDrop ? drop_z(seed, base + (int64_t)pxs[u] * p.C) : 0, p, d);
     bwd_terms<kFilm>(f, d, st, xh, g);
     if (ok[u]) {
 #pragma unroll
@@ -1023,14 +1094,16 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_apply_kernel(const Gn
   const int ch = c0 + gq * 8;
   const int64_t base = (int64_t)n * p.HW * p.C + ch;
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
+  const GnChan<kFilm, true> kc(p, n, ch);
+  GnQ qo(p);
   const GnSrc<kF32, true> in(p, base);
   uint4 v[in.kN][kChU];
   bool ok[kChU];
   int pxs[kChU];
   chunk_load(in.src, in.stride, chunk * kChunkPx, pl, p.HW, v, ok, pxs);
   GnBwdSetup st;
-  gn_bwd_setup<kFilm>(p, n, ch, st);
-  GnQ qo(p);
+  gn_bwd_setup<kFilm>(p, kc, st);
+  qo.setup(p);
 
   // channel totals over the chunks: four interleaved slices of chunks per channel (loads
   // in flight together), then the slices in order (deterministic)
@@ -1103,7 +1176,7 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_apply_kernel(const Gn
   for (int u = 0; u < kChU; ++u) {
     float f[8], d[8], xh[8], g[8];
     unpack_x<kF32>(v, u, f);
-    bwd_dout<kDrop>(v[in.kN - 1][u], seed, base + (int64_t)pxs[u] * p.C, p, d);
+    bwd_dout<kDrop>(v[in.kN - 1][u], kDrop ? drop_z(seed, base + (int64_t)pxs[u] * p.C) : 0, p, d);
     bwd_terms<kFilm>(f, d, st, xh, g);
     auto dx = [&](int e) __attribute__((always_inline)) {
       const int h = e >> 2;
@@ -1213,6 +1286,9 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
   const int gq = threadIdx.x & 7;
   const int pl = threadIdx.x >> 3;
   const int ch = c0 + gq * 8;
+  const GnChan<kFilm, false> kc(p, n, ch);
+  GnQ qo(p);
+  const uint64_t seed = kDrop ? *p.drop_seed : 0;
   const GnSrc<kF32, false> in(p, (int64_t)n * p.HW * p.C + ch);
   uint4 v[in.kN][U];
   bool ok[U];
@@ -1246,6 +1322,20 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
       if (p.xb_part) finish_xb_amax(p, xacc, qred);
     }
   }
+  // the dropout masks, hashed while the loads are in flight (beside 128 registers of fp32 x: at
+  // their use)
+  constexpr bool kEarly = kDrop && !(kF32 && U >= 16);
+  const uint64_t z0 = kDrop ? drop_z(seed, ((int64_t)n * p.HW + pl) * p.C + ch) : 0;
+  const uint64_t zs = (uint64_t)(PLN * p.C / 4) * kDropGolden;  // per pixel of the lane
+  auto mask_of = [&](int u) __attribute__((always_inline)) {
+    return kDrop ? drop_mask8(z0 + (uint64_t)u * zs, drop_keep2(p)) : uint4{};
+  };
+  uint4 mask[kEarly ? U : 1];
+  if constexpr (kEarly) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) mask[u] = mask_of(u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   float sm[2] = {0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < U; ++u)
@@ -1265,10 +1355,19 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
   const float mu[2] = {group_sum(hs, 2 * gq, p.cpg) * inv_cnt,
                        group_sum(hs, 2 * gq + 1, p.cpg) * inv_cnt};
   __syncthreads();
+  // with the masks held too, the unpacked values do not fit beside the packed ones: each pass
+  // unpacks again (hidden from the compiler)
+  auto reopen = [&](int u) __attribute__((always_inline)) {
+    if constexpr (kDrop && U >= 16) {
+#pragma unroll
+      for (int l = 0; l < in.kN; ++l) opaque_u4(v[l][u]);
+    }
+  };
   float q[2] = {0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < U; ++u)
     if (ok[u]) {
+      reopen(u);
       float f[8];
       unpack_x<kF32>(v, u, f);
 #pragma unroll
@@ -1297,17 +1396,17 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
     }
   }
   float A[8], B[8];
-  fwd_affine<kFilm>(p, n, ch, mu, rs, A, B);
+  fwd_affine<kFilm>(p, kc, mu, rs, A, B);
   uint16_t* ob = static_cast<uint16_t*>(p.out) + (int64_t)n * p.HW * p.C + ch;
-  const uint64_t seed = kDrop ? *p.drop_seed : 0;
-  GnQ qo(p);
+  qo.setup(p);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
+    reopen(u);
     float f[8];
     unpack_x<kF32>(v, u, f);
     const int64_t off = ((int64_t)n * p.HW + pxs[u]) * p.C + ch;
-    const uint32_t kb = kDrop ? drop_keep8(seed, off, p.drop_keep) : 0u;
-    const uint4 o = fwd_out8<kDrop>(f, A, B, kb, p.drop_scale);
+    const uint4 o = fwd_out8<kDrop>(f, A, B, kEarly ? mask[kEarly ? u : 0] : mask_of(u),
+                                    p.drop_scale);
     if (ok[u]) {
       if (p.q)
         qo.put(p, off, o);
@@ -1318,26 +1417,26 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
   if (p.q) qo.finish(p, qred);
 }
 
-// The backward keeps x in registers and, at 16 pixels per lane (where x and dout together
-// would exceed the register file), dout in LDS: DMA'd there at the start (lane i of a wave's
-// u-th transfer at 16-B slot u * 8 PLN + thread), read back by the same thread in both passes.
-template <int PLN, int U>
-struct GnResDout {
-  static constexpr bool kLds = U >= 16;
-  static constexpr int kBytes = kLds ? U * 8 * PLN * 16 : 16;
-};
+// The backward keeps x in registers (packed) and the fp32 g of every pixel, formed in the first
+// pass as the loads arrive: the sigmoid's exp2 and reciprocal, which issue at a quarter rate,
+// and the dropout hash are its largest costs and run once. At 16 pixels per lane, whose x and
+// g take 192 registers (fp32 x: 256), the first few pixels' g lie in LDS. 128 images of 32x32 x
+// 128 bf16 with FiLM and dropout: 41.3 us with g formed in both passes and dout in LDS, 33.2 so.
+template <int U, bool kFilm, bool kF32, bool kCat>
+constexpr int kGnResLdsG = U < 16 ? 0 : (kF32 ? 9 : (kCat ? 8 : (kFilm ? 6 : 3)));
 
 template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false>
 __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
   static_assert(!kCat || (!kF32 && PLN == 64 && U == 16) || (kF32 && PLN == 32 && U == 8),
                 "32x32 images (bf16 sources) or 16x16 (cat_h bf16 or fp32)");
-  using DL = GnResDout<PLN, U>;
-  __shared__ __attribute__((aligned(16))) uint8_t dls[DL::kBytes];
+  constexpr int kGL = kGnResLdsG<U, kFilm, kF32, kCat>;
+  __shared__ __attribute__((aligned(16))) uint8_t gls[kGL ? kGL * 2 * 8 * PLN * 16 : 16];
   __shared__ uint32_t qred[PLN / 8];
   __shared__ float red[(PLN / 8) * 8 * 16];
   __shared__ float hs[2][16];
-  // kCat without the dout copy in LDS: four pixel rows of the 2x2 window exchange
-  __shared__ __attribute__((aligned(16))) float xch[kCat && !DL::kLds ? 4 * (PLN / 4) * 8 * 16 : 4];
+  // kCat: the pixel rows of one 2x2 window exchange
+  constexpr int kXR = U >= 16 ? 2 : 4;
+  __shared__ __attribute__((aligned(16))) float xch[kCat ? kXR * (PLN / 4) * 8 * 16 : 4];
   const int n = blockIdx.y;
   const int c0 = blockIdx.x * kSlab;
   const int gq = threadIdx.x & 7;
@@ -1345,46 +1444,33 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
   const int ch = c0 + gq * 8;
   const int64_t base = (int64_t)n * p.HW * p.C + ch;
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
-  // x (and, without the LDS copy, dout) in registers
-  const GnSrc<kF32, !DL::kLds> in(p, base);
+  const GnChan<kFilm, true> kc(p, n, ch);
+  GnQ qo(p);
+  const GnSrc<kF32, true> in(p, base);
   uint4 v[in.kN][U];
   bool ok[U];
   int pxs[U];
   if constexpr (kCat) {
-    cat_load<in.kN, PLN, U, kF32, !DL::kLds>(p, n, ch, pl, v, ok, pxs);
+    cat_load<in.kN, PLN, U, kF32, true>(p, n, ch, pl, v, ok, pxs);
   } else {
     res_load<in.kN, PLN, U>(in.src, in.stride, pl, p.HW, v, ok, pxs);
   }
-  if constexpr (DL::kLds) {
-    const uint32_t lbase =
-        __builtin_amdgcn_readfirstlane(LDS_ADDR(dls) + (uint32_t)(threadIdx.x & ~63) * 16);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      dma16_lds(p.dout + base + (int64_t)pxs[u] * p.C, lbase + (uint32_t)(u * 8 * PLN * 16));
-    wait_vmcnt<0>();
-    asm volatile("" ::: "memory");  // the DMA writes are invisible to the compiler
-  }
-  // dout of pixel u
-  auto dout_u = [&](int u) __attribute__((always_inline)) {
-    if constexpr (DL::kLds)
-      return *reinterpret_cast<const uint4*>(dls + (u * 8 * PLN + threadIdx.x) * 16);
-    else
-      return v[in.kN - 1][u];
-  };
   GnBwdSetup st;
-  gn_bwd_setup<kFilm>(p, n, ch, st);
-  GnQ qo(p);
+  gn_bwd_setup<kFilm>(p, kc, st);
   // per-channel S1 = sum g, S2 = sum g * xhat over the image (every lane gets the totals)
   float acc[16];
 #pragma unroll
   for (int k = 0; k < 16; ++k) acc[k] = 0.f;
-  uint32_t keep[U];  // the dropout keep bits of each pixel, hashed once for both passes
+  // hash input of the lane's first pixel, and its step from one pixel of the lane to the next
+  const uint64_t z0 = kDrop ? drop_z(seed, base + (int64_t)pl * p.C) : 0;
+  const uint64_t zs = (uint64_t)(PLN * p.C / 4) * kDropGolden;
+  float gk[U][8];
+  v4f* gl = reinterpret_cast<v4f*>(gls) + threadIdx.x;  // pixel u < kGL: entries 2u, 2u + 1
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     float f[8], d[8], xh[8], g[8];
     unpack_x<kF32>(v, u, f);
-    keep[u] = kDrop ? drop_keep8(seed, base + (int64_t)pxs[u] * p.C, p.drop_keep) : 0u;
-    bwd_dout_kb<kDrop>(dout_u(u), keep[u], p.drop_scale, d);
+    bwd_dout<kDrop>(v[in.kN - 1][u], z0 + (uint64_t)u * zs, p, d);
     bwd_terms<kFilm>(f, d, st, xh, g);
     if (ok[u]) {
 #pragma unroll
@@ -1393,11 +1479,20 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
         acc[8 + e] += g[e] * xh[e];
       }
     }
+    if (u < kGL) {
+      gl[(2 * u) * 8 * PLN] = v4f{g[0], g[1], g[2], g[3]};
+      gl[(2 * u + 1) * 8 * PLN] = v4f{g[4], g[5], g[6], g[7]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) gk[u][e] = g[e];
+    }
     // one pixel at a time: the packed inputs stay resident, each pixel's unpacked terms die
     // before the next pixel's are formed (else the interleaved pixels exceed the registers)
     __builtin_amdgcn_sched_barrier(0);
   }
+  const GnChan<kFilm, true> kc2(p, n, ch);  // (again, not kept across the pixels)
   slab_reduce<16, PLN>(acc, red);
+  gn_bwd_setup<kFilm>(p, kc2, st);
   if (pl == 0) {
     const int64_t nc = (int64_t)p.N * p.C;
     float h1[2] = {0.f, 0.f}, h2[2] = {0.f, 0.f};
@@ -1435,18 +1530,21 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     m1[h] = group_sum(hs[0], 2 * gq + h, p.cpg) * inv_cnt;
     m2[h] = group_sum(hs[1], 2 * gq + h, p.cpg) * inv_cnt;
   }
-  // pixel u's dx (the fused concatenation's form; the loop below is the same per pixel)
+  qo.setup(p);
+  // pixel u's dx. The second pass unpacks x again from the packed registers: hidden from the
+  // compiler, which would otherwise keep the first pass's unpacked values of every pixel alive
+  // across the reduction (8 registers per pixel more)
   auto pixel_dx = [&](int u, float (&t)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int l = 0; l < in.kN; ++l) opaque_u4(v[l][u]);
-    float f[8], d[8], xh[8], g[8];
+    for (int l = 0; l < in.kX; ++l) opaque_u4(v[l][u]);
+    float f[8];
     unpack_x<kF32>(v, u, f);
-    bwd_dout_kb<kDrop>(dout_u(u), keep[u], p.drop_scale, d);
-    bwd_terms<kFilm>(f, d, st, xh, g);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int h = e >> 2;
-      t[e] = st.rs[h] * __builtin_fmaf(-xh[e], m2[h], g[e] * st.gC[e] - m1[h]);
+      const float xh = __builtin_fmaf(f[e], st.rs[h], st.nmr[h]);
+      const float g = u < kGL ? gl[(2 * u + h) * 8 * PLN][e & 3] : gk[u][e];
+      t[e] = st.rs[h] * __builtin_fmaf(-xh, m2[h], g * st.gC[e] - m1[h]);
     }
   };
   if constexpr (kCat) {
@@ -1457,21 +1555,18 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     // images are PLN / 2 wide, so pixel pl + PLN u is row 2u + pl / kW, column pl mod kW:
     // window (u, j) holds lanes 2j, 2j + 1 (row 2u) and 2j + kW, 2j + kW + 1 (row 2u + 1). The
     // odd lane's value comes by a shuffle (8 threads on), the lower row's two through LDS
-    // (the dout slots already read, or an exchange buffer), four pixels per exchange.
+    // (an exchange buffer), four pixels per exchange.
     constexpr int kW = PLN / 2;
     constexpr int kEnt = (kW / 2) * 8 * 16;  // floats per pixel row pair: (window, granule) x 16
     const bool in_a = ch < p.cat_ca;  // workgroup-uniform
     const bool even = (pl & 1) == 0;
-    float* xs = DL::kLds ? reinterpret_cast<float*>(dls) : xch;
-    constexpr int kSlot = DL::kLds ? 8 * PLN * 4 : kEnt;  // floats between pixel rows u
-    static_assert(kEnt <= kSlot, "an exchange fits a dout slot");
     bool hf = false;
     if constexpr (kF32) hf = p.cat_hf != 0;
 #pragma unroll
-    for (int u0 = 0; u0 < U; u0 += 4) {
-      float t[4][8];
+    for (int u0 = 0; u0 < U; u0 += kXR) {
+      float t[kXR][8];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < kXR; ++k) {
         const int u = u0 + k;
         pixel_dx(u, t[k]);
         if (p.dx_add) {
@@ -1499,18 +1594,18 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
         __builtin_amdgcn_sched_barrier(0);
       }
       if (in_a) {
-        __syncthreads();  // every thread has read the dout slots u0 .. u0 + 3 (or the buffer)
-        float r[4][8];  // the odd neighbour's values (lane + 8: pixel lane pl + 1)
+        __syncthreads();  // every thread has read the buffer
+        float r[kXR][8];  // the odd neighbour's values (lane + 8: pixel lane pl + 1)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < kXR; ++k)
 #pragma unroll
           for (int e = 0; e < 8; ++e) r[k][e] = __shfl_down(t[k][e], 8, 64);
         // row u0 + k, entry (window column j, granule gq): row 2u + 1's pair, 16 floats
         const int ent = (((pl % kW) >> 1) * 8 + gq) * 16;
         if (pl >= kW && even) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float* e0 = xs + (DL::kLds ? u0 + k : k) * kSlot + ent;
+          for (int k = 0; k < kXR; ++k) {
+            float* e0 = xch + k * kEnt + ent;
 #pragma unroll
             for (int q4 = 0; q4 < 2; ++q4) {
               *reinterpret_cast<v4f*>(e0 + 4 * q4) =
@@ -1523,8 +1618,8 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
         __syncthreads();
         if (pl < kW && even) {
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const float* e0 = xs + (DL::kLds ? u0 + k : k) * kSlot + ent;
+          for (int k = 0; k < kXR; ++k) {
+            const float* e0 = xch + k * kEnt + ent;
             float acc[8];
 #pragma unroll
             for (int q4 = 0; q4 < 2; ++q4) {
@@ -1548,26 +1643,20 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
                     uint4{w[0], w[1], w[2], w[3]});
           }
         }
-        // (the buffer's next writes come after the next four pixels' first barrier)
+        // (the buffer's next writes come after the next pixels' first barrier)
       }
     }
   } else {
+    // (the pixel numbers formed again, not kept across the reduction)
+    int pl2 = pl;
+    asm volatile("" : "+v"(pl2));
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // the second pass forms the per-pixel terms again from the packed registers: hidden
-      // from the compiler, which would otherwise keep the first pass's unpacked terms of
-      // every pixel alive across the reduction (8-16 registers per pixel more)
-#pragma unroll
-      for (int l = 0; l < in.kN; ++l) opaque_u4(v[l][u]);
-      float f[8], d[8], xh[8], g[8];
-      unpack_x<kF32>(v, u, f);
-      bwd_dout_kb<kDrop>(dout_u(u), keep[u], p.drop_scale, d);
-      bwd_terms<kFilm>(f, d, st, xh, g);
-      auto dx = [&](int e) __attribute__((always_inline)) {
-        const int h = e >> 2;
-        return st.rs[h] * __builtin_fmaf(-xh[e], m2[h], g[e] * st.gC[e] - m1[h]);
-      };
-      if (ok[u]) store_dx<kF32>(p, base + (int64_t)pxs[u] * p.C, dx, qo);
+      float t[8];
+      pixel_dx(u, t);
+      auto dx = [&](int e) __attribute__((always_inline)) { return t[e]; };
+      const int px = pl2 + u * PLN;
+      if (px < p.HW) store_dx<kF32>(p, base + (int64_t)px * p.C, dx, qo);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
@@ -1585,8 +1674,7 @@ static GnRes gn_res_shape(int HW) {
   if (HW <= kResMaxHW) return {64, 16};
   return {0, 0};
 }
-// The backward with an fp32 x holds 2 x 16 B of x per pixel in registers (dout goes to LDS at
-// 16 pixels per lane): that fits at 16 pixels per lane without FiLM and dropout (their
+// The backward with an fp32 x holds 2 x 16 B of x per pixel in registers: that fits at 16 pixels per lane without FiLM and dropout (their
 // per-channel terms and keep bits are the registers that do not fit); with them, images
 // above 256 pixels take the chunked form.
 static bool gn_res_bwd_ok(int HW, bool x_f32, bool film, bool drop) {
