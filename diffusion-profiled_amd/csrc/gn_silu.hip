@@ -1275,8 +1275,13 @@ __device__ __forceinline__ void cat_load(const GnArgs& p, int n, int ch, int pl,
   }
 }
 
+// Each pass unpacks x from the packed registers again and the pixel numbers are formed again at
+// the end, so that at 16 pixels per lane of bf16 x two workgroups fit a CU (128 registers) and
+// one's loads run under the other's arithmetic: the two-source form at 32x32 x 512 (2048
+// workgroups) 111 -> 94 us. With dropout the masks hashed under the loads take that room instead
+// (256 workgroups: 22.4 us with two per CU and the hash at the end, 20.4 so).
 template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false>
-__global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
+__global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void gn_res_fwd_kernel(const GnArgs p) {
   static_assert(!kCat || PLN * U == 1024 || (kF32 && PLN * U == 256), "32x32 or 16x16 images");
   __shared__ uint32_t qred[PLN / 8];
   __shared__ float red[(PLN / 8) * 8 * 2];
@@ -1358,7 +1363,7 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
   // with the masks held too, the unpacked values do not fit beside the packed ones: each pass
   // unpacks again (hidden from the compiler)
   auto reopen = [&](int u) __attribute__((always_inline)) {
-    if constexpr (kDrop && U >= 16) {
+    if constexpr (U >= 16 && !kF32) {
 #pragma unroll
       for (int l = 0; l < in.kN; ++l) opaque_u4(v[l][u]);
     }
@@ -1399,20 +1404,24 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_fwd_kernel(const GnArgs p) {
   fwd_affine<kFilm>(p, kc, mu, rs, A, B);
   uint16_t* ob = static_cast<uint16_t*>(p.out) + (int64_t)n * p.HW * p.C + ch;
   qo.setup(p);
+  // (the pixel numbers formed again, not kept across the reductions)
+  int pl2 = pl;
+  asm volatile("" : "+v"(pl2));
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     reopen(u);
     float f[8];
     unpack_x<kF32>(v, u, f);
-    const int64_t off = ((int64_t)n * p.HW + pxs[u]) * p.C + ch;
+    const int px = pl2 + u * PLN;
     const uint4 o = fwd_out8<kDrop>(f, A, B, kEarly ? mask[kEarly ? u : 0] : mask_of(u),
                                     p.drop_scale);
-    if (ok[u]) {
+    if (px < p.HW) {
       if (p.q)
-        qo.put(p, off, o);
+        qo.put(p, ((int64_t)n * p.HW + px) * p.C + ch, o);
       else
-        st_nt16(ob + (int64_t)pxs[u] * p.C, o);
+        st_nt16(ob + (int64_t)px * p.C, o);
     }
+    if constexpr (U >= 16) __builtin_amdgcn_sched_barrier(0);
   }
   if (p.q) qo.finish(p, qred);
 }
