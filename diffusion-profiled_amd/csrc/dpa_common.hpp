@@ -128,6 +128,26 @@ __device__ __forceinline__ uint2 quant8_rcp(uint4 v, float scale, float r) {
   return o;
 }
 
+// The same bytes for a current-scaling cast of a finite tensor (no NaN or infinity in it): then
+// |x| <= amax, so the quotient is at most 448 (1 + 2^-24), which rounds to 448 unclamped, and q0
+// is finite; and a zero result takes its sign from x, as the quotient's. 5.5 vector
+// instructions per element instead of 9.5.
+__device__ __forceinline__ uint2 quant8_finite(uint4 v, float scale, float r) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  float f[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x = __uint_as_float(i & 1 ? w[i >> 1] & 0xffff0000u : w[i >> 1] << 16);
+    const float q0 = x * r;
+    const float e = __builtin_fmaf(-q0, scale, x);
+    f[i] = __builtin_copysignf(__builtin_fmaf(e, r, q0), x);
+  }
+  uint2 o;
+  o.x = pack4_e4m3(f[0], f[1], f[2], f[3]);
+  o.y = pack4_e4m3(f[4], f[5], f[6], f[7]);
+  return o;
+}
+
 // 8 bf16 (one uint4) -> 8 e4m3 bytes (one uint2).
 __device__ __forceinline__ uint2 quant8(uint4 v, float scale) {
   const uint32_t w[4] = {v.x, v.y, v.z, v.w};

@@ -109,6 +109,25 @@ def test_special_values(K):
     check_current(K, torch.from_numpy(np.arange(1, 128, dtype=np.int16)).view(torch.bfloat16))
 
 
+@pytest.mark.parametrize("amax", [0x0001, 0x1F80, 0x2001, 0x3F80, 0x43E0, 0x4111, 0x7B7F, 0x7F7F])
+@pytest.mark.parametrize("size", ["grid", "deep", "deep+tail"])
+def test_every_bf16_value_through_both_cast_loops(K, amax, size):
+    """Every bf16 value of magnitude up to ``amax`` (both zeros, subnormals, scales on both
+    sides of the fast quotient's range) through the finite cast: one group per thread, and 2 x 4
+    or more groups per thread over 1024 workgroups, where the loads run ahead of the casts, with
+    whole and ragged ends. Bytes and scale are the oracle's."""
+    mags = np.arange(amax + 1, dtype=np.uint16)
+    u = np.concatenate([mags, mags | 0x8000])
+    q_ref, s_ref = O.quantize_fp8(u)
+    deep = 8 * 1024 * 256 * 8
+    n = {"grid": max(len(u), 20000), "deep": deep, "deep+tail": deep + 4 * 1024 * 2048 + 77}[size]
+    ut = torch.from_numpy(u.view(np.int16)).view(torch.bfloat16).cuda()
+    idx = torch.arange(n, device="cuda") % len(u)
+    q, s = K.quantize_fp8_tensor(ut[idx].contiguous())
+    assert np.float32(s.item()) == s_ref
+    assert torch.equal(q.view(torch.uint8), torch.from_numpy(q_ref).cuda()[idx])
+
+
 def test_delayed(K):
     x = randn_bf16((128, 128, 32, 32), seed=0)
     xb = bits(x)
