@@ -1,4 +1,4 @@
-// FP8 weight gradient of a 3x3 / stride-1 / pad-1 convolution for images W = 16 or 32 pixels
+// FP8 weight gradient of a 3x3 / stride-1 / pad-1 convolution for images a multiple of 8 pixels
 // wide: one workgroup computes the three taps of one kernel row, so each K-step's operand
 // blocks feed three times the MFMAs of a one-tap tile.
 //
@@ -28,9 +28,9 @@ constexpr int kHwThreads = 512;
 constexpr int kHwCi = 64;                              // input channels per tile
 constexpr int kHwCo = 128;                             // output channels per tile
 constexpr int kHwPix = 128;                            // output pixels per K-step
-constexpr int kHwXBytes = 9216;                        // x block: max over W of (128/W)(W+2) x 64 B
+constexpr int kHwXBytes = 10240;                       // x block: max over W of (128/W)(W+2) x 64 B
 constexpr int kHwDyBytes = kHwPix * kHwCo;             // 16 KB
-constexpr int kHwStageBytes = kHwXBytes + kHwDyBytes;  // 25 KB
+constexpr int kHwStageBytes = kHwXBytes + kHwDyBytes;  // 26 KB
 constexpr int kHwStages = 6;
 constexpr int kHwDyLoads = kHwDyBytes / 16 / 256;      // 4 dy DMAs per producer thread
 constexpr int kHwXLoads = kHwPix * kHwCi / 16 / 256;   // 2 x DMAs per producer thread
@@ -46,7 +46,7 @@ struct HwgradArgs {
   const uint8_t* x;   // [N][H][W][Cin]
   const uint8_t* dy;  // [N][H][W][Cout]
   float* partial;     // [splits][Cout][9 * Cin]
-  int N, H, Cin, Cout;
+  int N, H, W, Cin, Cout;
   int nchunks, splits, tiles, ci_tiles, total, per_xcd;
 };
 
@@ -188,7 +188,94 @@ __device__ __forceinline__ void hw_issue(const HwgradArgs& p, HwRows& r, bool li
   }
 }
 
+// The producers of a strip (kStrip: every image that is not exactly one tile row wide or whose
+// height a step does not divide). A K-step is a tile of RO = 128 / W rows x W columns of the
+// N * H image rows, strips of the row left to right; its x block has the W + 2 columns around
+// the tile, out-of-image ones and rows from the zero page, in 16-pixel transfers whose lanes
+// gather from anywhere: 9 of them (10 for W = 8), two per wave and the last one or two by the
+// first waves.
 template <int W>
+struct HwStrip {
+  static constexpr int RO = kHwPix / W;
+  static constexpr int kPx = RO * (W + 2);                     // x pixels of a step
+  static constexpr int kBlocks = (kPx + 15) / 16;
+  static constexpr int kExtra = kBlocks - 4 * kHwXLoads;       // waves with a third transfer
+  static_assert(kBlocks * 1024 <= kHwXBytes && kExtra >= 1 && kExtra <= 4, "x block");
+  uint32_t dyo[kHwDyLoads];
+  int dyg[kHwDyLoads];      // rows from the pixel's row to the end of the batch
+  int xo[kHwXLoads + 1];
+  int xg[kHwXLoads + 1];    // the same of the x pixel's output row; <= 0: no pixel
+  int xy[kHwXLoads + 1];    // its row in the image
+  int xc[kHwXLoads + 1];    // its column, relative to the strip
+  int x0;                   // the strip's first column
+
+  __device__ __forceinline__ HwStrip(const HwgradArgs& p, int chunk, int kr, int ci0, int co0,
+                                     int pw, int lane) {
+    const int strips = p.W / W, rows = p.N * p.H;
+    const int rb = chunk / strips;
+    x0 = (chunk - rb * strips) * W;
+    const int g0 = rb * RO;
+#pragma unroll
+    for (int j = 0; j < kHwDyLoads; ++j) {
+      const int r = pw * 32 + 8 * j + (lane >> 3);
+      const int g = (lane & 7) ^ hw_dyswz(r);
+      dyo[j] = (uint32_t)(((g0 + r / W) * p.W + x0 + r % W) * p.Cout + co0 + g * 16);
+      dyg[j] = rows - (g0 + r / W);
+    }
+#pragma unroll
+    for (int j = 0; j < kHwXLoads + 1; ++j) {
+      const int b = j < kHwXLoads ? 2 * pw + j : 4 * kHwXLoads + pw;
+      const int e = 16 * b + (lane >> 2);
+      const int row = e / (W + 2), col = e - row * (W + 2) - 1;
+      const int g = (lane & 3) ^ hw_xswz(e);
+      xc[j] = col;
+      xy[j] = (g0 + row) % p.H;
+      xg[j] = e < kPx ? rows - (g0 + row) : -0x40000000;
+      // may point outside x while the pixel is out of range; only used when valid
+      xo[j] = ((g0 + row + kr - 1) * p.W + x0 + col) * p.Cin + ci0 + 16 * g;
+    }
+  }
+
+  template <int ST>
+  __device__ __forceinline__ void issue(const HwgradArgs& p, bool live, int kr, int pw) {
+    const uint32_t st = LDS_ADDR(hw_smem) + ST * kHwStageBytes;
+    const bool wrap = x0 + W == p.W;  // the next tile begins the next row of strips
+    const int step = wrap ? (RO - 1) * p.W + W : W;  // pixels to the next tile
+#pragma unroll
+    for (int j = 0; j < kHwDyLoads; ++j) {
+      const uint8_t* src = live & (dyg[j] > 0) ? p.dy + dyo[j] : hw_zero16;
+      dma16_lds(src, st + kHwXBytes + (uint32_t)(pw * 32 + 8 * j) * 128);
+      dyo[j] += (uint32_t)(step * p.Cout);
+      dyg[j] -= wrap ? RO : 0;
+    }
+    const int yw = RO % p.H;
+#pragma unroll
+    for (int j = 0; j < kHwXLoads + 1; ++j) {
+      if (j == kHwXLoads && pw >= kExtra) break;
+      const int b = j < kHwXLoads ? 2 * pw + j : 4 * kHwXLoads + pw;
+      const bool ok = live & (xg[j] > 0) & ((unsigned)(xy[j] + kr - 1) < (unsigned)p.H) &
+                      ((unsigned)(x0 + xc[j]) < (unsigned)p.W);
+      const uint8_t* src = ok ? p.x + xo[j] : hw_zero16;
+      dma16_lds(src, st + (uint32_t)b * 1024);
+      xo[j] += step * p.Cin;
+      xg[j] -= wrap ? RO : 0;
+      int y = xy[j] + (wrap ? yw : 0);
+      xy[j] = y >= p.H ? y - p.H : y;
+    }
+    x0 = wrap ? 0 : x0 + W;
+  }
+
+  // until at most n stages of this wave's transfers are in flight
+  template <int N>
+  __device__ __forceinline__ void wait(int pw) const {
+    if (pw < kExtra)
+      wait_vmcnt<N * (kHwLoadsPerStage + 1)>();
+    else
+      wait_vmcnt<N * kHwLoadsPerStage>();
+  }
+};
+
+template <int W, bool kStrip>
 __global__ __launch_bounds__(kHwThreads, 1) void hwgrad_partial_kernel(const HwgradArgs p) {
   constexpr int RO = kHwPix / W;  // image rows per K-step
   const int logical = (blockIdx.x & 7) * p.per_xcd + (blockIdx.x >> 3);
@@ -212,7 +299,36 @@ __global__ __launch_bounds__(kHwThreads, 1) void hwgrad_partial_kernel(const Hwg
   const int wc = wave & 1;         // consumers: 32-channel half of the 64 input channels
   const int wo = (wave >> 1) & 1;  // consumers: 64-channel half of the 128 output channels
 
-  if (wave >= 4) {
+  if (kStrip && wave >= 4) {
+    // ---------------- producers of a strip ----------------
+    const int pw = wave - 4;
+    HwStrip<W> r(p, c_begin, kr, ci0, co0, pw, lane);
+    r.template issue<0>(p, 0 < nsteps, kr, pw);
+    r.template issue<1>(p, 1 < nsteps, kr, pw);
+    r.template issue<2>(p, 2 < nsteps, kr, pw);
+    r.template issue<3>(p, 3 < nsteps, kr, pw);
+    r.template issue<4>(p, 4 < nsteps, kr, pw);
+    r.template wait<4>(pw);  // stage 0 landed
+    lds_barrier();           // B0
+    // step s: wait for stage s + 1, barrier, refill the buffer of stage s - 1 with s + 5
+#define HW_PRODUCE(ST, S)                                                   \
+  do {                                                                      \
+    r.template wait<3>(pw);                                                 \
+    lds_barrier();                                                          \
+    r.template issue<(ST + 5) % kHwStages>(p, (S) + 5 < nsteps, kr, pw);    \
+  } while (0)
+    for (int s = 0; s < nsteps; s += 6) {
+      HW_PRODUCE(0, s);
+      if (s + 1 < nsteps) HW_PRODUCE(1, s + 1);
+      if (s + 2 < nsteps) HW_PRODUCE(2, s + 2);
+      if (s + 3 < nsteps) HW_PRODUCE(3, s + 3);
+      if (s + 4 < nsteps) HW_PRODUCE(4, s + 4);
+      if (s + 5 < nsteps) HW_PRODUCE(5, s + 5);
+    }
+#undef HW_PRODUCE
+    wait_vmcnt<0>();  // trailing DMAs land before LDS is reused
+    lds_barrier();
+  } else if (wave >= 4) {
     // ---------------- producers ----------------
     const int pw = wave - 4;
     HwRows r;
@@ -297,8 +413,9 @@ __global__ __launch_bounds__(kHwThreads, 1) void hwgrad_partial_kernel(const Hwg
         T1[v] = (uint32_t)(64 * eq + 16 * ((2 * wc + 1) ^ b2) + 8 * h);
       }
     }
-    // zero the padding pixels (x columns -1 and W) of every stage; no DMA writes them
-    for (int i = threadIdx.x; i < kHwStages * RO * 2 * 4; i += kHwConsumers) {
+    // zero the padding pixels (x columns -1 and W) of every stage; no DMA writes them (but a
+    // strip's)
+    for (int i = threadIdx.x; !kStrip && i < kHwStages * RO * 2 * 4; i += kHwConsumers) {
       const int g = i & 3, side = (i >> 2) & 1, rs = i >> 3;
       const int row = rs % RO, stg = rs / RO;
       const int e = row * (W + 2) + (side ? W + 1 : 0);
@@ -358,18 +475,37 @@ __global__ __launch_bounds__(kHwThreads, 1) void hwgrad_partial_kernel(const Hwg
   }
 }
 
+// Columns of a K-step's tile: the widest of 32, 16 and 8 that divides the image.
+static int hwgrad_cols(int W) { return W % 32 == 0 ? 32 : (W % 16 == 0 ? 16 : 8); }
+static bool hwgrad_whole_rows(int H, int W) {
+  return (W == 16 || W == 32) && H % (kHwPix / W) == 0;
+}
+static int64_t hwgrad_chunks(int N, int H, int W) {
+  const int tw = hwgrad_cols(W);
+  return ceil_div((int64_t)N * H, kHwPix / tw) * (W / tw);
+}
+
+int hwgrad_splits(int N, int H, int W, int Cin, int Cout, int split_k);
+
+// Strips pay where each workgroup has a long run of K-steps: with at least 16 of them (in the
+// library's own split) the three-tap tile's smaller fetch wins over the one-tap kernel
+// (wgrad.hip), with fewer its deeper ring and its extra splits cost more. us with the split
+// sum, one-tap / strips: 32 x 64x64 x 128 (24 steps) 34.1 / 28.7, 16 x 48x48 x 256 (28) 39.1 /
+// 33.0; 32 x 24x24 x 256 (14) 27.8 / 28.3, 8 x 64x64 x 128 (6) 23.0 / 24.5, 128 x 8x8 x 256 (6)
+// 23.0 / 25.8.
+constexpr int kHwStripSteps = 16;
+
 bool hwgrad_supported(int N, int H, int W, int Cin, int Cout) {
-  if (N <= 0 || H <= 0) return false;
-  if (W != 16 && W != 32) return false;
-  if (H % (kHwPix / W) != 0) return false;
+  if (N <= 0 || H <= 0 || W <= 0 || W % 8 != 0) return false;
   if (Cin % kHwCi != 0 || Cout % kHwCo != 0) return false;
   if ((int64_t)N * H * W * Cin > 0x7fffffff || (int64_t)N * H * W * Cout > 0x7fffffff)
     return false;
-  return true;
+  return hwgrad_whole_rows(H, W) ||
+         hwgrad_chunks(N, H, W) >= (int64_t)kHwStripSteps * hwgrad_splits(N, H, W, Cin, Cout, 0);
 }
 
 int hwgrad_splits(int N, int H, int W, int Cin, int Cout, int split_k) {
-  const int nchunks = (int)((int64_t)N * H * W / kHwPix);
+  const int nchunks = (int)hwgrad_chunks(N, H, W);
   const int tiles = 3 * (Cin / kHwCi) * (Cout / kHwCo);
   int s = split_k;
   if (s <= 0) {
@@ -392,18 +528,27 @@ int hwgrad_partial_run(const void* xq, const void* dyq, float* partial, int N, i
   a.x = (const uint8_t*)xq;
   a.dy = (const uint8_t*)dyq;
   a.partial = partial;
-  a.N = N; a.H = H; a.Cin = Cin; a.Cout = Cout;
-  a.nchunks = (int)((int64_t)N * H * W / kHwPix);
+  a.N = N; a.H = H; a.W = W; a.Cin = Cin; a.Cout = Cout;
+  a.nchunks = (int)hwgrad_chunks(N, H, W);
   a.splits = splits;
   a.ci_tiles = Cin / kHwCi;
   a.tiles = 3 * a.ci_tiles * (Cout / kHwCo);
   a.total = a.tiles * splits;
   a.per_xcd = (int)ceil_div(a.total, 8);
   const unsigned grid = (unsigned)(a.per_xcd * 8);
-  if (W == 32)
-    hwgrad_partial_kernel<32><<<grid, kHwThreads, 0, s>>>(a);
-  else
-    hwgrad_partial_kernel<16><<<grid, kHwThreads, 0, s>>>(a);
+  const int tw = hwgrad_cols(W);
+  if (hwgrad_whole_rows(H, W)) {
+    if (tw == 32)
+      hwgrad_partial_kernel<32, false><<<grid, kHwThreads, 0, s>>>(a);
+    else
+      hwgrad_partial_kernel<16, false><<<grid, kHwThreads, 0, s>>>(a);
+  } else if (tw == 32) {
+    hwgrad_partial_kernel<32, true><<<grid, kHwThreads, 0, s>>>(a);
+  } else if (tw == 16) {
+    hwgrad_partial_kernel<16, true><<<grid, kHwThreads, 0, s>>>(a);
+  } else {
+    hwgrad_partial_kernel<8, true><<<grid, kHwThreads, 0, s>>>(a);
+  }
   return launch_status();
 }
 

@@ -380,3 +380,34 @@ def test_fragment_weight_convs_on_every_tile(K, shape):
     assert_bf16_close(nhwc_bits(y[k].cpu()), O.conv2d_fwd(xb, wb, f32(xs), f32(ws)), f"fwd {shape}")
     assert_bf16_close(nhwc_bits(dx[k].cpu()), O.conv2d_dgrad(db, wb, f32(dys), f32(ws), (h, w)),
                       f"dgrad {shape}")
+
+
+# the three-tap weight gradient's strips: tiles of 32, 16 and 8 columns, one or more strips
+# a row, heights that a tile's rows do not divide (tiles that straddle images, a ragged last one)
+STRIP_SHAPES = [(6, 256, 256, 64, 64), (10, 256, 256, 33, 64), (18, 256, 256, 30, 48),
+                (57, 256, 256, 9, 40), (19, 256, 256, 24, 56)]
+
+
+@pytest.mark.parametrize("shape", STRIP_SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_weight_gradient_strips(K, shape):
+    """dw on strips (shapes with at least 16 K-steps a workgroup) against the sum over the images
+    of the exact oracle, and in fp32 the same values."""
+    n, cin, cout, h, w = shape
+    xq, xs, _, _, dyq, dys = quantized_inputs(K, n, cin, cout, h, w, seed=sum(shape))
+    split = 2
+    dw = K.conv2d_fp8_wgrad_general(xq, dyq, xs, dys)
+    dw32 = K.conv2d_fp8_wgrad_general(xq, dyq, xs, dys, split_k=split, out_f32=True)
+    xf, df = xq.float().double(), dyq.float().double()
+    xp = torch.nn.functional.pad(xf, (1, 1, 1, 1))
+    ref = torch.empty((cout, cin, 3, 3), dtype=torch.float64, device="cuda")
+    d2 = df.permute(1, 0, 2, 3).reshape(cout, -1).contiguous()
+    for r in range(3):
+        for s in range(3):
+            x2 = xp[:, :, r:r + h, s:s + w].permute(0, 2, 3, 1).reshape(-1, cin).contiguous()
+            ref[:, :, r, s] = d2 @ x2
+    ref *= float(xs) * float(dys)
+    for got in (dw, dw32):
+        # one bf16 rounding (2^-8 of a value at most, 2^-7 over a binade's edge) beside the
+        # fp32 sums' error, which is below 2^-12 of the root mean square here
+        tol = 2**-7 * ref.abs() + 2**-12 * ref.square().mean().sqrt()
+        assert bool(((got.double() - ref).abs() <= tol).all())
