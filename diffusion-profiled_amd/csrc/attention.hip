@@ -62,14 +62,39 @@ __device__ __forceinline__ uint2 ld_tr16(const uint16_t* p) {
   return __builtin_bit_cast(uint2, v);
 }
 
-// A fragment (rows = dims d0 + frow, k-slice fq) of the transpose of a row-major [rows][72]
-// LDS array X, k running over X's rows: elements 0-3 = X[r1 + t][d0 + frow] and 4-7 =
-// X[r2 + t][d0 + frow], t = 0..3 (r1, r2: this lane group's first rows).
-__device__ __forceinline__ uint4 frag_tr(const uint16_t* x, int r1, int r2, int d0, int frow) {
-  const int off = (frow >> 2) * 72 + d0 + 4 * (frow & 3);
-  const uint2 lo = ld_tr16(x + r1 * 72 + off);
-  const uint2 hi = ld_tr16(x + r2 * 72 + off);
+// Rows of a head in LDS: 128 B (64 dims) each, the 16-B granule g of row r at g ^ (r & 7). Rows
+// come by DMA (a transfer is 8 whole rows, its lanes' sources permuted to match), and neither
+// the row reads (16 rows at one granule per 16 lanes) nor the transpose reads conflict.
+// At B = 128, 4 heads, L = 256 (512 workgroups, 268 MB forward and backward), against 144-B
+// rows staged through registers with the whole head awaited before the first product: forward
+// and backward 83.8 -> 80.0 us; both wait for their rows first and then for LDS and latency.
+__device__ __forceinline__ int att_off(int row, int g) { return row * 64 + ((g ^ (row & 7)) << 3); }
+
+// A fragment (rows = dims 16 hb + frow, k-slice fq) of the transpose of such an array x, k
+// running over x's rows: elements 0-3 = x[r1 + t][16 hb + frow] and 4-7 = x[r2 + t][16 hb +
+// frow], t = 0..3 (r1, r2: this lane group's first rows, multiples of 4).
+__device__ __forceinline__ uint4 frag_tr(const uint16_t* x, int r1, int r2, int hb, int frow) {
+  const int rr = frow >> 2, g = 2 * hb + ((frow & 3) >> 1), half = 4 * (frow & 1);
+  const uint2 lo = ld_tr16(x + att_off(r1 + rr, g) + half);
+  const uint2 hi = ld_tr16(x + att_off(r2 + rr, g) + half);
   return uint4{lo.x, lo.y, hi.x, hi.y};
+}
+
+__device__ __attribute__((aligned(64))) uint32_t att_zero16[4];
+__device__ uint32_t att_inf = 0x7f800000u;
+
+// 8 rows of src (row pitch in elements) per wave into the rows array at x: chunk c = row c / 8,
+// granule c % 8; rows from L on are zero.
+__device__ __forceinline__ void att_dma(const uint16_t* src, int64_t pitch, int c, int L,
+                                        uint32_t x) {
+  const int j = c >> 3, g = (c & 7) ^ (j & 7);
+  const void* a = j < L ? static_cast<const void*>(src + j * pitch + 8 * g) : att_zero16;
+  dma16_lds(a, x + (uint32_t)__builtin_amdgcn_readfirstlane(c & ~63) * 16);
+}
+
+// 4 B per lane to lds + 4 * lane (lds wave-uniform), from any 4-byte aligned source.
+__device__ __forceinline__ void dma4_lds(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(lds) : "m0");
 }
 
 struct AttnArgs {
@@ -108,24 +133,25 @@ __device__ __forceinline__ void att_store_partial(us2 am, uint32_t* part) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Forward: one workgroup (4 waves) per (image, head); K and V rows of the head in LDS
-// (row-major, 144-B rows); wave w takes query blocks w, w + 4, ... of 16 queries. Per block,
-// S^T = K Q^T (A = K rows, B = the block's queries from global, loaded one block ahead: lane
+// Forward: one workgroup (4 waves) per (image, head); K and V rows of the head in LDS; wave w
+// takes query blocks w, w + 4, ... of 16 queries. Per block,
+// S^T = K Q^T (A = K rows, B = the block's queries, loaded one block ahead: lane
 // (q = frow, k-slice fq) holds dims 8 fq .. + 7 of each 32-wide half), so lane (frow, fq)
 // holds scores of query frow at keys 16 kb + 4 fq + t: the row max and sum need only the
 // lane's own values and two shuffles. O^T = V^T P^T: B = P^T straight from those registers
 // (k-step kk pairs score blocks 2 kk and 2 kk + 1, i.e. keys 32 kk + 4 fq + t and
 // 32 kk + 16 + 4 fq + t in the lane's slice), A = V^T by transpose reads of the V rows at the
-// same keys.
+// same keys. The first block's scores and softmax run while V is still on its way.
 // ---------------------------------------------------------------------------------------
 template <int LP>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
-  constexpr int KP = 72;          // K / V row pitch in LDS (144 B: 16 rows on distinct banks)
   constexpr int NKB = LP / 16;    // key blocks
-  __shared__ __attribute__((aligned(16))) uint16_t ks[LP * KP];
-  __shared__ __attribute__((aligned(16))) uint16_t vs[LP * KP];
+  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t vs[LP * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t q1[64 * 64];  // the first block of each wave
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int frow = lane & 15, fq = lane >> 4;
   const int bh = blockIdx.x;
   const int b = bh / p.heads, h = bh - b * p.heads;
@@ -135,34 +161,27 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
   const uint16_t* kg = qg + C;
   const uint16_t* vg = qg + 2 * C;
 
-  // K and V rows into LDS (padded keys zero): every load in flight before the first store
-  constexpr int NF = LP * 8 / 256;  // 16-B chunks per thread
+  // the waves' first queries, K, then V (padded rows zero)
+  constexpr int NF = LP * 8 / 256;  // transfers per wave of K, of V
+#pragma unroll
+  for (int r = 0; r < 2; ++r) att_dma(qg, S3, tid + 256 * r, L, LDS_ADDR(q1));
+#pragma unroll
+  for (int r = 0; r < NF; ++r) att_dma(kg, S3, tid + 256 * r, L, LDS_ADDR(ks));
+#pragma unroll
+  for (int r = 0; r < NF; ++r) att_dma(vg, S3, tid + 256 * r, L, LDS_ADDR(vs));
+  wait_vmcnt<NF>();  // queries and K
+  lds_barrier();
+  uint4 qf0, qf1;
   {
-    uint4 kv[NF], vv[NF];
-#pragma unroll
-    for (int r = 0; r < NF; ++r) {
-      const int c = tid + 256 * r, j = c >> 3, d0 = (c & 7) * 8;
-      kv[r] = vv[r] = uint4{0u, 0u, 0u, 0u};
-      if (j < L) {
-        kv[r] = ld16(kg + j * S3 + d0);
-        vv[r] = ld16(vg + j * S3 + d0);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < NF; ++r) {
-      const int c = tid + 256 * r, j = c >> 3, d0 = (c & 7) * 8;
-      *reinterpret_cast<uint4*>(ks + j * KP + d0) = kv[r];
-      *reinterpret_cast<uint4*>(vs + j * KP + d0) = vv[r];
-    }
+    const int row = wave * 16 + frow;
+    qf0 = ld16(q1 + att_off(row, fq));
+    qf1 = ld16(q1 + att_off(row, 4 + fq));
   }
-  // B fragments of the wave's first query block, then always one block ahead
-  uint4 qf0 = {0u, 0u, 0u, 0u}, qf1 = {0u, 0u, 0u, 0u};
-  if (wave * 16 < L) {
-    const uint16_t* qr = qg + (wave * 16 + frow) * S3 + 8 * fq;
-    qf0 = ld16(qr);
-    qf1 = ld16(qr + 32);
-  }
-  __syncthreads();
+  // V complete; every wave passes this once
+  auto wait_v = [&]() __attribute__((always_inline)) {
+    wait_vmcnt<0>();
+    lds_barrier();
+  };
 
   us2 am = {0, 0};
   for (int q0 = wave * 16; q0 < L; q0 += 64) {
@@ -175,9 +194,9 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
     v4f s[NKB];
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
-      const uint16_t* kr = ks + (16 * kb + frow) * KP + 8 * fq;
-      s[kb] = mfma16x16x32_bf16(ld16(kr), qf0, v4f{0.f, 0.f, 0.f, 0.f});
-      s[kb] = mfma16x16x32_bf16(ld16(kr + 32), qf1, s[kb]);
+      const int row = 16 * kb + frow;
+      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off(row, fq)), qf0, v4f{0.f, 0.f, 0.f, 0.f});
+      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off(row, 4 + fq)), qf1, s[kb]);
     }
     if (L < LP) {
 #pragma unroll
@@ -213,6 +232,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
     __builtin_amdgcn_sched_barrier(0);
+    if (q0 < 64) wait_v();  // the wave's first block
 
     v4f o[4];
 #pragma unroll
@@ -222,7 +242,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
       const uint4 pf = {pk[2 * kk][0], pk[2 * kk][1], pk[2 * kk + 1][0], pk[2 * kk + 1][1]};
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb)
-        o[hb] = mfma16x16x32_bf16(frag_tr(vs, 32 * kk + 4 * fq, 32 * kk + 16 + 4 * fq, 16 * hb, frow),
+        o[hb] = mfma16x16x32_bf16(frag_tr(vs, 32 * kk + 4 * fq, 32 * kk + 16 + 4 * fq, hb, frow),
                                   pf, o[hb]);
       if (kk % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
@@ -236,14 +256,17 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
     qf0 = nq0;
     qf1 = nq1;
   }
+  if (wave * 16 >= L) wait_v();  // a wave without queries
   if (p.amax_part) att_store_partial<4>(am, p.amax_part);
 }
 
 // ---------------------------------------------------------------------------------------
-// Backward: one workgroup (8 waves) per (image, head). The head's Q, K and dO rows (row-major,
-// 144-B rows), the log-sum-exp and D = rowsum(dO * O) of every query go into LDS once, with
-// all their loads in flight together. Wave w owns KB key blocks (keys kw0 = 16 KB w ..) and
-// keeps their K and V rows as B fragments and the dK^T, dV^T accumulators in registers;
+// Backward: one workgroup (8 waves) per (image, head). The head's Q, K and dO rows, the
+// log-sum-exp and D = rowsum(dO * O) of every query go into LDS, all by DMA issued at the
+// start: K and V, then Q, dO and O in parts of 64 rows. The first query blocks run on the first
+// part while the others are on their way; part r is awaited, and its D formed, in block 2 r - 1.
+// (V passes through the dS buffers on its way to registers.) Wave w owns KB key blocks (keys
+// kw0 = 16 KB w ..) and keeps their K and V rows as B fragments and the dK^T, dV^T accumulators in registers;
 // query blocks of 32 rows stream through:
 //   S = Q K^T and dP = dO V^T (A = Q / dO rows from LDS) in the layout lane (frow, fq) <->
 //   (query 16 sub + 4 fq + t, key frow);  P = 2^(S log2(e)/8 - lse), dS = P (dP - D);
@@ -258,15 +281,21 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
 template <int LP>
 __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   constexpr int KB = LP >= 256 ? 2 : 1;  // key blocks per wave
-  constexpr int RP = 72;                 // Q / K / dO row pitch (144 B)
-  constexpr int TP = LP + 8;             // dS row pitch
-  __shared__ __attribute__((aligned(16))) uint16_t qs[LP * RP];
-  __shared__ __attribute__((aligned(16))) uint16_t ks[LP * RP];
-  __shared__ __attribute__((aligned(16))) uint16_t gs[LP * RP];
-  __shared__ __attribute__((aligned(16))) uint16_t dsb[2][32 * TP];
-  __shared__ float lse_s[LP], dd_s[LP];
+  constexpr int TP = LP + 16;            // dS row pitch (LP = 256, 128: rows 2 bank slots apart)
+  constexpr int NCH = LP * 8;            // 16-B chunks of a rows array
+  constexpr int NF = (NCH + 511) / 512;  // its transfers per wave, and the parts
+  constexpr int OB = NF < 3 ? NF : 3;    // O parts in flight (a fourth reuses the first's room)
+  __shared__ __attribute__((aligned(1024))) uint16_t qs[LP * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t gs[LP * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t os[OB][64 * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t dsb[2][32 * TP];
+  __shared__ __attribute__((aligned(256))) float lse_s[LP < 64 ? 64 : LP];
+  __shared__ float dd_s[LP];
+  static_assert(2 * 32 * TP >= LP * 64, "V fits the dS buffers");
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int frow = lane & 15, fq = lane >> 4;
   const int bh = blockIdx.x;
   const int b = bh / p.heads, h = bh - b * p.heads;
@@ -282,71 +311,80 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   uint16_t* dkg = dqg + C;
   uint16_t* dvg = dqg + 2 * C;
 
-  // Q, K, dO rows, the log-sum-exp and D per query (padded rows: zeros, lse = +inf, so their
-  // P is 0); chunk c = row c / 8, dims 8 (c % 8) ..
-  constexpr int NCH = LP * 8;
-  constexpr int NF = (NCH + 511) / 512;
-  // this wave's keys: B fragments of K and V (lane (key frow, k-slice fq): dims 8 fq .. + 7
-  // of each 32-wide half), zero for padded keys; issued with the staging loads below
+  // Padded rows: zeros, lse = +inf, so their P is 0.
   const int kw0 = wave * 16 * KB;
   const bool kact = kw0 < LP;  // wave-uniform
-  uint4 kf[KB][2], vf[KB][2];
-#pragma unroll
-  for (int kb = 0; kb < KB; ++kb) {
-    const int key = kw0 + 16 * kb + frow;
-#pragma unroll
-    for (int hs = 0; hs < 2; ++hs) {
-      kf[kb][hs] = key < L ? ld16(kg + key * S3 + 32 * hs + 8 * fq) : uint4{0u, 0u, 0u, 0u};
-      vf[kb][hs] = key < L ? ld16(vg + key * S3 + 32 * hs + 8 * fq) : uint4{0u, 0u, 0u, 0u};
-    }
+  const bool has = wave * 64 < NCH;  // this wave moves chunks
+  auto dma_o = [&](int r) __attribute__((always_inline)) {
+    // part r's 64 rows at os[r % OB]: as rows 0 .. 63 of its own array
+    att_dma(og + (int64_t)64 * r * C, C, tid, L - 64 * r, LDS_ADDR(os[r % OB]));
+  };
+  if (wave * 64 < LP) {
+    const void* a = tid < L ? static_cast<const void*>(p.lse + (int64_t)bh * L + tid) : &att_inf;
+    dma4_lds(a, LDS_ADDR(lse_s) + 256 * wave);
   }
-  const float lse_t = tid < L ? p.lse[(int64_t)bh * L + tid] : __builtin_inff();
-  {
-    uint4 kv[NF], qv[NF], ov[NF], gv[NF];
+  if (has) {
+#pragma unroll
+    for (int r = 0; r < NF; ++r) att_dma(kg, S3, tid + 512 * r, L, LDS_ADDR(ks));
+#pragma unroll
+    for (int r = 0; r < NF; ++r) att_dma(vg, S3, tid + 512 * r, L, LDS_ADDR(dsb));
 #pragma unroll
     for (int r = 0; r < NF; ++r) {
-      const int c = tid + 512 * r, j = c >> 3, d0 = (c & 7) * 8;
-      kv[r] = qv[r] = ov[r] = gv[r] = uint4{0u, 0u, 0u, 0u};
-      if (c < NCH && j < L) {
-        kv[r] = ld16(kg + j * S3 + d0);
-        qv[r] = ld16(qg + j * S3 + d0);
-        ov[r] = ld16(og + j * C + d0);
-        gv[r] = ld16(dg + j * C + d0);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < NF; ++r) {
-      const int c = tid + 512 * r, j = c >> 3, d0 = (c & 7) * 8;
-      if (NCH % 512 != 0 && c >= NCH) continue;  // wave-uniform (NCH % 64 == 0)
-      *reinterpret_cast<uint4*>(ks + j * RP + d0) = kv[r];
-      *reinterpret_cast<uint4*>(qs + j * RP + d0) = qv[r];
-      *reinterpret_cast<uint4*>(gs + j * RP + d0) = gv[r];
-      float fo[8], fg[8];
-      unpack8_bf16(ov[r], fo);
-      unpack8_bf16(gv[r], fg);
-      float dot8 = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) dot8 += fo[e] * fg[e];
-      dot8 += __shfl_xor(dot8, 1, 64);
-      dot8 += __shfl_xor(dot8, 2, 64);
-      dot8 += __shfl_xor(dot8, 4, 64);
-      if ((c & 7) == 0) dd_s[j] = dot8;
+      att_dma(qg, S3, tid + 512 * r, L, LDS_ADDR(qs));
+      att_dma(dg, C, tid + 512 * r, L, LDS_ADDR(gs));
+      if (r < OB) dma_o(r);
     }
   }
-  if (tid < LP) lse_s[tid] = lse_t;
+  // D of part r's rows from this thread's chunk of dO and O (its own transfers' data)
+  auto form_d = [&](int r) __attribute__((always_inline)) {
+    if (!has) return;
+    const int c = tid + 512 * r;
+    float fo[8], fg[8];
+    unpack8_bf16(ld16(os[r % OB] + tid * 8), fo);
+    unpack8_bf16(ld16(gs + c * 8), fg);
+    float dot8 = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dot8 += fo[e] * fg[e];
+    dot8 += __shfl_xor(dot8, 1, 64);
+    dot8 += __shfl_xor(dot8, 2, 64);
+    dot8 += __shfl_xor(dot8, 4, 64);
+    if ((c & 7) == 0) dd_s[c >> 3] = dot8;
+  };
   v4f dvt[4][KB], dkt[4][KB];
 #pragma unroll
   for (int hb = 0; hb < 4; ++hb)
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) dvt[hb][kb] = dkt[hb][kb] = v4f{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();  // Q, K, dO rows, lse and D complete
+  // outstanding transfers after K, V and part 0: of parts 1 .. NF - 1
+  constexpr int kLater = 2 * (NF - 1) + (OB - 1);
+  wait_vmcnt<kLater>();
+  asm volatile("" ::: "memory");  // (the DMAs' writes are invisible to the compiler)
+  form_d(0);
+  wait_lgkmcnt0();
+  asm volatile("" ::: "memory");
+  if (NF > OB && has) dma_o(OB);  // into os[0], whose chunks only their own wave read
+  lds_barrier();                  // K, V, part 0 and its D, lse
 
+  // this wave's keys: B fragments of K and V (lane (key frow, k-slice fq): dims 8 fq .. + 7
+  // of each 32-wide half)
+  uint4 kf[KB][2], vf[KB][2];
+  const uint16_t* vrow = &dsb[0][0];
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+    for (int hs = 0; hs < 2; ++hs) {
+      const int o = kact ? att_off(kw0 + 16 * kb + frow, 4 * hs + fq) : 0;
+      kf[kb][hs] = ld16(ks + o);
+      vf[kb][hs] = ld16(vrow + o);
+    }
   // the K^T operand of this wave's dQ block (dims 16 (wave & 3) ..) over all keys: the same
   // for every query block, so read once
   uint4 ktf[LP / 32];
 #pragma unroll
   for (int kk = 0; kk < LP / 32; ++kk)
-    ktf[kk] = frag_tr(ks, 32 * kk + 8 * fq, 32 * kk + 8 * fq + 4, 16 * (wave & 3), frow);
+    ktf[kk] = frag_tr(ks, 32 * kk + 8 * fq, 32 * kk + 8 * fq + 4, wave & 3, frow);
+  wait_lgkmcnt0();
+  lds_barrier();  // V read: the dS buffers are free
 
   // A fragments of a query block: rows q0 + 16 sub + frow of Q and dO (read one block ahead,
   // during the previous block's dQ products)
@@ -356,7 +394,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int hs = 0; hs < 2; ++hs) {
-        const int o = (q0 + 16 * sub + frow) * RP + 32 * hs + 8 * fq;
+        const int o = att_off(q0 + 16 * sub + frow, 4 * hs + fq);
         qa[sub][hs] = ld16(qs + o);
         da[sub][hs] = ld16(gs + o);
       }
@@ -424,8 +462,8 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
       const int r1 = q0 + 4 * fq, r2 = q0 + 16 + 4 * fq;
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb) {
-        const uint4 da4 = frag_tr(gs, r1, r2, 16 * hb, frow);
-        const uint4 qa4 = frag_tr(qs, r1, r2, 16 * hb, frow);
+        const uint4 da4 = frag_tr(gs, r1, r2, hb, frow);
+        const uint4 qa4 = frag_tr(qs, r1, r2, hb, frow);
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
           dvt[hb][kb] = mfma16x16x32_bf16(da4, pb[kb], dvt[hb][kb]);
@@ -433,10 +471,33 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
         }
       }
     }
+    // part (blk + 1) / 2, which the next block reads: behind it are the transfers of later
+    // parts (and stores, which are not counted here: waiting for more is only slower)
+    if constexpr (NF > 1) {
+      if (blk & 1) {
+        const int r = (blk + 1) >> 1;
+        if (r == 1) {
+          wait_vmcnt<NF == 4 ? 6 : 0>();
+          asm volatile("" ::: "memory");
+          form_d(1);
+        } else if (NF > 2 && r == 2) {
+          wait_vmcnt<3>();
+          asm volatile("" ::: "memory");
+          form_d(2 < NF ? 2 : 0);
+        } else if (NF > 2 && r == 3) {
+          wait_vmcnt<0>();
+          asm volatile("" ::: "memory");
+          form_d(3 < NF ? 3 : 0);
+        }
+      }
+    }
     if (blk > 0) dq_block(q0 - 32, dsb[(blk - 1) & 1]);
-    __syncthreads();  // this block's dS complete
+    wait_lgkmcnt0();
+    lds_barrier();  // this block's dS (and the next part and its D) complete
     if (kact && q0 + 32 < L) load_a(q0 + 32);
   }
+  // no transfer may outlive the workgroup's LDS: parts past the last query were not awaited
+  if ((L + 31) / 32 < 2 * NF - 2) wait_vmcnt<0>();
   dq_block(q_last, dsb[((L + 31) / 32 - 1) & 1]);
 
   // dK, dV of this wave's keys: lane holds dims 16 hb + 4 fq + t of key kw0 + 16 kb + frow

@@ -115,6 +115,32 @@ def test_attention_vs_fp32_and_sdpa(b, l, heads, scale):
         assert e <= 2e-2 and e <= 1.5 * s + 2e-3, name
 
 
+@pytest.mark.parametrize("l", [32, 80, 112, 128, 160, 176, 192, 208, 240])
+def test_attention_lengths_between_the_grids(l):
+    """Every 64-row part of a head partly filled, filled and empty (the rows arrive in parts
+    while the first query blocks run), at the padded lengths the grids above leave out, with a
+    log-sum-exp that is only 4-byte aligned. Tolerances: this file's normwise ones."""
+    print(f"attention L={l}", flush=True)
+    b, heads = 3, 2
+    c = 64 * heads
+    qkv = _qkv(b, l, heads, seed=l)
+    dout = torch.randn((b, l, c), generator=torch.Generator().manual_seed(l + 1))
+    dout = dout.to(torch.bfloat16).cuda()
+    out = torch.empty_like(dout)
+    dqkv = torch.empty_like(qkv)
+    lse = torch.empty(b * heads * l + 1, device="cuda", dtype=torch.float32)[1:]
+    call, st = dpa_mod("_lib").call, torch.cuda.current_stream().cuda_stream
+    call("dpa_attention_fwd_bf16", qkv.data_ptr(), out.data_ptr(), lse.data_ptr(), b, l, c, heads,
+         st)
+    call("dpa_attention_bwd_bf16", qkv.data_ptr(), out.data_ptr(), dout.data_ptr(),
+         lse.data_ptr(), dqkv.data_ptr(), b, l, c, heads, st)
+    torch.cuda.synchronize()
+    ro, rd, _ = _ref_fp32(qkv, heads, dout)
+    assert _rel(out, ro) <= 1e-2
+    for i in range(3):
+        assert _rel(dqkv[..., i * c:(i + 1) * c], rd[..., i * c:(i + 1) * c]) <= 2e-2, "qkv"[i]
+
+
 def test_attention_lse_vs_float64():
     """The forward's saved log-sum-exp: log2 sum_k 2^(s_k log2(e) / 8) per (image, head, query)."""
     b, l, heads = 4, 256, 4
