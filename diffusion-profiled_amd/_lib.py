@@ -16,13 +16,21 @@ from . import build as _build
 
 
 @torch.compiler.disable
+def _current_stream_untraced(t: "torch.Tensor") -> int:
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
 def current_stream(t: "torch.Tensor") -> int:
     """The hipStream_t of torch's current stream on t's device, where every launch goes (so
     launches order with torch's own kernels and graph capture records them). Dynamo never
-    traces it: under torch.compile a call here ends the graph and the ctypes launch that
+    traces past it: under torch.compile a call here ends the graph and the ctypes launch that
     follows runs eagerly. The FP8 ops call it inside torch.library custom-op bodies, which
     Dynamo does not enter."""
-    return torch.cuda.current_stream(t.device).cuda_stream
+    if torch.compiler.is_compiling() or not t.is_cuda:     # (which refuses a CPU tensor)
+        return _current_stream_untraced(t)
+    # the handle alone: a torch.cuda.Stream object around it costs as much as a launch
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
 
 c_float_p = POINTER(c_float)
 
@@ -263,9 +271,11 @@ def check(status: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call an entry point that returns a status code; raise on failure."""
-    check(getattr(load(), name)(*args), name)
+    status = getattr(_lib or load(), name)(*args)
+    if status != 0:
+        check(status, name)
 
 
 def query(name: str, *args) -> int:
     """Call an entry point that returns a size."""
-    return int(getattr(load(), name)(*args))
+    return getattr(_lib or load(), name)(*args)

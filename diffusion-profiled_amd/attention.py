@@ -17,6 +17,7 @@ from torch.amp.autocast_mode import custom_bwd, custom_fwd
 
 from . import _lib
 from . import fp8_kernels as _fp8
+from .eager import apply
 
 HEAD_DIM = 64
 
@@ -78,4 +79,4 @@ class SelfAttentionQKV(torch.autograd.Function):
 
 
 def self_attention_qkv(qkv: torch.Tensor, heads: int) -> torch.Tensor:
-    return SelfAttentionQKV.apply(qkv, heads)
+    return apply(SelfAttentionQKV, qkv, heads)

@@ -20,6 +20,7 @@ import torch
 from torch.amp.autocast_mode import custom_bwd, custom_fwd
 
 from . import _lib
+from .eager import apply, run, run_in
 
 # diffusion/fp8_kernels.py:11-12
 FP8_DTYPE = torch.float8_e4m3fn
@@ -318,7 +319,7 @@ def quantize_fp8_delayed(tensor: torch.Tensor, prev_scale: torch.Tensor) -> tupl
         f"{tensor.dtype} {tensor.is_cuda} {tensor.ndim}"
     )
     torch_checks_scale(prev_scale, tensor.device)
-    return _ops.quantize_delayed(tensor, prev_scale)
+    return run(_ops.quantize_delayed, tensor, prev_scale)
 
 
 def quantize_fp8(tensor: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
@@ -326,16 +327,16 @@ def quantize_fp8(tensor: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     assert tensor.dtype == torch.bfloat16 and tensor.is_cuda and tensor.ndim == 4, (
         f"{tensor.dtype} {tensor.is_cuda} {tensor.ndim}"
     )
-    return _ops.quantize(tensor)
+    return run(_ops.quantize, tensor)
 
 
 def quantize_fp8_tensor(tensor: torch.Tensor, prev_scale: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor]:
     """``quantize_fp8`` / ``quantize_fp8_delayed`` for a bf16 tensor of any rank."""
     assert tensor.dtype == torch.bfloat16 and tensor.is_cuda, f"{tensor.dtype} {tensor.is_cuda}"
     if prev_scale is None:
-        return _ops.quantize(tensor)
+        return run(_ops.quantize, tensor)
     torch_checks_scale(prev_scale, tensor.device)
-    return _ops.quantize_delayed(tensor, prev_scale)
+    return run(_ops.quantize_delayed, tensor, prev_scale)
 
 
 # --------------------------------------------------------------------------------------
@@ -630,7 +631,7 @@ def conv2d_fwd_fp8_prequantized(
     fwd_shapes(x, weight, FP8_DTYPE)
     torch_checks_scale(x_scale, x.device)
     torch_checks_scale(weight_scale, x.device)
-    return _ops.conv_fwd(x, weight, x_scale, weight_scale, 1, 1)
+    return run(_ops.conv_fwd, x, weight, x_scale, weight_scale, 1, 1)
 
 
 def conv2d_fwd_fp8(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -657,7 +658,7 @@ def conv2d_bwd_input_fp8_prequantized(
     batch, cin, cout, height, width = xgrad_shapes(dy, weight, FP8_DTYPE)
     torch_checks_scale(dy_scale, dy.device)
     torch_checks_scale(weight_scale, dy.device)
-    return _ops.conv_dgrad(dy, weight, dy_scale, weight_scale, height, width, 1, 1)
+    return run(_ops.conv_dgrad, dy, weight, dy_scale, weight_scale, height, width, 1, 1)
 
 
 def conv2d_bwd_input_fp8(dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -685,7 +686,7 @@ def conv2d_bwd_weight_fp8_prequantized(
     if not (x.is_contiguous(memory_format=torch.channels_last)
             and dy.is_contiguous(memory_format=torch.channels_last)):
         raise NotImplementedError
-    return _ops.conv_wgrad(x, dy, x_scale, dy_scale, 3, 1, 1, split_k or 0, out_f32)
+    return run(_ops.conv_wgrad, x, dy, x_scale, dy_scale, 3, 1, 1, split_k or 0, out_f32)
 
 
 def conv2d_bwd_weight_fp8(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
@@ -708,11 +709,11 @@ def _conv_current_fwd(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: i
     cout, wcin, kh, kw = weight.shape
     assert wcin == cin and kh == kw
     frag = frag_shape(batch, cin, cout, height, width, kh, stride, padding)
-    x_fp8, x_scale, w_fp8, w_t, w_scale = _ops.quantize_with_weight(x, weight, frag)
+    x_fp8, x_scale, w_fp8, w_t, w_scale = run_in(ctx, _ops.quantize_with_weight, x, weight, frag)
     ctx.save_for_backward(x_fp8, w_t, x_scale, w_scale)
     ctx.geom = (cin, height, width, kh, stride, padding)
     ctx.dw_f32 = weight.dtype == torch.float32
-    return _ops.conv_fwd_prepared(x_fp8, w_fp8, x_scale, w_scale, cout, stride, padding)
+    return run_in(ctx, _ops.conv_fwd_prepared, x_fp8, w_fp8, x_scale, w_scale, cout, stride, padding)
 
 
 def _conv_current_bwd(ctx: Any, dy: torch.Tensor, need_dx: bool = True):
@@ -723,9 +724,9 @@ def _conv_current_bwd(ctx: Any, dy: torch.Tensor, need_dx: bool = True):
     dy_fp8, dy_scale = quantize_fp8(dy)
     dx = None
     if need_dx:
-        dx = _ops.conv_dgrad_prepared(dy_fp8, w_t, dy_scale, w_scale, cin, height, width, k,
+        dx = run(_ops.conv_dgrad_prepared, dy_fp8, w_t, dy_scale, w_scale, cin, height, width, k,
                                       stride, padding)
-    dw = _ops.conv_wgrad(x_fp8, dy_fp8, x_scale, dy_scale, k, stride, padding, 0, ctx.dw_f32)
+    dw = run(_ops.conv_wgrad, x_fp8, dy_fp8, x_scale, dy_scale, k, stride, padding, 0, ctx.dw_f32)
     return dx, dw
 
 
@@ -849,7 +850,7 @@ def triton_conv2d_fp8(
     do_delayed: bool = False,
 ) -> torch.Tensor | tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Reference-named entry point (diffusion/fp8_kernels.py:916-923); runs the HIP kernels."""
-    return Conv2dFP8Specialized.apply(x, weight, hist_scales, dy_ptrs, do_delayed)
+    return apply(Conv2dFP8Specialized, x, weight, hist_scales, dy_ptrs, do_delayed)
 
 
 hip_conv2d_fp8 = triton_conv2d_fp8
@@ -876,7 +877,7 @@ class Conv2dFP8General(torch.autograd.Function):
 
 
 def conv2d_fp8(x: torch.Tensor, weight: torch.Tensor, stride: int = 1, padding: int = 1) -> torch.Tensor:
-    return Conv2dFP8General.apply(x, weight, stride, padding)
+    return apply(Conv2dFP8General, x, weight, stride, padding)
 
 
 def linear_fp8_prequantized(
@@ -1017,9 +1018,9 @@ class LinearFP8Function(torch.autograd.Function):
         assert x.shape[-1] == k
         x2 = x.to(torch.bfloat16).reshape(-1, k).contiguous()
         assert x2.is_cuda and weight.is_cuda, f"{x2.is_cuda} {weight.is_cuda}"
-        xq, xs, wq, wt, wsc = _ops.quantize_with_weight(x2, weight, False)
+        xq, xs, wq, wt, wsc = run_in(ctx, _ops.quantize_with_weight, x2, weight, False)
         b32 = None if bias is None else bias.detach().float().contiguous()
-        y = _ops.gemm(xq, wq, xs, wsc, b32)
+        y = run_in(ctx, _ops.gemm, xq, wq, xs, wsc, b32)
         ctx.save_for_backward(xq, wt, xs, wsc)
         ctx.dw_f32 = weight.dtype == torch.float32
         ctx.lead = lead
@@ -1035,9 +1036,9 @@ class LinearFP8Function(torch.autograd.Function):
         dyq, dys = quantize_fp8_tensor(dy2)
         dx = dw = db = None
         if ctx.needs_input_grad[0]:
-            dx = _ops.gemm_dgrad_wt(dyq, wt, dys, wsc).reshape(*ctx.lead, k)
+            dx = run(_ops.gemm_dgrad_wt, dyq, wt, dys, wsc).reshape(*ctx.lead, k)
         if ctx.needs_input_grad[1]:
-            dw = _ops.gemm_wgrad(xq, dyq, xs, dys, ctx.dw_f32)
+            dw = run(_ops.gemm_wgrad, xq, dyq, xs, dys, ctx.dw_f32)
         if ctx.has_bias and ctx.needs_input_grad[2]:
             db = dy2.float().sum(0)
         return dx, dw, db
@@ -1208,7 +1209,7 @@ class LinearFP8Prepared(torch.autograd.Function):
 
 
 def linear_fp8_autograd(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
-    return LinearFP8Function.apply(x, weight, bias)
+    return apply(LinearFP8Function, x, weight, bias)
 
 
 # registers the torch.ops.dpa_fp8 custom ops the reference-named functions above call

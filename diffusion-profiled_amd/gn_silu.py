@@ -17,6 +17,7 @@ import torch
 
 from . import _lib
 from . import fp8_kernels as _fp8
+from .eager import apply
 from .fp8_kernels import FP8_DTYPE, Fp8Handoff, placeholder
 
 
@@ -284,7 +285,7 @@ class GroupNormSiLUTee(torch.autograd.Function):
 def group_norm_silu_tee(x, gamma, beta, groups: int, eps: float = 1e-5, skip_bf16: bool = False,
                         hand: Fp8Handoff | None = None):
     """With ``hand`` the first output is a placeholder and the e4m3 conv input is ``hand.q``."""
-    return GroupNormSiLUTee.apply(x, gamma, beta, groups, eps, skip_bf16, hand)
+    return apply(GroupNormSiLUTee, x, gamma, beta, groups, eps, skip_bf16, hand)
 
 
 def upcat_ok(a: torch.Tensor, h: torch.Tensor, up: bool) -> bool:
@@ -382,7 +383,7 @@ def upcat_group_norm_silu_tee(a, h, gamma, beta, groups: int, eps: float = 1e-5,
                               hand: Fp8Handoff | None = None):
     """group_norm_silu_tee(upsample_concat(a, h, True), ..., skip_bf16=True) without the fp32
     concatenation (upcat_ok(a, h, True) must hold)."""
-    return UpcatGroupNormSiLUTee.apply(a, h, gamma, beta, groups, eps, hand)
+    return apply(UpcatGroupNormSiLUTee, a, h, gamma, beta, groups, eps, hand)
 
 
 class GroupNormSiLUFilm(torch.autograd.Function):
@@ -469,9 +470,9 @@ def group_norm_silu_film(x, gamma, beta, groups: int, eps: float, film_wb, p_dro
                          hand: Fp8Handoff | None = None, dx_hand: Fp8Handoff | None = None):
     """With ``hand`` the output is a placeholder and the e4m3 conv input is ``hand.q``; with
     ``dx_hand`` the backward writes the e4m3 dx there (the dy of the conv producing x)."""
-    return GroupNormSiLUFilm.apply(x, gamma, beta, groups, eps, film_wb, float(p_drop), hand,
+    return apply(GroupNormSiLUFilm, x, gamma, beta, groups, eps, film_wb, float(p_drop), hand,
                                    dx_hand)
 
 
 def group_norm_silu(x, gamma, beta, groups: int, eps: float = 1e-5, film_scale=None, film_shift=None):
-    return GroupNormSiLU.apply(x, gamma, beta, groups, eps, film_scale, film_shift)
+    return apply(GroupNormSiLU, x, gamma, beta, groups, eps, film_scale, film_shift)

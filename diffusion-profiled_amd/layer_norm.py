@@ -15,6 +15,7 @@ import torch
 
 from . import _lib
 from . import fp8_kernels as _fp8
+from .eager import apply
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -116,10 +117,10 @@ class LayerNormTee(torch.autograd.Function):
 
 
 def layer_norm_bf16(x: torch.Tensor, norm: torch.nn.LayerNorm) -> torch.Tensor:
-    return LayerNormBF16.apply(x, norm.weight, norm.bias, norm.eps)
+    return apply(LayerNormBF16, x, norm.weight, norm.bias, norm.eps)
 
 
 def layer_norm_tee(x: torch.Tensor, norm: torch.nn.LayerNorm):
     """(bf16(norm(x)), x) with the skip gradient added inside the LayerNorm backward; x a
     contiguous bf16 or fp32 token view."""
-    return LayerNormTee.apply(x, norm.weight, norm.bias, norm.eps)
+    return apply(LayerNormTee, x, norm.weight, norm.bias, norm.eps)

@@ -6,7 +6,8 @@ breaks the graph there; a custom op is one node of the graph, with a fake implem
 that gives AOTAutograd and Inductor the outputs' shapes, dtypes and strides without touching
 the device. Each op's body is the C-ABI launch sequence of ``fp8_kernels`` (fresh outputs
 from torch's caching allocator, launches on torch's current stream), so eager calls, graph
-capture and compiled graphs run the same kernels. The ops are CUDA-only: a CPU tensor raises
+capture and compiled graphs run the same kernels; an eager call that has nothing to record or
+trace goes to the body directly (``eager.run``). The ops are CUDA-only: a CPU tensor raises
 instead of falling back.
 
 Namespace ``dpa_fp8``:
@@ -38,6 +39,7 @@ from typing import Optional
 import torch
 
 from . import fp8_kernels as K
+from .eager import custom_op
 
 _CL = torch.channels_last
 _BF16 = torch.bfloat16
@@ -48,7 +50,7 @@ def _empty_cl(shape, device, dtype=_BF16) -> torch.Tensor:
 
 
 # ---- quantization --------------------------------------------------------------------
-@torch.library.custom_op("dpa_fp8::quantize", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::quantize")
 def quantize(tensor: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     q, s = K._quantize_impl(tensor, None)
     return q, s
@@ -61,7 +63,7 @@ def _quantize_fake(tensor):
             t.new_empty((), dtype=torch.float32))
 
 
-@torch.library.custom_op("dpa_fp8::quantize_delayed", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::quantize_delayed")
 def quantize_delayed(tensor: torch.Tensor, prev_scale: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     q, s = K._quantize_impl(tensor, prev_scale)
     return q, s
@@ -72,7 +74,7 @@ def _quantize_delayed_fake(tensor, prev_scale):
     return _quantize_fake(tensor)
 
 
-@torch.library.custom_op("dpa_fp8::quantize_with_weight", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::quantize_with_weight")
 def quantize_with_weight(x: torch.Tensor, weight: torch.Tensor, frag: bool
                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """(e4m3 x, x scale, e4m3 w, its data-gradient copy, w scale), the weight's copies in the
@@ -97,7 +99,7 @@ def _quantize_with_weight_fake(x, weight, frag):
 
 
 # ---- convolution ---------------------------------------------------------------------
-@torch.library.custom_op("dpa_fp8::conv_fwd", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv_fwd")
 def conv_fwd(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor,
              weight_scale: torch.Tensor, stride: int, padding: int) -> torch.Tensor:
     return K.conv2d_fp8_fwd_general(x, weight, x_scale, weight_scale, stride, padding)
@@ -111,7 +113,7 @@ def _conv_fwd_fake(x, weight, x_scale, weight_scale, stride, padding):
     return _empty_cl((batch, cout, oh, ow), x.device)
 
 
-@torch.library.custom_op("dpa_fp8::conv_dgrad", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv_dgrad")
 def conv_dgrad(dy: torch.Tensor, weight: torch.Tensor, dy_scale: torch.Tensor,
                weight_scale: torch.Tensor, height: int, width: int, stride: int,
                padding: int) -> torch.Tensor:
@@ -124,7 +126,7 @@ def _conv_dgrad_fake(dy, weight, dy_scale, weight_scale, height, width, stride, 
     return _empty_cl((dy.shape[0], weight.shape[1], height, width), dy.device)
 
 
-@torch.library.custom_op("dpa_fp8::conv_wgrad", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv_wgrad")
 def conv_wgrad(x: torch.Tensor, dy: torch.Tensor, x_scale: torch.Tensor, dy_scale: torch.Tensor,
                kernel_size: int, stride: int, padding: int, split_k: int,
                out_f32: bool) -> torch.Tensor:
@@ -139,7 +141,7 @@ def _conv_wgrad_fake(x, dy, x_scale, dy_scale, kernel_size, stride, padding, spl
                      torch.float32 if out_f32 else _BF16)
 
 
-@torch.library.custom_op("dpa_fp8::conv_fwd_prepared", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv_fwd_prepared")
 def conv_fwd_prepared(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tensor,
                       weight_scale: torch.Tensor, cout: int, stride: int,
                       padding: int) -> torch.Tensor:
@@ -157,7 +159,7 @@ def _conv_fwd_prepared_fake(x, weight, x_scale, weight_scale, cout, stride, padd
     return _empty_cl((batch, cout, oh, ow), x.device)
 
 
-@torch.library.custom_op("dpa_fp8::conv_dgrad_prepared", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv_dgrad_prepared")
 def conv_dgrad_prepared(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torch.Tensor,
                         weight_scale: torch.Tensor, cin: int, height: int, width: int, k: int,
                         stride: int, padding: int) -> torch.Tensor:
@@ -175,7 +177,7 @@ def _conv_dgrad_prepared_fake(dy, weight_t, dy_scale, weight_scale, cin, height,
 
 
 # ---- GEMM (the FP8 linear) -------------------------------------------------------------
-@torch.library.custom_op("dpa_fp8::gemm", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::gemm")
 def gemm(a: torch.Tensor, b: torch.Tensor, a_scale: torch.Tensor, b_scale: torch.Tensor,
          bias: Optional[torch.Tensor]) -> torch.Tensor:
     return K.linear_fp8_prequantized(a, b, a_scale, b_scale, bias)
@@ -186,7 +188,7 @@ def _gemm_fake(a, b, a_scale, b_scale, bias):
     return a.new_empty((a.shape[0], b.shape[0]), dtype=_BF16)
 
 
-@torch.library.custom_op("dpa_fp8::gemm_dgrad", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::gemm_dgrad")
 def gemm_dgrad(dy: torch.Tensor, weight: torch.Tensor, dy_scale: torch.Tensor,
                weight_scale: torch.Tensor) -> torch.Tensor:
     return K.linear_fp8_dgrad_prequantized(dy, weight, dy_scale, weight_scale)
@@ -197,7 +199,7 @@ def _gemm_dgrad_fake(dy, weight, dy_scale, weight_scale):
     return dy.new_empty((dy.shape[0], weight.shape[1]), dtype=_BF16)
 
 
-@torch.library.custom_op("dpa_fp8::gemm_dgrad_wt", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::gemm_dgrad_wt")
 def gemm_dgrad_wt(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torch.Tensor,
                   weight_scale: torch.Tensor) -> torch.Tensor:
     """gemm_dgrad with the transposed e4m3 weight [K][N] of quantize_with_weight."""
@@ -209,7 +211,7 @@ def _gemm_dgrad_wt_fake(dy, weight_t, dy_scale, weight_scale):
     return dy.new_empty((dy.shape[0], weight_t.shape[0]), dtype=_BF16)
 
 
-@torch.library.custom_op("dpa_fp8::gemm_wgrad", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::gemm_wgrad")
 def gemm_wgrad(x: torch.Tensor, dy: torch.Tensor, x_scale: torch.Tensor, dy_scale: torch.Tensor,
                out_f32: bool) -> torch.Tensor:
     return K.linear_fp8_wgrad_prequantized(x, dy, x_scale, dy_scale, out_f32)
@@ -221,7 +223,7 @@ def _gemm_wgrad_fake(x, dy, x_scale, dy_scale, out_f32):
 
 
 # ---- current-scaling conv and linear with autograd --------------------------------------
-@torch.library.custom_op("dpa_fp8::conv2d_fp8", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::conv2d_fp8")
 def conv2d_fp8(x: torch.Tensor, weight: torch.Tensor, stride: int, padding: int
                ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """(y, e4m3 x, e4m3 w, x scale, w scale): bf16 casts of x and the weight, current-scaling
@@ -273,7 +275,7 @@ def _conv2d_fp8_backward(ctx, dy, *_unused):
 conv2d_fp8.register_autograd(_conv2d_fp8_backward, setup_context=_conv2d_fp8_setup)
 
 
-@torch.library.custom_op("dpa_fp8::linear_fp8", mutates_args=(), device_types="cuda")
+@custom_op("dpa_fp8::linear_fp8")
 def linear_fp8(x: torch.Tensor, weight: torch.Tensor
                ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """(y [..., N], e4m3 x [M, K], e4m3 w, x scale, w scale) of y = x @ w^T with current

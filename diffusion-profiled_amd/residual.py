@@ -12,6 +12,7 @@ import torch
 
 from . import _lib
 from . import fp8_kernels as _fp8
+from .eager import apply
 from .fp8_kernels import FP8_DTYPE, Fp8Handoff, mark_amax_partials, placeholder
 
 # torch divides by a CPU scalar as a product with the fp32 reciprocal of the scalar
@@ -160,16 +161,16 @@ def residual_join(a: torch.Tensor, b: torch.Tensor, hand: Fp8Handoff | None = No
         if not join_kernel_ok(a, b):
             raise ValueError("FP8 hand-off through the residual join: no kernel for these operands")
         if a.dtype == torch.bfloat16:
-            return ResidualScale.apply(a, b, hand)
-        return ResidualScaleF32.apply(a, b, hand)
+            return apply(ResidualScale, a, b, hand)
+        return apply(ResidualScaleF32, a, b, hand)
     if a.is_cuda and _same_dense(a, b) and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0:
         if a.dtype == torch.bfloat16 and b.dtype == torch.bfloat16 and a.numel() % 8 == 0:
-            return ResidualScale.apply(a, b)
+            return apply(ResidualScale, a, b)
         if a.numel() % 4 == 0:
             if a.dtype == torch.float32 and b.dtype == torch.bfloat16:
-                return ResidualScaleF32.apply(a, b)
+                return apply(ResidualScaleF32, a, b)
             if a.dtype == torch.bfloat16 and b.dtype == torch.float32:
-                return ResidualScaleF32.apply(b, a)
+                return apply(ResidualScaleF32, b, a)
     return (a + b) / math.sqrt(2.0)
 
 
@@ -216,7 +217,7 @@ def upsample_concat(a: torch.Tensor, h: torch.Tensor, up: bool) -> torch.Tensor:
             and a.shape[0] == h.shape[0]
             and a.shape[2] << int(up) == h.shape[2] and a.shape[3] << int(up) == h.shape[3]
             and a.data_ptr() % 16 == 0 and h.data_ptr() % 16 == 0):
-        return UpsampleConcat.apply(a, h, up)
+        return apply(UpsampleConcat, a, h, up)
     import torch.nn.functional as F
     x = F.interpolate(a, scale_factor=2.0, mode="nearest") if up else a
     return torch.concat([x, h], dim=1)
@@ -287,7 +288,7 @@ def _down_ok(a: torch.Tensor) -> bool:
 def downsample2(a: torch.Tensor) -> torch.Tensor:
     """F.interpolate(a, scale_factor=0.5, mode="nearest") (fp32 under autocast)."""
     if _down_ok(a):
-        return Downsample2.apply(a)
+        return apply(Downsample2, a)
     import torch.nn.functional as F
     return F.interpolate(a, scale_factor=0.5, mode="nearest")
 
@@ -296,5 +297,5 @@ def downsample2_tee(a: torch.Tensor):
     """(downsample2(a), a) with the second output's gradient added inside the downsampling's
     backward (Downsample2Tee); elsewhere (a, the plain downsampling)."""
     if _down_ok(a):
-        return Downsample2Tee.apply(a)
+        return apply(Downsample2Tee, a)
     return downsample2(a), a

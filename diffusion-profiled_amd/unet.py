@@ -244,7 +244,7 @@ class LinearFP8(_PreparedFP8Weight, nn.Linear):
                 return K.LinearFP8Prepared.apply(x, self.weight, self.bias, pw.q, pw.qt, pw.scale,
                                                  self._fp8_plan.x_cache)
             self._note_fp8_mode("linear", self.weight)
-            return K.LinearFP8Function.apply(x, self.weight, self.bias)
+            return K.linear_fp8_autograd(x, self.weight, self.bias)
         return super().forward(x)
 
 
