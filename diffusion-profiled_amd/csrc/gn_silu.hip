@@ -12,11 +12,12 @@
 // waves. Each lane keeps four 16-B loads in flight. The kernels make several passes over
 // their inputs (after the first mostly from L2).
 //
-// Images of 256+ pixels use a chunked form instead, which spreads each (image, slab) over
-// workgroups of 128 pixels (2048 workgroups at 32x32 x 128 channels, batch 128, against 256
-// for one workgroup per slab, whose passes were latency-bound): every workgroup holds its
-// chunk in registers, and the per-group statistics cross workgroups through a workspace
-// between two launches.
+// Images of up to 1024 pixels, and of up to 4096 in launches that fill the GPU, use a resident
+// form instead, whose workgroups hold their slab in registers. Others of 256+ pixels use a
+// chunked form, which spreads each (image, slab) over workgroups of 128 pixels (against one
+// workgroup per slab, whose passes were latency-bound): every workgroup holds its chunk in
+// registers, and the per-group statistics cross workgroups through a workspace between two
+// launches.
 //   forward:  stats (chunk mean and sum of squared deviations per group) ->
 //             apply (merge the chunks in order, Chan et al.'s pairwise update; normalise)
 //   backward: sums (per-channel chunk sums of the four backward terms) ->
@@ -144,25 +145,24 @@ __device__ __forceinline__ void unpack8(uint4 v, float (&f)[8]) {
   }
 }
 
-// Sum v over the PLN pixel lanes that share this thread's granule (8 per wave by shuffles,
+// Sum v over the PLN pixel lanes that share this thread's granule (64 / NG per wave by shuffles,
 // then the waves in order through LDS); result valid in every lane. red holds
-// (PLN / 8) waves x 8 granules x NV floats.
-template <int NV, int PLN>
+// (NG PLN / 64) waves x NG granules x NV floats.
+template <int NV, int PLN, int NG = 8>
 __device__ __forceinline__ void slab_reduce(float (&v)[NV], float* red) {
-  constexpr int kWaves = PLN / 8;
-  const int gq = threadIdx.x & 7;
+  constexpr int kWaves = NG * PLN / 64;
+  const int gq = threadIdx.x & (NG - 1);
   const int wave = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     float s = v[k];
-    s += __shfl_xor(s, 8, 64);
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
+#pragma unroll
+    for (int x = NG; x < 64; x *= 2) s += __shfl_xor(s, x, 64);
     v[k] = s;
   }
-  if ((threadIdx.x & 63) < 8) {
+  if ((threadIdx.x & 63) < NG) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) red[(wave * 8 + gq) * NV + k] = v[k];
+    for (int k = 0; k < NV; ++k) red[(wave * NG + gq) * NV + k] = v[k];
   }
   __syncthreads();
 #pragma unroll
@@ -171,7 +171,7 @@ __device__ __forceinline__ void slab_reduce(float (&v)[NV], float* red) {
 #pragma unroll(NV <= 2 ? kWaves : 1)
   for (int w = 1; w < kWaves; ++w) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] += red[(w * 8 + gq) * NV + k];
+    for (int k = 0; k < NV; ++k) v[k] += red[(w * NG + gq) * NV + k];
   }
   __syncthreads();
 }
@@ -652,6 +652,12 @@ __device__ __forceinline__ void unpack_x(const uint4 (&v)[NL][U], int u, float (
   }
 }
 
+// This workgroup's number and the launch's workgroups
+struct GnBlk {
+  uint32_t blk = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+  uint32_t count = gridDim.x * gridDim.y * gridDim.z;
+};
+
 // The producer-fused cast in one thread (GnArgs::q): the window scale, its reciprocal for the
 // fast quotient, and the running amax of the bf16 values cast.
 struct GnQ {
@@ -670,14 +676,26 @@ struct GnQ {
     acc = absmax8(acc, v);
   }
   // the workgroup's amax partial (every thread; red: one u32 per wave)
-  __device__ __forceinline__ void finish(const GnArgs& p, uint32_t* red) const {
-    const uint32_t blk = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    store_amax_partial(acc, red, p.q_part, p.q_count, blk, gridDim.x * gridDim.y * gridDim.z);
+  __device__ __forceinline__ void finish(const GnArgs& p, uint32_t* red, GnBlk b = GnBlk()) const {
+    store_amax_partial(acc, red, p.q_part, p.q_count, b.blk, b.count);
   }
 };
 
+// A 16-B store of a slab of NG granules: nontemporal where the slab covers whole cache lines;
+// the pieces of a line that thinner slabs write meet in the L2 (32-B pieces, forward and
+// backward of 32 images of 64x64 x 128: nontemporal 42.0 / 53.6 us, plain 19.5 / 29.1; 64-B
+// pieces of 64 images of 2048 pixels: 15.7 / 28.4 and 18.2 / 27.3, so the forward of those
+// stores as whole lines do).
+template <int NG>
+__device__ __forceinline__ void gn_st16(void* dst, uint4 v) {
+  if constexpr (NG == 8)
+    st_nt16(dst, v);
+  else
+    *static_cast<uint4*>(dst) = v;
+}
+
 // dx of 8 channels at element offset off, in x's type; dx(e) gives channel e's value
-template <bool kF32, typename F>
+template <bool kF32, int NG = 8, typename F>
 __device__ __forceinline__ void store_dx(const GnArgs& p, int64_t off, F dx, GnQ& qo) {
   // with dx_add: dx + add as torch's gradient accumulation forms it (one fp32 add; in bf16 the
   // sum of the two bf16 gradients, rounded once more)
@@ -705,8 +723,8 @@ __device__ __forceinline__ void store_dx(const GnArgs& p, int64_t off, F dx, GnQ
     float* d = static_cast<float*>(p.out) + off;
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      st_nt16(d + 4 * h, uint4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]),
-                               __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])});
+      gn_st16<NG>(d + 4 * h, uint4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]),
+                                   __float_as_uint(v[4 * h + 2]), __float_as_uint(v[4 * h + 3])});
   } else {
     float v[8];
 #pragma unroll
@@ -727,26 +745,27 @@ __device__ __forceinline__ void store_dx(const GnArgs& p, int64_t off, F dx, GnQ
     if (p.q)
       qo.put(p, off, uint4{o[0], o[1], o[2], o[3]});
     else
-      st_nt16(static_cast<uint16_t*>(p.out) + off, uint4{o[0], o[1], o[2], o[3]});
+      gn_st16<NG>(static_cast<uint16_t*>(p.out) + off, uint4{o[0], o[1], o[2], o[3]});
   }
 }
 
 // fp32 x also stored rounded to bf16 (RNE), for a consumer that rounds it anyway (the residual
 // block's 1x1 skip conv), so no separate cast pass reads x again
+template <int NG = 8>
 __device__ __forceinline__ uint4 store_x_bf16(const GnArgs& p, int64_t off, const float (&f)[8]) {
   uint32_t o[4];
 #pragma unroll
   for (int e = 0; e < 8; e += 2) o[e >> 1] = pack_bf16x2(f[e], f[e + 1]);
   const uint4 w = uint4{o[0], o[1], o[2], o[3]};
-  st_nt16(p.x_bf16 + off, w);
+  gn_st16<NG>(p.x_bf16 + off, w);
   return w;
 }
 
 // The workgroup's amax partial of the bf16 copy of x (every thread; red: one u32 per wave), for
 // the current-scaling FP8 conv that quantizes that copy next
-__device__ __forceinline__ void finish_xb_amax(const GnArgs& p, us2 acc, uint32_t* red) {
-  const uint32_t blk = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-  store_amax_partial(acc, red, p.xb_part, nullptr, blk, gridDim.x * gridDim.y * gridDim.z);
+__device__ __forceinline__ void finish_xb_amax(const GnArgs& p, us2 acc, uint32_t* red,
+                                               GnBlk b = GnBlk()) {
+  store_amax_partial(acc, red, p.xb_part, nullptr, b.blk, b.count);
 }
 
 // The channel constants of this thread's 8 channels (gamma, beta, FiLM) and, for the backward,
@@ -1187,11 +1206,43 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_apply_kernel(const Gn
   if (p.q) qo.finish(p, qred);
 }
 
-// ---- resident form (HW <= kResMaxHW: the 32x32, 16x16, 8x8 and 4x4 levels): one workgroup
-// per (image, slab) of PLN pixel lanes x 8 granules holds all of the slab's pixels in
-// registers (U per lane, packed as loaded), so the forward and the backward each read their
+// ---- resident form (HW <= kResMaxHW: the 32x32, 16x16, 8x8 and 4x4 levels; up to four times
+// that on slabs of NG = 4 or 2 granules, see gn_res_shape): one workgroup per (image, slab) of
+// PLN pixel lanes x NG granules holds all of the slab's pixels in registers (U per lane, packed as loaded), so the forward and the backward each read their
 // inputs once and write their outputs once; every pass unpacks from those registers ----
 constexpr int kResMaxHW = 1024;
+
+// A workgroup's image and slab of 8 NG channels. 64-channel slabs: grid (C / 64, N). Thinner ones
+// take part of every cache line of an image, so the workgroups of one image go to one XCD (its
+// L2 then reads and writes each line once): grid 8 ceil(slabs / 8), block b on XCD b mod 8,
+// which has a contiguous range of the slabs in image order.
+template <int NG>
+struct GnSlab {
+  int n, c0;
+  uint32_t idx, total;
+  __device__ __forceinline__ explicit GnSlab(const GnArgs& p) {
+    if constexpr (NG == 8) {
+      n = blockIdx.y;
+      c0 = blockIdx.x * kSlab;
+      idx = total = 0;
+    } else {
+      const uint32_t per_image = p.C / (8 * NG);
+      total = per_image * p.N;
+      idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+      n = (int)(idx / per_image);
+      c0 = (int)(idx - n * per_image) * 8 * NG;
+    }
+  }
+  __device__ __forceinline__ bool live() const { return NG == 8 || idx < total; }
+  __device__ __forceinline__ GnBlk blk() const {
+    GnBlk b;
+    if (NG != 8) {
+      b.blk = idx;
+      b.count = total;
+    }
+    return b;
+  }
+};
 
 // v unchanged, but opaque to the optimiser (no value numbering across this point)
 __device__ __forceinline__ void opaque_u4(uint4& v) {
@@ -1280,17 +1331,19 @@ __device__ __forceinline__ void cat_load(const GnArgs& p, int n, int ch, int pl,
 // one's loads run under the other's arithmetic: the two-source form at 32x32 x 512 (2048
 // workgroups) 111 -> 94 us. With dropout the masks hashed under the loads take that room instead
 // (256 workgroups: 22.4 us with two per CU and the hash at the end, 20.4 so).
-template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false>
-__global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void gn_res_fwd_kernel(const GnArgs p) {
+template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8>
+__global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void gn_res_fwd_kernel(const GnArgs p) {
+  static_assert(!kCat || NG == 8, "64-channel slabs");
   static_assert(!kCat || PLN * U == 1024 || (kF32 && PLN * U == 256), "32x32 or 16x16 images");
-  __shared__ uint32_t qred[PLN / 8];
-  __shared__ float red[(PLN / 8) * 8 * 2];
+  __shared__ uint32_t qred[NG * PLN / 64];
+  __shared__ float red[(NG * PLN / 64) * NG * 2];
   __shared__ float hs[16];
-  const int n = blockIdx.y;
-  const int c0 = blockIdx.x * kSlab;
-  const int gq = threadIdx.x & 7;
-  const int pl = threadIdx.x >> 3;
-  const int ch = c0 + gq * 8;
+  GnSlab<NG> sl(p);
+  if (!sl.live()) return;  // (workgroup-uniform)
+  const int n = sl.n;
+  const int gq = threadIdx.x & (NG - 1);
+  const int pl = threadIdx.x / NG;
+  const int ch = sl.c0 + gq * 8;
   const GnChan<kFilm, false> kc(p, n, ch);
   GnQ qo(p);
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
@@ -1312,7 +1365,7 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
           st_nt16(p.x_bf16 + ((int64_t)n * p.HW + pxs[u]) * p.C + ch, v[0][u]);
           xacc = absmax8(xacc, v[0][u]);
         }
-      if (p.xb_part) finish_xb_amax(p, xacc, qred);
+      if (p.xb_part) finish_xb_amax(p, xacc, qred, sl.blk());
     }
   } else if constexpr (kF32) {
     if (p.x_bf16) {
@@ -1322,9 +1375,9 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
         if (ok[u]) {
           float f[8];
           unpack_x<kF32>(v, u, f);
-          xacc = absmax8(xacc, store_x_bf16(p, ((int64_t)n * p.HW + pxs[u]) * p.C + ch, f));
+          xacc = absmax8(xacc, store_x_bf16<NG>(p, ((int64_t)n * p.HW + pxs[u]) * p.C + ch, f));
         }
-      if (p.xb_part) finish_xb_amax(p, xacc, qred);
+      if (p.xb_part) finish_xb_amax(p, xacc, qred, sl.blk());
     }
   }
   // the dropout masks, hashed while the loads are in flight (beside 128 registers of fp32 x: at
@@ -1350,7 +1403,7 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
       sm[0] += (f[0] + f[1]) + (f[2] + f[3]);
       sm[1] += (f[4] + f[5]) + (f[6] + f[7]);
     }
-  slab_reduce<2, PLN>(sm, red);
+  slab_reduce<2, PLN, NG>(sm, red);
   if (pl == 0) {
     hs[2 * gq] = sm[0];
     hs[2 * gq + 1] = sm[1];
@@ -1381,7 +1434,7 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
         q[e >> 2] += d * d;
       }
     }
-  slab_reduce<2, PLN>(q, red);
+  slab_reduce<2, PLN, NG>(q, red);
   if (pl == 0) {
     hs[2 * gq] = q[0];
     hs[2 * gq + 1] = q[1];
@@ -1419,11 +1472,11 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
       if (p.q)
         qo.put(p, ((int64_t)n * p.HW + px) * p.C + ch, o);
       else
-        st_nt16(ob + (int64_t)px * p.C, o);
+        gn_st16<kF32 || NG != 4 ? NG : 8>(ob + (int64_t)px * p.C, o);
     }
     if constexpr (U >= 16) __builtin_amdgcn_sched_barrier(0);
   }
-  if (p.q) qo.finish(p, qred);
+  if (p.q) qo.finish(p, qred, sl.blk());
 }
 
 // The backward keeps x in registers (packed) and the fp32 g of every pixel, formed in the first
@@ -1434,23 +1487,24 @@ __global__ __launch_bounds__(8 * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void g
 template <int U, bool kFilm, bool kF32, bool kCat>
 constexpr int kGnResLdsG = U < 16 ? 0 : (kF32 ? 9 : (kCat ? 8 : (kFilm ? 6 : 3)));
 
-template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false>
-__global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
+template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8>
+__global__ __launch_bounds__(NG * PLN) void gn_res_bwd_kernel(const GnArgs p) {
   static_assert(!kCat || (!kF32 && PLN == 64 && U == 16) || (kF32 && PLN == 32 && U == 8),
                 "32x32 images (bf16 sources) or 16x16 (cat_h bf16 or fp32)");
   constexpr int kGL = kGnResLdsG<U, kFilm, kF32, kCat>;
-  __shared__ __attribute__((aligned(16))) uint8_t gls[kGL ? kGL * 2 * 8 * PLN * 16 : 16];
-  __shared__ uint32_t qred[PLN / 8];
-  __shared__ float red[(PLN / 8) * 8 * 16];
+  __shared__ __attribute__((aligned(16))) uint8_t gls[kGL ? kGL * 2 * NG * PLN * 16 : 16];
+  __shared__ uint32_t qred[NG * PLN / 64];
+  __shared__ float red[(NG * PLN / 64) * NG * 16];
   __shared__ float hs[2][16];
   // kCat: the pixel rows of one 2x2 window exchange
   constexpr int kXR = U >= 16 ? 2 : 4;
   __shared__ __attribute__((aligned(16))) float xch[kCat ? kXR * (PLN / 4) * 8 * 16 : 4];
-  const int n = blockIdx.y;
-  const int c0 = blockIdx.x * kSlab;
-  const int gq = threadIdx.x & 7;
-  const int pl = threadIdx.x >> 3;
-  const int ch = c0 + gq * 8;
+  GnSlab<NG> sl(p);
+  if (!sl.live()) return;  // (workgroup-uniform)
+  const int n = sl.n;
+  const int gq = threadIdx.x & (NG - 1);
+  const int pl = threadIdx.x / NG;
+  const int ch = sl.c0 + gq * 8;
   const int64_t base = (int64_t)n * p.HW * p.C + ch;
   const uint64_t seed = kDrop ? *p.drop_seed : 0;
   const GnChan<kFilm, true> kc(p, n, ch);
@@ -1489,8 +1543,8 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
       }
     }
     if (u < kGL) {
-      gl[(2 * u) * 8 * PLN] = v4f{g[0], g[1], g[2], g[3]};
-      gl[(2 * u + 1) * 8 * PLN] = v4f{g[4], g[5], g[6], g[7]};
+      gl[(2 * u) * NG * PLN] = v4f{g[0], g[1], g[2], g[3]};
+      gl[(2 * u + 1) * NG * PLN] = v4f{g[4], g[5], g[6], g[7]};
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e) gk[u][e] = g[e];
@@ -1500,7 +1554,7 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     __builtin_amdgcn_sched_barrier(0);
   }
   const GnChan<kFilm, true> kc2(p, n, ch);  // (again, not kept across the pixels)
-  slab_reduce<16, PLN>(acc, red);
+  slab_reduce<16, PLN, NG>(acc, red);
   gn_bwd_setup<kFilm>(p, kc2, st);
   if (pl == 0) {
     const int64_t nc = (int64_t)p.N * p.C;
@@ -1552,7 +1606,7 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     for (int e = 0; e < 8; ++e) {
       const int h = e >> 2;
       const float xh = __builtin_fmaf(f[e], st.rs[h], st.nmr[h]);
-      const float g = u < kGL ? gl[(2 * u + h) * 8 * PLN][e & 3] : gk[u][e];
+      const float g = u < kGL ? gl[(2 * u + h) * NG * PLN][e & 3] : gk[u][e];
       t[e] = st.rs[h] * __builtin_fmaf(-xh, m2[h], g * st.gC[e] - m1[h]);
     }
   };
@@ -1665,29 +1719,48 @@ __global__ __launch_bounds__(8 * PLN) void gn_res_bwd_kernel(const GnArgs p) {
       pixel_dx(u, t);
       auto dx = [&](int e) __attribute__((always_inline)) { return t[e]; };
       const int px = pl2 + u * PLN;
-      if (px < p.HW) store_dx<kF32>(p, base + (int64_t)px * p.C, dx, qo);
+      if (px < p.HW) store_dx<kF32, NG>(p, base + (int64_t)px * p.C, dx, qo);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (p.q) qo.finish(p, qred);
+  if (p.q) qo.finish(p, qred, sl.blk());
 }
 
-// Resident-form geometry for an image of HW pixels: (pixel lanes, pixels per lane), or
-// (0, 0) when HW exceeds kResMaxHW.
+// Resident-form geometry for an image of HW pixels: pixel lanes, pixels per lane and granules
+// of a slab, or zeros where none is taken. Above kResMaxHW pixels a slab has fewer channels,
+// which have to be whole groups, and a workgroup takes about 12 us (forward) and 19 us
+// (backward) however few there are, so the chunked form's two passes over memory stay the
+// better choice where the launch leaves half of the register room of its rounds unused; for
+// the forward on 16-channel slabs, whose one round ends with the SiLU's arithmetic and nothing
+// under it, an eighth. Forward / backward, us, chunked -> resident, bf16 unless said:
+//   32 images of 64x64 x 128 (all of the room)   21.3 / 42.6 -> 19.6 / 29.0 (fp32: 33.8 / 51.7
+//                                                -> 23.1 / 37.3)
+//   50 of 64x64 x 128 (two rounds, 78 %)         34.1 / 58.0 -> 26.1 / 47.4
+//   30 of 3000 pixels x 128 (69 %)               14.1 / 30.2 -> 15.2 / 25.0
+//   64 of 2048 pixels x 128                      17.8 / 39.0 -> 15.6 / 27.2
+//   40 of 36x36 x 256 (40 %)                     14.1 / 34.1 -> 18.6 / 35.8
+//   1 of 64x64 x 128                              9.6 / 12.4 -> 12.1 / 18.5
 struct GnRes {
-  int pln, u;
+  int pln, u, ng;
 };
-static GnRes gn_res_shape(int HW) {
-  if (HW <= 128) return {32, 4};
-  if (HW <= 256) return {32, 8};
-  if (HW <= kResMaxHW) return {64, 16};
-  return {0, 0};
+static GnRes gn_res_shape(int N, int HW, int C, int G, bool bwd) {
+  if (HW <= 128) return {32, 4, 8};
+  if (HW <= 256) return {32, 8, 8};
+  if (HW <= kResMaxHW) return {64, 16, 8};
+  const int ng = HW <= 2 * kResMaxHW ? 4 : 2;
+  if (HW > 4 * kResMaxHW || (8 * ng) % (C / G) != 0) return {0, 0, 0};
+  const int64_t slabs = (int64_t)(C / (8 * ng)) * N;
+  const int64_t room = ceil_div(slabs, 256) * 256 * (512 * 16 * 8);  // 512 threads of 16 pixels
+  const int64_t used = (int64_t)N * HW * C;
+  const bool strict = !bwd && ng == 2 && slabs <= 256;
+  if (strict ? 8 * used < 7 * room : 2 * used < room) return {0, 0, 0};
+  return {512 / ng, 16, ng};
 }
-// The backward with an fp32 x holds 2 x 16 B of x per pixel in registers: that fits at 16 pixels per lane without FiLM and dropout (their
-// per-channel terms and keep bits are the registers that do not fit); with them, images
-// above 256 pixels take the chunked form.
-static bool gn_res_bwd_ok(int HW, bool x_f32, bool film, bool drop) {
-  return HW <= kResMaxHW && (!x_f32 || HW <= 256 || (!film && !drop));
+// The backward with an fp32 x holds 2 x 16 B of x per pixel in registers: that fits at 16 pixels
+// per lane without FiLM and dropout (their per-channel terms and keep bits are the registers
+// that do not fit); with them, images above 256 pixels take the chunked form.
+static bool gn_res_bwd_ok(const GnRes& rs, bool x_f32, bool film, bool drop) {
+  return rs.ng > 0 && (!x_f32 || rs.u < 16 || (!film && !drop));
 }
 
 static int gn_chunks(int HW) {
@@ -1743,11 +1816,19 @@ struct GnQOut {
 };
 
 // Workgroups of the launch that writes the output (one amax partial each), 0 for the form
-// without the fused cast (HW > 8192 pixels).
-static int64_t gn_q_blocks(int N, int HW, int C) {
-  if (HW <= kResMaxHW) return (int64_t)(C / kSlab) * N;
+// without the fused cast (HW > 8192 pixels). The forward's; the backward never has more (it takes
+// the resident form wherever the forward does, and a slab is more than its chunks).
+static int64_t gn_q_blocks(int N, int HW, int C, int G) {
+  const GnRes rs = gn_res_shape(N, HW, C, G, false);
+  if (rs.ng > 0) return (int64_t)(C / (8 * rs.ng)) * N;
   const int nchunk = gn_chunks(HW);
   return nchunk > 0 ? (int64_t)(C / kSlab) * N * nchunk : 0;
+}
+
+// Launch grid of a resident kernel (GnSlab)
+static dim3 gn_res_grid(const GnRes& rs, int N, int C) {
+  if (rs.ng == 8) return dim3((unsigned)(C / kSlab), (unsigned)N);
+  return dim3((unsigned)(8 * ceil_div((int64_t)(C / (8 * rs.ng)) * N, 8)));
 }
 
 static int gn_set_q(GnArgs& a, const GnQOut* qo, int64_t nblk) {
@@ -1807,10 +1888,12 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
   a.rstd = rstd;
   a.N = N; a.HW = HW; a.C = C; a.G = G; a.cpg = C / G; a.eps = eps;
   const int nchunk = gn_chunks(HW);
-  const GnRes rs = gn_res_shape(HW);
-  const bool resident = rs.pln > 0;
-  const bool chunked = !resident && nchunk > 0 && workspace &&
-                       workspace_bytes >= gn_fwd_workspace(N, HW, G) && aligned(workspace, 8);
+  const GnRes rs = gn_res_shape(N, HW, C, G, false);
+  const bool ws_ok = nchunk > 0 && workspace && workspace_bytes >= gn_fwd_workspace(N, HW, G) &&
+                     aligned(workspace, 8);
+  // (above kResMaxHW a call without the chunked form's workspace keeps its one-launch form)
+  const bool resident = rs.ng > 0 && (HW <= kResMaxHW || ws_ok);
+  const bool chunked = !resident && ws_ok;
   // fp32 x and dropout: the resident form or the chunked form (workspace)
   if ((x_f32 || drop_seed) && !chunked && !resident)
     return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
@@ -1822,7 +1905,7 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
     // the chunked form's apply launch)
     if (!x_bf16) return DPA_ERR_NULL;
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    if (xb_part_cap < gn_q_blocks(N, HW, C)) return DPA_ERR_WORKSPACE;
+    if (xb_part_cap < gn_q_blocks(N, HW, C, G)) return DPA_ERR_WORKSPACE;
     if (!aligned(xb_part, 4)) return DPA_ERR_ALIGN;
     a.xb_part = xb_part;
   }
@@ -1830,7 +1913,7 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
   if (dst != DPA_OK) return dst;
   if (qo) {
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C));
+    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C, G));
     if (qst != DPA_OK) return qst;
     a.out = qo->q;  // not written: the kernels store through a.q
   }
@@ -1850,20 +1933,25 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
     });
     return launch_status();
   }
-  dim3 grid((unsigned)(C / kSlab), (unsigned)N);
   if (resident) {
+    const dim3 rgrid = gn_res_grid(rs, N, C);
     dispatch3(a.fs || a.wb, x_f32, a.drop_seed != nullptr, [&](auto FILM, auto F32, auto DROP) {
       constexpr bool kF = decltype(FILM)::value, k3 = decltype(F32)::value,
                      kD = decltype(DROP)::value;
       if (rs.u == 4)
-        gn_res_fwd_kernel<32, 4, kF, k3, kD><<<grid, 8 * 32, 0, s>>>(a);
+        gn_res_fwd_kernel<32, 4, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
       else if (rs.u == 8)
-        gn_res_fwd_kernel<32, 8, kF, k3, kD><<<grid, 8 * 32, 0, s>>>(a);
+        gn_res_fwd_kernel<32, 8, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
+      else if (rs.ng == 8)
+        gn_res_fwd_kernel<64, 16, kF, k3, kD><<<rgrid, 8 * 64, 0, s>>>(a);
+      else if (rs.ng == 4)
+        gn_res_fwd_kernel<128, 16, kF, k3, kD, false, 4><<<rgrid, 4 * 128, 0, s>>>(a);
       else
-        gn_res_fwd_kernel<64, 16, kF, k3, kD><<<grid, 8 * 64, 0, s>>>(a);
+        gn_res_fwd_kernel<256, 16, kF, k3, kD, false, 2><<<rgrid, 2 * 256, 0, s>>>(a);
     });
     return launch_status();
   }
+  dim3 grid((unsigned)(C / kSlab), (unsigned)N);
   const int pln = gn_pixel_lanes(HW);
   if (pln == 128)
     gn_silu_fwd_kernel<128><<<grid, 8 * 128, 0, (hipStream_t)stream>>>(a);
@@ -1995,11 +2083,13 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
   a.N = N; a.HW = HW; a.C = C; a.G = G; a.cpg = C / G; a.eps = 0.f;
   hipStream_t s = (hipStream_t)stream;
   const int nchunk = gn_chunks(HW);
-  const GnRes rs = gn_res_shape(HW);
+  const GnRes rs = gn_res_shape(N, HW, C, G, true);
+  const bool ws_ok = nchunk > 0 && workspace_bytes >= gn_bwd_workspace(N, HW, C) &&
+                     aligned(workspace, 16);
   const bool resident =
-      gn_res_bwd_ok(HW, x_f32, film_scale || film_wb, drop_seed != nullptr);
-  const bool chunked = !resident && nchunk > 0 && workspace_bytes >= gn_bwd_workspace(N, HW, C) &&
-                       aligned(workspace, 16);
+      gn_res_bwd_ok(rs, x_f32, film_scale || film_wb, drop_seed != nullptr) &&
+      (HW <= kResMaxHW || ws_ok);
+  const bool chunked = !resident && ws_ok;
   if ((x_f32 || drop_seed || dx_add) && !chunked && !resident)
     return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
   if (!aligned(dx_add, 16)) return DPA_ERR_ALIGN;
@@ -2010,7 +2100,7 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
   if (qo) {
     if (x_f32 || dx_add) return DPA_ERR_SHAPE;  // e4m3 of a bf16 dx, nothing added
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C));
+    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C, G));
     if (qst != DPA_OK) return qst;
   }
   const bool film = a.fs || a.wb;
@@ -2031,16 +2121,22 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
           <<<cgrid, 8 * kChPLN, 0, s>>>(a, cp, nchunk);
     });
   } else if (resident) {
-    dim3 grid((unsigned)(C / kSlab), (unsigned)N);
+    const dim3 rgrid = gn_res_grid(rs, N, C);
     dispatch3(film, x_f32, a.drop_seed != nullptr, [&](auto FILM, auto F32, auto DROP) {
       constexpr bool kF = decltype(FILM)::value, k3 = decltype(F32)::value,
                      kD = decltype(DROP)::value;
       if (rs.u == 4)
-        gn_res_bwd_kernel<32, 4, kF, k3, kD><<<grid, 8 * 32, 0, s>>>(a);
+        gn_res_bwd_kernel<32, 4, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
       else if (rs.u == 8)
-        gn_res_bwd_kernel<32, 8, kF, k3, kD><<<grid, 8 * 32, 0, s>>>(a);
-      else if constexpr (!k3 || (!kF && !kD))  // (gn_res_bwd_ok)
-        gn_res_bwd_kernel<64, 16, kF, k3, kD><<<grid, 8 * 64, 0, s>>>(a);
+        gn_res_bwd_kernel<32, 8, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
+      else if constexpr (!k3 || (!kF && !kD)) {  // (gn_res_bwd_ok)
+        if (rs.ng == 8)
+          gn_res_bwd_kernel<64, 16, kF, k3, kD><<<rgrid, 8 * 64, 0, s>>>(a);
+        else if (rs.ng == 4)
+          gn_res_bwd_kernel<128, 16, kF, k3, kD, false, 4><<<rgrid, 4 * 128, 0, s>>>(a);
+        else
+          gn_res_bwd_kernel<256, 16, kF, k3, kD, false, 2><<<rgrid, 2 * 256, 0, s>>>(a);
+      }
     });
   } else {
     dim3 grid((unsigned)(C / kSlab), (unsigned)N);
@@ -2106,7 +2202,7 @@ extern "C" int dpa_gn_silu_bwd_ex(const void* x, int x_dtype, const void* dout, 
 
 extern "C" int dpa_gn_silu_fp8_partials(int N, int HW, int C, int G) {
   if (!gn_shape_ok(N, HW, C, G)) return 0;
-  const int64_t nb = gn_q_blocks(N, HW, C);
+  const int64_t nb = gn_q_blocks(N, HW, C, G);
   return nb <= INT32_MAX ? (int)nb : 0;
 }
 
@@ -2221,7 +2317,7 @@ extern "C" int dpa_upcat_gn_silu_fwd(const void* a, const void* h, int h_dtype, 
   g.rstd = rstd;
   g.x_bf16 = (uint16_t*)x_bf16;
   g.N = N; g.HW = HW; g.C = C; g.G = G; g.cpg = C / G; g.eps = eps;
-  const int64_t nblk = gn_q_blocks(N, HW, C);
+  const int64_t nblk = gn_q_blocks(N, HW, C, G);
   if (xb_partials) {
     if (xb_partials_cap < nblk) return DPA_ERR_WORKSPACE;
     g.xb_part = xb_partials;

@@ -7,7 +7,8 @@ conv consumes after its ``x.to(torch.bfloat16)`` (diffusion/fp8_kernels.py:835).
 (the residual stream below the first level and the decoder's concatenations are fp32 under
 autocast, as in the reference) is normalised as it is, as autocast's fp32 GroupNorm does, and
 its gradient is returned in fp32 by the kernels, for images of up to 8192 pixels (the
-resident form up to 1024 pixels, the chunked form above); other inputs are cast to bf16 first.
+resident form up to 1024 pixels, above that the chunked form or, in launches that fill the GPU,
+the resident form on thinner slabs); other inputs are cast to bf16 first.
 """
 from __future__ import annotations
 
@@ -29,8 +30,7 @@ DTYPE_BF16, DTYPE_F32 = 0, 1  # include/dpa_fp8.h DPA_DTYPE_*
 
 
 def f32_input_ok(x: torch.Tensor) -> bool:
-    """fp32 x that the kernels read directly: resident (<= 1024 pixels) or chunked form
-    (<= 8192 pixels)."""
+    """fp32 x that the kernels read directly: the resident and chunked forms (<= 8192 pixels)."""
     hw = x.shape[2] * x.shape[3]
     return x.dtype == torch.float32 and hw <= 64 * 128
 
@@ -122,7 +122,8 @@ def _xb_partials(x_bf16, groups):
 
 def _fwd_call(x, gamma, beta, fs, fb, wb, out, mean, rstd, groups, eps, seed=None, p_drop=0.0,
               x_bf16=None):
-    """The workspace form of the forward (chunked for images of 1025+ pixels); x bf16 or fp32;
+    """The workspace form of the forward (what the chunked form of images of 1025+ pixels
+    needs); x bf16 or fp32;
     seed: dropout seed tensor (int64 [1]) or None. A bf16 copy x_bf16 of an fp32 x carries the
     amax partials its writer left (for the current-scaling 1x1 skip conv that reads it)."""
     n, c, h, w = x.shape

@@ -264,7 +264,9 @@ int dpa_gn_silu_fwd_bf16(const void* x, const float* gamma, const float* beta,
  *     holding the slab's pixels in registers (no workspace read);
  *   1024 < HW <= 8192 with the workspace: the chunked form, two launches, each (image, slab)
  *     spread over workgroups of 128 pixels whose group statistics (chunk mean and squared
- *     deviations, merged in chunk order) cross through the workspace;
+ *     deviations, merged in chunk order) cross through the workspace; or, for HW <= 4096 in
+ *     launches that fill the GPU and groups that 32 (HW <= 2048) or 16 channels hold, the
+ *     resident form on slabs of that many channels;
  *   otherwise (HW > 8192, or no workspace): one launch of one workgroup per (image, slab)
  *     making three passes over the slab.
  * The FiLM is either film_scale/film_shift (fp32 [N, C]) or film_wb (the bf16 time
@@ -280,8 +282,9 @@ int dpa_gn_silu_fwd_ws_bf16(const void* x, const float* gamma, const float* beta
  * and, from 256 pixels, room for the chunk sums of the chunked backward (two launches like
  * the forward). The backward runs the resident form up to 1024 pixels (fp32 x with FiLM or
  * dropout: up to 256 pixels, since x, the FiLM terms and the keep bits exceed the register
- * file at 16 pixels per lane), the chunked form above that up to 8192 pixels with the full
- * workspace, and the one-launch form with a workspace of only 2*N*C floats. */
+ * file at 16 pixels per lane), above that up to 8192 pixels with the full workspace the
+ * chunked form or, as in the forward, the resident form on thinner slabs, and the one-launch
+ * form with a workspace of only 2*N*C floats. */
 int64_t dpa_gn_silu_bwd_workspace_bytes(int N, int HW, int C, int G);
 
 /* Backward of dpa_gn_silu_fwd_bf16 given dout (bf16, same layout as out). Writes dx (bf16)
@@ -318,7 +321,7 @@ int dpa_gn_silu_film_bwd_bf16(const void* x, const void* dout, const float* gamm
  * in fp32 (nn.GroupNorm runs in float32, diffusion/unet.py:151, :157) and returns an fp32
  * input gradient; with DPA_DTYPE_F32 the kernels read the fp32 x as it is and write dx in
  * fp32 (the output y stays bf16). fp32 x takes the resident form (images of up to 1024
- * pixels; the backward with FiLM or dropout up to 256) or the chunked form (above that, up to
+ * pixels; the backward with FiLM or dropout up to 256) or the forms for larger images (up to
  * 8192 pixels, with a workspace of the *_workspace_bytes size); larger images return
  * DPA_ERR_SHAPE, a missing workspace DPA_ERR_WORKSPACE.
  * Optional dropout of the output (diffusion/unet.py:160, nn.Dropout(p) before conv_2):
@@ -363,8 +366,9 @@ int dpa_gn_silu_bwd_ex(const void* x, int x_dtype, const void* dout, const float
  * dpa_delayed_windows_finalize. Bytes and window record equal those of the unfused pair
  * (bf16 entry, then the deferred cast). Arguments otherwise as dpa_gn_silu_fwd_ex /
  * dpa_gn_silu_bwd_ex; the backward takes bf16 x and no dx_add. The resident form (images of
- * up to 1024 pixels, one partial per (image, 64-channel slab)) and the chunked form (up to
- * 8192 pixels with the workspace, one partial per 128-pixel chunk of each slab) cast; larger
+ * up to 1024 pixels, one partial per (image, slab)) and the forms of larger images (up to
+ * 8192 pixels with the workspace, one partial per 128-pixel chunk of each slab, or per slab
+ * where the resident form runs) cast; larger
  * images return DPA_ERR_SHAPE, a chunked-size image without the workspace
  * DPA_ERR_WORKSPACE. q_partials_cap < dpa_gn_silu_fp8_partials(...) returns
  * DPA_ERR_WORKSPACE. */

@@ -515,3 +515,82 @@ def test_gn_silu_tee_bf16_skip_copy(G, n, c, h, w, x32):
     assert xa.grad.dtype == x.dtype
     assert torch.equal(xa.grad, xb.grad)
     assert torch.equal(ga.grad, gb.grad) and torch.equal(ba.grad, bb.grad)
+
+
+@pytest.mark.parametrize("n,c,groups,h,w,film,f32,p_drop", [
+    (64, 128, 32, 33, 32, False, False, 0.0),    # 32-channel slabs, half of the lanes' room
+    (51, 128, 32, 48, 41, True, False, 0.2),     # ragged pixels, images not a multiple of 8
+    (16, 512, 32, 32, 64, False, True, 0.0),     # 2048 pixels, fp32
+    (64, 128, 4, 32, 64, True, False, 0.0),      # one group a slab
+    (31, 128, 32, 61, 61, False, False, 0.0),    # 16-channel slabs, odd image
+    (33, 128, 32, 64, 64, True, True, 0.2),      # more slabs than one round; fp32, FiLM, dropout
+    (8, 512, 32, 64, 64, True, False, 0.2),      # one group a slab
+    (9, 256, 32, 64, 57, False, False, 0.0),     # the backward alone takes the thin slabs
+], ids=str)
+def test_thin_resident_slabs_vs_single_images(G, n, c, groups, h, w, film, f32, p_drop):
+    """Images of 1025 to 4096 pixels in batches that fill the GPU run as resident slabs of 32
+    or 16 channels; each image by itself runs the chunked form, which sums in another order.
+    fp32 statistics differ by a few ulps (1e-5 holds every fp32 result); a bf16 result differs
+    where that crosses a rounding boundary, by one ulp: of values off by 2e-6 relative at most
+    one in 2^8 * 2e-6, so 2^-8 sqrt(5e-4) = 9e-5 normwise, 2e-4 with a margin. The dropout mask
+    hashes the element's index in the batch, so with dropout image 0 alone compares."""
+    print("thin slabs", n, c, groups, h, w, film, f32, p_drop, flush=True)
+    L, K = dpa_mod("_lib"), dpa_mod("fp8_kernels")
+    g = torch.Generator(device="cuda").manual_seed(n + c + h)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x = (rnd(n, c, h, w) * 1.5 + 0.3).contiguous(memory_format=torch.channels_last)
+    x = x if f32 else x.to(torch.bfloat16)
+    dout = (rnd(n, c, h, w) * 1e-2).to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    gamma, beta = 1.0 + 0.3 * rnd(c), 0.3 * rnd(c)
+    wb = (0.3 * rnd(n, 2 * c)).to(torch.bfloat16) if film else None
+    seed = torch.tensor([987654321], dtype=torch.int64, device="cuda") if p_drop else None
+    p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    hw, dt, st = h * w, int(f32), torch.cuda.current_stream().cuda_stream
+
+    def run(lo, hi):
+        m = hi - lo
+        xs, ds, ws = x[lo:hi], dout[lo:hi], None if wb is None else wb[lo:hi]
+        out, dx = torch.empty_like(xs, dtype=torch.bfloat16), torch.empty_like(xs)
+        stats = [torch.empty(m * groups, device="cuda") for _ in range(2)]
+        dg, db = torch.empty(c, device="cuda"), torch.empty(c, device="cuda")
+        dwb = None if wb is None else torch.empty_like(ws)
+        nb = L.query("dpa_gn_silu_fwd_workspace_bytes", m, hw, c, groups)
+        buf = torch.empty(nb, device="cuda", dtype=torch.uint8)
+        L.call("dpa_gn_silu_fwd_ex", xs.data_ptr(), dt, gamma.data_ptr(), beta.data_ptr(), None,
+               None, p(ws), out.data_ptr(), stats[0].data_ptr(), stats[1].data_ptr(),
+               buf.data_ptr(), nb, m, hw, c, groups, 1e-5, p(seed), p_drop, None, st)
+        nb = L.query("dpa_gn_silu_bwd_workspace_bytes", m, hw, c, groups)
+        buf = torch.empty(nb, device="cuda", dtype=torch.uint8)
+        L.call("dpa_gn_silu_bwd_ex", xs.data_ptr(), dt, ds.data_ptr(), gamma.data_ptr(),
+               beta.data_ptr(), None, None, p(ws), stats[0].data_ptr(), stats[1].data_ptr(),
+               dx.data_ptr(), None, 0, dg.data_ptr(), db.data_ptr(), None, None, p(dwb),
+               buf.data_ptr(), nb, m, hw, c, groups, p(seed), p_drop, st)
+        return out, dx, stats[0], stats[1], dg, db, dwb
+
+    close = lambda a, b: float((a.double() - b.double()).norm() / b.double().norm())  # noqa: E731
+    whole = run(0, n)
+    singles = [run(i, i + 1) for i in range(1 if p_drop else n)]
+    for i, one in enumerate(singles):
+        assert close(whole[0][i], one[0][0]) < 2e-4, i
+        assert close(whole[1][i], one[1][0]) < (1e-5 if f32 else 2e-4), i
+        for k in (2, 3):
+            assert close(whole[k][i * groups:(i + 1) * groups], one[k]) < 1e-5, i
+        if film:
+            assert close(whole[6][i], one[6][0]) < 2e-4, i
+    if not p_drop:
+        for k in (4, 5):
+            assert close(whole[k], torch.stack([one[k].double() for one in singles]).sum(0)) < 1e-5
+    # the e4m3 output and the bf16 copy of an fp32 x come from the same values
+    hand = K.Fp8Handoff(torch.tensor(0.01, device="cuda"), torch.zeros(1 << 16, device="cuda",
+                        dtype=torch.int32), torch.zeros(1, device="cuda", dtype=torch.int32))
+    part = [torch.zeros_like(hand.partials), torch.zeros_like(hand.count)]
+    x16 = torch.empty_like(x, dtype=torch.bfloat16) if f32 else None
+    stats = [torch.empty(n * groups, device="cuda") for _ in range(2)]
+    G._fwd_fp8_call(x, gamma, beta, wb, hand, *stats, groups, 1e-5, seed, p_drop, x16)
+    q = K.quantize_fp8_delayed_deferred(whole[0], hand.scale, *part)
+    assert torch.equal(hand.q.view(torch.uint8), q.view(torch.uint8))
+    assert int(hand.partials[:int(hand.count)].max()) == int(part[0][:int(part[1])].max())
+    if f32:
+        assert torch.equal(x16, x.to(torch.bfloat16))
+        (qa, sa), (qb, sb) = K.quantize_fp8_from_producer(x16, x16), K.quantize_fp8(x16)
+        assert torch.equal(sa, sb) and torch.equal(qa.view(torch.uint8), qb.view(torch.uint8))
