@@ -169,15 +169,18 @@ class ConvWorkload:
 
     def kernel_names(self):
         """Kernels the library launches for this layer's GEMMs, following its dispatch
-        (csrc/igemm.hip use_hconv, csrc/wgrad.hip use_hwgrad): 3x3 / stride-1 convs of 16- or
-        32-wide images go to the halo-patch and three-tap kernels."""
+        (csrc/igemm.hip use_hconv and onetap_ok, csrc/wgrad.hip use_hwgrad): 3x3 / stride-1 convs
+        of 16- or 32-wide images go to the halo-patch and three-tap kernels, 1x1 convs that reduce
+        over at most 512 channels to the one-tap kernel."""
         s1 = self.k == 3 and self.stride == 1 and self.pad == 1 and self.w in (16, 32)
         conv = "hconv_fp8_kernel" if (s1 and self.h % (256 // self.w) == 0) else "igemm_fp8_kernel"
         if s1 and self.h % (128 // self.w) == 0 and self.cin % 64 == 0:
             wg = f"hwgrad_partial_kernel<{self.w}>+wgrad_reduce_kernel"
         else:
             wg = "wgrad_partial_kernel+wgrad_reduce_kernel"
-        return {"fwd": conv, "dgrad": conv, "wgrad": wg}
+        fwd, dgrad = ("onetap_fp8_kernel" if self.k == 1 and c <= 512 else conv
+                      for c in (self.cin, self.cout))
+        return {"fwd": fwd, "dgrad": dgrad, "wgrad": wg}
 
     def config(self):
         return {
@@ -756,7 +759,7 @@ def main():
     tflops = wl.step_flop() / dt / 1e12
     # dominant kernel = the MFMA kernel with the most device time per step: the conv kernel
     # (one fwd and one dgrad launch) or the weight-gradient pair (partial + split reduce)
-    names = wl.kernel_names() if hasattr(wl, "kernel_names") else {"fwd": "igemm_fp8_kernel"}
+    names = wl.kernel_names() if hasattr(wl, "kernel_names") else {"fwd": "onetap_fp8_kernel"}
     conv_launches = [parts[k] for k in ("fwd", "dgrad") if k in parts]
     if "wgrad" in parts and parts["wgrad"] > sum(conv_launches):
         dominant, dom_us, dom_bytes = names["wgrad"], parts["wgrad"], wl.bytes["wgrad"]

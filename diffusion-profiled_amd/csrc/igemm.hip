@@ -4,7 +4,8 @@
 //   conv2d_fwd_fp8_kernel  :142-247 (+ launcher :604-639)  -> dpa_conv2d_fwd_fp8
 //   conv2d_dx_fp8_kernel   :250-318 (+ launcher :671-709)  -> dpa_conv2d_dgrad_fp8
 //
-// One kernel serves every case. The GEMM is
+// One kernel serves every case but the one-tap launches with a short K (onetap_fp8_kernel
+// below). The GEMM is
 //   out[pix, co] = sum_{tap, c} act[pix shifted by tap, c] * wgt[co, tap, c]
 // over a tap grid (ty, tx) in [0, ny) x [0, nx) whose input offset and weight tap are linear
 // in (ty, tx). Forward convs (stride 1 or 2, 3x3 or 1x1) use the natural grid; the data
@@ -430,6 +431,152 @@ __global__ __launch_bounds__(kIgThreads, 1) void igemm_fp8_kernel(const IgemmArg
   wait_vmcnt<0>();  // trailing zero-page DMAs land before the workgroup retires
 }
 
+// One tap, one stride, K = 128 KC <= 512 (the 1x1 convs and the linears): a workgroup of 4 waves
+// keeps one 128-channel block's weights in registers (wave w: channels 32 w .. + 31 over all of
+// K) and streams 64-pixel tiles of the activation through a two-stage LDS ring. Such a launch is
+// bound by its output, 2 B per pixel and channel against K / Cout B read, so what counts is that
+// stores never stop: several workgroups per CU, each a whole load-product-store sequence at its
+// own pace, and a tile leaves in 256-B runs through an LDS block. The sums are those of
+// igemm_fp8_kernel (K ascending), so are the bytes. us, igemm_fp8_kernel -> this: 32768 x 256 ->
+// 768 21.7 -> 14.4 (50 MB out at 3.5 TB/s), 131072 x 128 -> 512 44.1 -> 28.4 (4.7 TB/s), 131072 x
+// 256 -> 128 18.6 -> 12.2, 32768 x 256 -> 256 10.8 -> 8.0, 8192 x 256 -> 768 9.5 -> 7.0, 40000 x
+// 512 -> 1024 48.5 -> 35.0.
+struct OneTapArgs {
+  const uint8_t* act;  // [M][C]
+  const uint8_t* wgt;  // [Cout][C]
+  uint16_t* out;       // bf16 [M][Cout]
+  const float* sa;
+  const float* sb;
+  const float* bias;   // [Cout] or null
+  int M, C, Cout, tiles_n;
+  int tm_per_xcd, slots;  // 64-pixel tiles per XCD, workgroups per XCD and channel block
+};
+constexpr int kOtThreads = 256;
+constexpr int kOtBM = 64;
+constexpr int kOtSlotBytes = kOtBM * kBN * 2;
+
+template <int KC>
+__global__ __launch_bounds__(kOtThreads, KC <= 2 ? 3 : 2) void onetap_fp8_kernel(const OneTapArgs p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t st[2][KC * kOtBM * kBK];
+  __shared__ __attribute__((aligned(1024))) uint8_t slot[kOtSlotBytes];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frow = lane & 15, fq = lane >> 4;
+
+  // XCD x owns 64-pixel tiles [x * tm_per_xcd, + tm_per_xcd); its workgroups are (slot, channel
+  // block), the blocks of one slot side by side, so a tile is read from the L2 by all of them
+  // at about the same time; slot i takes tiles i, i + slots, ...
+  const int wi = blockIdx.x >> 3;
+  const int sl = wi / p.tiles_n;
+  const int n0 = (wi - sl * p.tiles_n) * kBN;
+  const int t_first = (blockIdx.x & 7) * p.tm_per_xcd;
+  const int tiles_m = (p.M + kOtBM - 1) / kOtBM;
+  int t_end = t_first + p.tm_per_xcd;
+  if (t_end > tiles_m) t_end = tiles_m;
+  const int t_begin = t_first + sl;
+  if (t_begin >= t_end) return;
+
+  // tile t into stage b: rows of 128 B per 128-channel chunk, granule g of row r at g ^ swz(r)
+  auto issue = [&](int b, int t) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int row = wave * 16 + 8 * r + (lane >> 3);
+      const int m = t * kOtBM + row;
+      const bool ok = (t < t_end) & (m < p.M);
+      const uint8_t* src = p.act + ((uint32_t)m * (uint32_t)p.C + ((lane & 7) ^ swz(row)) * 16);
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc)
+        dma16(ok ? src + kc * kBK : (const uint8_t*)g_zero16,
+              st[b] + (kc * kOtBM + wave * 16 + 8 * r) * kBK);
+    }
+  };
+
+  issue(0, t_begin);
+  const float scale = p.sa[0] * p.sb[0];
+  v8i fb[2][KC];
+  v4f bias[2];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb) {
+    const int c = n0 + wave * 32 + cb * 16;
+    const uint8_t* w = p.wgt + (uint32_t)((c + frow) * p.C + 32 * fq);
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      const uint4 lo = *reinterpret_cast<const uint4*>(w + kc * kBK);
+      const uint4 hi = *reinterpret_cast<const uint4*>(w + kc * kBK + 16);
+      fb[cb][kc] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w,
+                       (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
+    }
+    bias[cb] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[cb][e] = p.bias[c + 4 * fq + e];
+    }
+  }
+  wait_vmcnt<0>();
+
+  int b = 0;
+  for (int t = t_begin; t < t_end; t += p.slots) {
+    // tile t has landed (waited for below or above); every wave is past the stage and the slot
+    // of the tile before
+    wait_lgkmcnt0();
+    lds_barrier();
+    issue(b ^ 1, t + p.slots);
+    v4f acc[2][4];
+#pragma unroll
+    for (int pf = 0; pf < 4; ++pf) {
+      acc[0][pf] = acc[1][pf] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const v8i fa = ld_frag(st[b] + kc * kOtBM * kBK, pf * 16 + frow, fq);
+        acc[0][pf] = mfma16x16x128_e4m3(fb[0][kc], fa, acc[0][pf]);
+        acc[1][pf] = mfma16x16x128_e4m3(fb[1][kc], fa, acc[1][pf]);
+      }
+    }
+    // slot rows of 256 B (a pixel's 128 channels), granule g of row r at g ^ (r & 15)
+#pragma unroll
+    for (int pf = 0; pf < 4; ++pf) {
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[cb][pf][e] * scale;
+        if (p.bias) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = v[e] + bias[cb][e];
+        }
+        const int g = wave * 4 + cb * 2 + (fq >> 1);
+        *reinterpret_cast<uint2*>(slot + (pf * 16 + frow) * 256 + ((g ^ frow) * 16) +
+                                  (fq & 1) * 8) =
+            uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+      }
+    }
+    wait_lgkmcnt0();
+    lds_barrier();
+    const int m0 = t * kOtBM, g = tid & 15;
+    if (m0 + kOtBM <= p.M) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = r * 16 + (tid >> 4);
+        const uint4 v = *reinterpret_cast<const uint4*>(slot + row * 256 + ((g ^ (row & 15)) * 16));
+        st_nt16(p.out + (uint32_t)((m0 + row) * p.Cout + n0 + g * 8), v);
+      }
+      // the next tile's DMAs, issued before these four stores
+      wait_vmcnt<4>();
+    } else {  // (the launch's last tile of pixels)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = r * 16 + (tid >> 4);
+        const uint4 v = *reinterpret_cast<const uint4*>(slot + row * 256 + ((g ^ (row & 15)) * 16));
+        if (m0 + row < p.M) st_nt16(p.out + (uint32_t)((m0 + row) * p.Cout + n0 + g * 8), v);
+      }
+      wait_vmcnt<0>();
+    }
+    b ^= 1;
+  }
+  wait_vmcnt<0>();  // trailing zero-page DMAs land before the workgroup retires
+}
+
 // wt[ci][r][s][co] = w[co][r][s][ci] (e4m3 bytes): 32x32 byte tiles through LDS.
 __global__ __launch_bounds__(256) void weight_transpose_kernel(const uint8_t* __restrict__ w,
                                                                uint8_t* __restrict__ wt,
@@ -535,6 +682,40 @@ static int64_t igemm_workspace(IgemmArgs& a) {
   return bytes;
 }
 
+// Launches of onetap_fp8_kernel: with K <= 256 of any size, with 384 and 512 those whose tiles
+// reach a quarter of the CUs (below, 64 x 32 tiles of the general kernel load fewer weights per
+// workgroup: 128 x 512 -> 512 4.9 us there, 5.1 here; 4096 x 512 -> 128, 64 tiles, 5.5 and 5.4;
+// 10001 x 128 -> 128 5.3 and 3.5). K > 512 would not leave registers for the weights.
+static bool onetap_ok(const IgemmArgs& a) {
+  if (a.iy_step != 1 || a.ix_step != 1 || a.oy_step != 1 || a.ox_step != 1) return false;
+  return a.nk <= 2 || (a.nk <= 4 && ceil_div(a.M, kOtBM) * a.tiles_n * 4 >= num_cus());
+}
+
+static int launch_onetap(const IgemmArgs& a, hipStream_t s) {
+  const int kc = a.C / kBK;
+  OneTapArgs o{};
+  o.act = a.act; o.wgt = a.wgt; o.out = a.out;
+  o.sa = a.sa; o.sb = a.sb; o.bias = a.bias;
+  o.M = a.M; o.C = a.C; o.Cout = a.Cout;
+  o.tiles_n = a.Cout / kBN;
+  o.tm_per_xcd = (int)ceil_div(ceil_div(a.M, kOtBM), 8);
+  // workgroups of a CU (32, 48, 64 or 80 KB of LDS each). us with 2 / 3 / 4 of them: 32768 x 256 ->
+  // 256 10.1 / 8.0 / 10.5 (4: more than fit), 131072 x 128 -> 512 32.5 / 28.4 / 29.6
+  const int per_cu = kc <= 2 ? 3 : 2;
+  int slots = (num_cus() / 8) * per_cu / o.tiles_n;
+  if (slots < 1) slots = 1;
+  if (slots > o.tm_per_xcd) slots = o.tm_per_xcd;
+  o.slots = slots;
+  const unsigned grid = 8u * (unsigned)slots * (unsigned)o.tiles_n;
+  switch (kc) {
+    case 1: onetap_fp8_kernel<1><<<grid, kOtThreads, 0, s>>>(o); break;
+    case 2: onetap_fp8_kernel<2><<<grid, kOtThreads, 0, s>>>(o); break;
+    case 3: onetap_fp8_kernel<3><<<grid, kOtThreads, 0, s>>>(o); break;
+    default: onetap_fp8_kernel<4><<<grid, kOtThreads, 0, s>>>(o); break;
+  }
+  return launch_status();
+}
+
 // act geometry (N, Hi, Wi, C), output geometry, tap grid already in `a`; split K when a
 // workspace of the planned size is given
 static int launch_igemm(IgemmArgs& a, int N, hipStream_t s, void* workspace,
@@ -547,6 +728,8 @@ static int launch_igemm(IgemmArgs& a, int N, hipStream_t s, void* workspace,
     return DPA_ERR_SIZE;
   finish_geometry(a);
   if (a.nclass <= 1) a.nclass = 1;  // one class: the scalar tap grid
+  if (a.nclass == 1 && a.T == 1 && onetap_ok(a))
+    return launch_onetap(a, s);
   // Launches whose 256-pixel tiles would leave at least half the CUs idle take 128-pixel
   // tiles (twice as many) unsplit, when a tile has at most kHalfMaxSteps K-steps, and
   // 64-pixel tiles when the 128-pixel ones would still leave half the CUs idle.

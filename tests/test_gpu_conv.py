@@ -411,3 +411,37 @@ def test_weight_gradient_strips(K, shape):
         # fp32 sums' error, which is below 2^-12 of the root mean square here
         tol = 2**-7 * ref.abs() + 2**-12 * ref.square().mean().sqrt()
         assert bool(((got.double() - ref).abs() <= tol).all())
+
+
+# the one-tap kernel: 1 to 4 K chunks, ragged and single-row tiles, fewer tiles than XCDs, several
+# tiles per workgroup with a ragged last one, more channel blocks than an XCD has workgroups
+ONE_TAP = [(1, 128, 128), (63, 256, 384), (65, 128, 256), (700, 256, 128), (4161, 512, 128),
+           (5000, 384, 512), (20001, 256, 768), (60000, 128, 384), (130, 128, 128 * 101),
+           (9000, 512, 1024)]
+
+
+@pytest.mark.parametrize("m,k,n", ONE_TAP, ids=lambda v: str(v))
+def test_one_tap_products(K, m, k, n):
+    """The linear with and without bias and the 1x1 conv against the general kernel, bit for bit:
+    the same operands with zero columns up to K = 640 are that kernel's, and its sums run over
+    K ascending too, so the zeros add nothing. Rows past the last stay as they were; the first
+    rows against the exact oracle."""
+    lib = dpa_mod("_lib")
+    xq, xs = K.quantize_fp8_tensor(randn_bf16((m, k), seed=m).cuda())
+    wq, ws = K.quantize_fp8_tensor(randn_bf16((n, k), seed=n, std=0.05).cuda())
+    bias = torch.linspace(-1, 1, n, device="cuda")
+    wide_x, wide_w = (F.pad(t.view(torch.uint8), (0, 640 - k)).view(t.dtype) for t in (xq, wq))
+    out = torch.full((m + 64, n), 3.0, device="cuda", dtype=torch.bfloat16)
+    stream = torch.cuda.current_stream().cuda_stream
+    for b in (bias, None):
+        lib.call("dpa_gemm_fp8", xq.data_ptr(), wq.data_ptr(), xs.data_ptr(), ws.data_ptr(),
+                 0 if b is None else b.data_ptr(), out.data_ptr(), m, n, k, stream)
+        assert torch.equal(out[:m], K.linear_fp8_prequantized(wide_x, wide_w, xs, ws, b))
+        assert bool((out[m:] == 3.0).all())
+    x4 = xq.view(m, 1, 1, k).permute(0, 3, 1, 2)
+    w4 = wq.view(n, 1, 1, k).permute(0, 3, 1, 2)
+    y4 = K.conv2d_fp8_fwd_general(x4, w4, xs, ws, 1, 0)
+    assert torch.equal(y4.permute(0, 2, 3, 1).reshape(m, n), out[:m])
+    xb, wb = (nhwc_bits(t.cpu().view(torch.uint8)) for t in (x4[:8], w4[:256]))
+    assert_bf16_close(nhwc_bits(y4[:8, :256].cpu()),
+                      O.conv2d_fwd(xb, wb, f32(xs), f32(ws), stride=1, pad=0), f"{m} {k} {n}")
