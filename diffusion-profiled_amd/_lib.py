@@ -72,6 +72,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "dpa_conv2d_fwd_fp8_frag": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_void_p]),
     "dpa_conv2d_dgrad_fp8_frag": (c_int, [c_void_p] * 5 + [c_int] * 5 + [c_void_p]),
     "dpa_conv2d_frag_supported": (c_int, [c_int] * 5),
+    "dpa_conv2d_kernel": (c_char_p, [c_int, c_void_p] + [c_int] * 9),
     "dpa_conv2d_wgrad_workspace_bytes": (c_int64, [c_int] * 10),
     "dpa_conv2d_wgrad_fp8": (
         c_int,

@@ -691,6 +691,12 @@ static bool onetap_ok(const IgemmArgs& a) {
   return a.nk <= 2 || (a.nk <= 4 && ceil_div(a.M, kOtBM) * a.tiles_n * 4 >= num_cus());
 }
 
+// Whether a launch (its geometry finished) takes it: its epilogue stores 16 B per lane, while the
+// entries accept an output that is aligned to 8 B, which igemm_fp8_kernel stores.
+static bool use_onetap(const IgemmArgs& a) {
+  return a.nclass <= 1 && a.T == 1 && onetap_ok(a) && aligned(a.out, 16);
+}
+
 static int launch_onetap(const IgemmArgs& a, hipStream_t s) {
   const int kc = a.C / kBK;
   OneTapArgs o{};
@@ -728,8 +734,7 @@ static int launch_igemm(IgemmArgs& a, int N, hipStream_t s, void* workspace,
     return DPA_ERR_SIZE;
   finish_geometry(a);
   if (a.nclass <= 1) a.nclass = 1;  // one class: the scalar tap grid
-  if (a.nclass == 1 && a.T == 1 && onetap_ok(a))
-    return launch_onetap(a, s);
+  if (use_onetap(a)) return launch_onetap(a, s);
   // Launches whose 256-pixel tiles would leave at least half the CUs idle take 128-pixel
   // tiles (twice as many) unsplit, when a tile has at most kHalfMaxSteps K-steps, and
   // 64-pixel tiles when the 128-pixel ones would still leave half the CUs idle.
@@ -981,6 +986,25 @@ extern "C" int dpa_conv2d_fwd_fp8(const void* xq, const void* wq, const float* x
   if (!aligned(xq, 16) || !aligned(wq, 16) || !aligned(y, 8)) return DPA_ERR_ALIGN;
   return conv_fwd(xq, wq, x_scale, w_scale, bias, y, N, H, W, Cin, Cout, R, S, stride, pad,
                   (hipStream_t)stream);
+}
+
+extern "C" const char* dpa_conv2d_kernel(int product, const void* out, int N, int H, int W, int Cin,
+                                         int Cout, int R, int S, int stride, int pad) {
+  const bool bwd = product == 1;
+  if (product < 0 || product > 1) return nullptr;
+  if (!conv_shape_ok(N, H, W, bwd ? Cout : Cin, bwd ? Cin : Cout, R, S, stride, pad))
+    return nullptr;
+  if (use_hconv(N, H, W, bwd ? Cout : Cin, bwd ? Cin : Cout, R, S, stride, pad) &&
+      aligned(out, 16))
+    return "hconv_fp8_kernel";
+  IgemmArgs a{};
+  a.out = (uint16_t*)out;
+  if (!bwd)
+    fwd_geometry(a, N, H, W, Cin, Cout, R, S, stride, pad);
+  else if (dgrad_geometry(a, N, H, W, Cin, Cout, R, S, stride, pad, 0, 0) != DPA_OK)
+    return nullptr;
+  finish_geometry(a);
+  return use_onetap(a) ? "onetap_fp8_kernel" : "igemm_fp8_kernel";
 }
 
 extern "C" int64_t dpa_conv2d_dgrad_workspace_bytes(int Cin, int Cout, int R, int S) {

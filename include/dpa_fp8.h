@@ -170,6 +170,13 @@ int dpa_conv2d_dgrad_fp8_frag(const void* dyq, const void* wf_dgrad, const float
                               const float* w_scale, void* dx, int N, int H, int W, int Cin,
                               int Cout, void* stream);
 
+/* Name of the kernel that forms a product into out: product 0 = forward (dpa_conv2d_fwd_fp8 and
+ * its _split form; a linear [M, K] x [N, K]^T is the 1x1 conv N = M, H = W = 1, Cin = K, Cout =
+ * N), 1 = data gradient (dpa_conv2d_dgrad_fp8, _wt, _wt_split). Of out only the alignment counts,
+ * nothing is launched. NULL: those entries refuse the shape. */
+const char* dpa_conv2d_kernel(int product, const void* out, int N, int H, int W, int Cin, int Cout,
+                              int R, int S, int stride, int pad);
+
 /* Bytes of workspace dpa_conv2d_dgrad_fp8 needs (the transposed weight, Cout*R*S*Cin). */
 int64_t dpa_conv2d_dgrad_workspace_bytes(int Cin, int Cout, int R, int S);
 

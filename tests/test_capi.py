@@ -246,3 +246,23 @@ def test_fragment_conv_shapes_agree_with_the_python_rule(lib):
     assert q(fake, 16, fake, fake, fake, 2, 128, 9, 64, fake, fake, fake, fake, need, nul) == -4
     assert q(fake, 16, fake, fake, odd, 0, 128, 9, 128, fake, fake, fake, fake, need, nul) == -3
     assert q(fake, 16, fake, fake, fake, 0, 128, 9, 128, fake, fake, fake, fake, need - 4, nul) == -5
+
+
+def test_wide_store_kernels_need_an_aligned_output(lib):
+    """The entries accept an output aligned to 8 B. The kernels whose epilogue stores 16 B per
+    lane take only 16-B aligned ones; the rest go to the kernel that stores 8 B."""
+    def kernel(product, out, n, h, w, cin, cout, k=1, stride=1):
+        return lib.dpa_conv2d_kernel(product, out, n, h, w, cin, cout, k, k, stride, k // 2)
+
+    for out, onetap, hconv in ((0x1000, b"onetap_fp8_kernel", b"hconv_fp8_kernel"),
+                               (0x1008, b"igemm_fp8_kernel", b"igemm_fp8_kernel")):
+        for k in (128, 256, 384, 512):
+            assert kernel(0, out, 4096, 1, 1, k, 768) == onetap       # a linear, y
+            assert kernel(1, out, 4096, 1, 1, 768, k) == onetap       # its dx
+            assert kernel(0, out, 16, 16, 16, k, 256) == onetap       # a 1x1 conv
+        assert kernel(0, out, 4, 32, 32, 128, 128, 3) == hconv
+        assert kernel(1, out, 4, 32, 32, 128, 128, 3) == hconv
+        assert kernel(0, out, 4096, 1, 1, 640, 768) == b"igemm_fp8_kernel"
+        assert kernel(0, out, 4, 32, 32, 128, 128, 3, 2) == b"igemm_fp8_kernel"
+        assert kernel(1, out, 4, 32, 32, 128, 128, 3, 2) == b"igemm_fp8_kernel"
+    assert kernel(0, 0x1000, 4, 32, 32, 96, 128) is None and kernel(2, 0x1000, 4, 1, 1, 128, 128) is None

@@ -445,3 +445,26 @@ def test_one_tap_products(K, m, k, n):
     xb, wb = (nhwc_bits(t.cpu().view(torch.uint8)) for t in (x4[:8], w4[:256]))
     assert_bf16_close(nhwc_bits(y4[:8, :256].cpu()),
                       O.conv2d_fwd(xb, wb, f32(xs), f32(ws), stride=1, pad=0), f"{m} {k} {n}")
+
+
+@pytest.mark.parametrize("m,k,n", [(700, 256, 128), (4161, 512, 128)], ids=str)
+def test_one_tap_products_into_outputs_aligned_to_8(K, m, k, n):
+    """An output at 8 mod 16 B, which the entries accept: the linear and its data gradient write
+    the same bits as into an aligned one, and nothing before or behind it."""
+    lib = dpa_mod("_lib")
+    xq, xs = K.quantize_fp8_tensor(randn_bf16((m, k), seed=m).cuda())
+    wq, ws = K.quantize_fp8_tensor(randn_bf16((n, k), seed=n, std=0.05).cuda())
+    bias = torch.linspace(-1, 1, n, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    buf = torch.full((8 + m * n + 60,), 3.0, device="cuda", dtype=torch.bfloat16)
+    y = buf[4:4 + m * n]
+    assert buf.data_ptr() % 16 == 0 and y.data_ptr() % 16 == 8
+    lib.call("dpa_gemm_fp8", xq.data_ptr(), wq.data_ptr(), xs.data_ptr(), ws.data_ptr(),
+             bias.data_ptr(), y.data_ptr(), m, n, k, stream)
+    assert torch.equal(y.view(m, n), K.linear_fp8_prequantized(xq, wq, xs, ws, bias))
+    assert bool((buf[:4] == 3.0).all()) and bool((buf[4 + m * n:] == 3.0).all())
+    # the same product as the data gradient of a linear with n inputs and k outputs
+    lib.call("dpa_conv2d_dgrad_fp8_wt", xq.data_ptr(), wq.data_ptr(), xs.data_ptr(), ws.data_ptr(),
+             y.data_ptr(), m, 1, 1, n, k, 1, 1, 1, 0, stream)
+    assert torch.equal(y.view(m, n), K.linear_fp8_prequantized(xq, wq, xs, ws))
+    assert bool((buf[:4] == 3.0).all()) and bool((buf[4 + m * n:] == 3.0).all())
