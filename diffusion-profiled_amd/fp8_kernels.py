@@ -148,6 +148,7 @@ def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool
     quantize_fp8 of x and of the bf16 weight. weight: fp32 or bf16, [Cout, Cin, k, k] or [N, K].
     The weight's copies are the OHWI / [N][K] bytes and their [Cin][k][k][Cout] / [K][N]
     transpose, or with ``frag`` the halo-patch conv's two fragment layouts (flat uint8)."""
+    assert x.is_cuda and weight.device == x.device, f"{x.device} {weight.device}"
     if not _dense(x):
         x = x.contiguous()
     if weight.dtype not in (torch.float32, torch.bfloat16) or weight.data_ptr() % 16:
@@ -704,7 +705,7 @@ def _conv_current_fwd(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: i
     """Current-scaling conv forward of a bf16 channels-last x and an fp32 or bf16 weight, saving
     e4m3 x and the weight's data-gradient copy."""
     assert x.dtype == torch.bfloat16 and x.is_cuda and x.ndim == 4, f"{x.dtype} {x.is_cuda} {x.ndim}"
-    assert weight.is_cuda and weight.ndim == 4, f"{weight.is_cuda} {weight.ndim}"
+    assert weight.device == x.device and weight.ndim == 4, f"{weight.device} {x.device} {weight.ndim}"
     batch, cin, height, width = x.shape
     cout, wcin, kh, kw = weight.shape
     assert wcin == cin and kh == kw
@@ -1017,7 +1018,7 @@ class LinearFP8Function(torch.autograd.Function):
         n, k = weight.shape
         assert x.shape[-1] == k
         x2 = x.to(torch.bfloat16).reshape(-1, k).contiguous()
-        assert x2.is_cuda and weight.is_cuda, f"{x2.is_cuda} {weight.is_cuda}"
+        assert x2.is_cuda and weight.device == x2.device, f"{x2.device} {weight.device}"
         xq, xs, wq, wt, wsc = run_in(ctx, _ops.quantize_with_weight, x2, weight, False)
         b32 = None if bias is None else bias.detach().float().contiguous()
         y = run_in(ctx, _ops.gemm, xq, wq, xs, wsc, b32)
