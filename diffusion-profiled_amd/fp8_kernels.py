@@ -148,7 +148,9 @@ def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool
     quantize_fp8 of x and of the bf16 weight. weight: fp32 or bf16, [Cout, Cin, k, k] or [N, K].
     The weight's copies are the OHWI / [N][K] bytes and their [Cin][k][k][Cout] / [K][N]
     transpose, or with ``frag`` the halo-patch conv's two fragment layouts (flat uint8)."""
+    assert x.dtype == torch.bfloat16, f"{x.dtype}"
     assert x.is_cuda and weight.device == x.device, f"{x.device} {weight.device}"
+    assert weight.ndim in (2, 4) and (weight.ndim == 4 or not frag)
     if not _dense(x):
         x = x.contiguous()
     if weight.dtype not in (torch.float32, torch.bfloat16) or weight.data_ptr() % 16:
@@ -453,6 +455,7 @@ def conv2d_fp8_dgrad_wt(
 ) -> torch.Tensor:
     """conv2d_fp8_dgrad_general on the transposed weight alone: [Cin, k, k, Cout] bytes."""
     assert dy.dtype == FP8_DTYPE and weight_t.dtype == FP8_DTYPE and weight_t.is_contiguous()
+    assert dy.is_cuda and weight_t.device == dy.device, f"{dy.device} {weight_t.device}"
     torch_checks_scale(dy_scale, dy.device)
     torch_checks_scale(weight_scale, dy.device)
     dy = _nhwc(dy)
@@ -460,6 +463,7 @@ def conv2d_fp8_dgrad_wt(
     cin, kh, kw, wcout = weight_t.shape
     assert wcout == cout and kh == kw
     height, width = input_hw
+    assert tuple(dy.shape[2:]) == _out_hw(height, width, kh, stride, padding)
     dx = torch.empty((batch, cin, height, width), device=dy.device, dtype=torch.bfloat16,
                      memory_format=torch.channels_last)
     geom = (batch, height, width, cin, cout, kh, kw, stride, padding)
@@ -546,9 +550,15 @@ def conv2d_fp8_fwd_frag(x: torch.Tensor, wf: torch.Tensor, x_scale: torch.Tensor
                         bias: torch.Tensor | None = None) -> torch.Tensor:
     """conv2d_fp8_fwd_wf for every frag_shape, on the tile that fills the GPU."""
     assert x.dtype == FP8_DTYPE and wf.dtype == torch.uint8 and wf.is_contiguous()
+    assert x.is_cuda and wf.device == x.device, f"{x.device} {wf.device}"
+    torch_checks_scale(x_scale, x.device)
+    torch_checks_scale(weight_scale, x.device)
     x = _nhwc(x)
     batch, cin, height, width = x.shape
     assert wf.numel() == cout * 9 * cin and frag_shape(batch, cin, cout, height, width)
+    if bias is not None:
+        assert bias.dtype == torch.float32 and bias.numel() == cout and bias.is_contiguous()
+        assert bias.device == x.device
     y = torch.empty((batch, cout, height, width), device=x.device, dtype=torch.bfloat16,
                     memory_format=torch.channels_last)
     _lib.call("dpa_conv2d_fwd_fp8_frag", x.data_ptr(), wf.data_ptr(), x_scale.data_ptr(),
@@ -561,6 +571,9 @@ def conv2d_fp8_dgrad_frag(dy: torch.Tensor, wf_dgrad: torch.Tensor, dy_scale: to
                           weight_scale: torch.Tensor, cin: int) -> torch.Tensor:
     """conv2d_fp8_dgrad_wf for every frag_shape, on the tile that fills the GPU."""
     assert dy.dtype == FP8_DTYPE and wf_dgrad.dtype == torch.uint8 and wf_dgrad.is_contiguous()
+    assert dy.is_cuda and wf_dgrad.device == dy.device, f"{dy.device} {wf_dgrad.device}"
+    torch_checks_scale(dy_scale, dy.device)
+    torch_checks_scale(weight_scale, dy.device)
     dy = _nhwc(dy)
     batch, cout, height, width = dy.shape
     assert wf_dgrad.numel() == cout * 9 * cin and frag_shape(batch, cin, cout, height, width)
@@ -1147,6 +1160,13 @@ class Conv2dFP8GeneralPrepared(torch.autograd.Function):
 
 def _linear_dgrad_wt(dy: torch.Tensor, wq_t: torch.Tensor, dy_scale, w_scale):
     """linear_fp8_dgrad_prequantized with the transposed weight [K][N] given."""
+    assert dy.dtype == FP8_DTYPE and wq_t.dtype == FP8_DTYPE and dy.ndim == wq_t.ndim == 2
+    assert dy.is_cuda and wq_t.device == dy.device, f"{dy.device} {wq_t.device}"
+    assert dy.shape[1] == wq_t.shape[1]
+    torch_checks_scale(dy_scale, dy.device)
+    torch_checks_scale(w_scale, dy.device)
+    dy = dy.contiguous()
+    wq_t = wq_t.contiguous()
     m, n = dy.shape
     k = wq_t.shape[0]
     dx = torch.empty((m, k), device=dy.device, dtype=torch.bfloat16)

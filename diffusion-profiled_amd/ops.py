@@ -146,8 +146,11 @@ def conv_fwd_prepared(x: torch.Tensor, weight: torch.Tensor, x_scale: torch.Tens
                       weight_scale: torch.Tensor, cout: int, stride: int,
                       padding: int) -> torch.Tensor:
     """conv_fwd with the weight as quantize_with_weight left it."""
+    assert weight.device == x.device, f"{x.device} {weight.device}"
     if weight.dtype == torch.uint8:
+        assert stride == 1 and padding == 1
         return K.conv2d_fp8_fwd_frag(x, weight, x_scale, weight_scale, cout)
+    assert weight.shape[0] == cout
     return K.conv2d_fp8_fwd_general(x, weight, x_scale, weight_scale, stride, padding)
 
 
@@ -165,7 +168,9 @@ def conv_dgrad_prepared(dy: torch.Tensor, weight_t: torch.Tensor, dy_scale: torc
                         stride: int, padding: int) -> torch.Tensor:
     """conv_dgrad with the weight's data-gradient copy of quantize_with_weight."""
     if weight_t.dtype == torch.uint8:
+        assert (k, stride, padding) == (3, 1, 1) and tuple(dy.shape[2:]) == (height, width)
         return K.conv2d_fp8_dgrad_frag(dy, weight_t, dy_scale, weight_scale, cin)
+    assert weight_t.shape[0] == cin and weight_t.shape[1] == k
     return K.conv2d_fp8_dgrad_wt(dy, weight_t, dy_scale, weight_scale, (height, width), stride,
                                  padding)
 

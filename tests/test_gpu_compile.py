@@ -161,6 +161,22 @@ def test_ops_are_registered_with_fakes():
         (torch.ops.dpa_fp8.gemm_wgrad.default, (aq, cq, as_, cs, False)),
         (torch.ops.dpa_fp8.linear_fp8.default, (a.float().requires_grad_(), b.float())),
     ]
+    # x and the weight quantized together, and the products on the weight's copies
+    for frag, stride in ((True, 1), (False, 2)):
+        qx, sx, qw, qt, sw = ops.quantize_with_weight(x, w, frag)
+        dy = ops.conv_fwd_prepared(qx, qw, sx, sw, 256, stride, 1)
+        qd, sd = ops.quantize(dy)
+        checks += [
+            (torch.ops.dpa_fp8.quantize_with_weight.default, (x, w, frag)),
+            (torch.ops.dpa_fp8.conv_fwd_prepared.default, (qx, qw, sx, sw, 256, stride, 1)),
+            (torch.ops.dpa_fp8.conv_dgrad_prepared.default,
+             (qd, qt, sd, sw, 128, 16, 16, 3, stride, 1)),
+        ]
+    _, _, _, bt, _ = ops.quantize_with_weight(a, b, False)
+    checks += [
+        (torch.ops.dpa_fp8.quantize_with_weight.default, (a, b.float(), False)),
+        (torch.ops.dpa_fp8.gemm_dgrad_wt.default, (cq, bt, cs, bs)),
+    ]
     for op, args in checks:
         # (test_schema is left out: it compares e4m3 tensors with arithmetic torch does not
         # implement for float8)
