@@ -15,6 +15,11 @@ import torch
 from . import build as _build
 
 
+# the handle alone: a torch.cuda.Stream object around it costs as much as a launch (None where
+# torch keeps it elsewhere)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 @torch.compiler.disable
 def _current_stream_untraced(t: "torch.Tensor") -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
@@ -26,10 +31,9 @@ def current_stream(t: "torch.Tensor") -> int:
     traces past it: under torch.compile a call here ends the graph and the ctypes launch that
     follows runs eagerly. The FP8 ops call it inside torch.library custom-op bodies, which
     Dynamo does not enter."""
-    if torch.compiler.is_compiling() or not t.is_cuda:     # (which refuses a CPU tensor)
-        return _current_stream_untraced(t)
-    # the handle alone: a torch.cuda.Stream object around it costs as much as a launch
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    if torch.compiler.is_compiling() or _raw_stream is None or not t.is_cuda:
+        return _current_stream_untraced(t)      # (which refuses a CPU tensor)
+    return _raw_stream(t.get_device())
 
 
 c_float_p = POINTER(c_float)

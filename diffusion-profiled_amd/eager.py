@@ -17,31 +17,51 @@ from typing import Any, Callable
 import torch
 from torch.autograd import forward_ad as _fwd_ad
 
-_Key, _KeySet = torch._C.DispatchKey, torch._C.DispatchKeySet
 _TYPES = (torch.Tensor, torch.nn.Parameter)
-# dispatch keys of an ordinary GPU tensor (an inference tensor has no autograd keys) ...
-_INFERENCE = _KeySet(_Key.CUDA).add(_Key.AutocastCUDA)
-_TENSOR_KEYS = frozenset((
-    _INFERENCE.raw_repr(), _INFERENCE.add(_Key.AutogradCUDA).add(_Key.ADInplaceOrView).raw_repr()))
-# ... and those that a thread adds to every call when no mode is active (in inference mode, and
-# otherwise): the Python modes, functorch's transforms, functionalization and tracing add theirs
-_THREAD_KEYS = frozenset((
-    _KeySet(_Key.BackendSelect).raw_repr(),
-    _KeySet(_Key.BackendSelect).add(_Key.ADInplaceOrView).raw_repr()))
+
+
+def _torch_state():
+    """What ``plain`` reads of torch, which has no public way to ask for it: (keys of a tensor,
+    keys that this thread adds to a call, function modes active, profiler active, forward-mode
+    level, the keys of an ordinary GPU tensor, those of a thread with no mode active)."""
+    key, key_set = torch._C.DispatchKey, torch._C.DispatchKeySet
+    # an ordinary GPU tensor (an inference tensor has no autograd keys) ...
+    inference = key_set(key.CUDA).add(key.AutocastCUDA)
+    tensor_keys = frozenset((
+        inference.raw_repr(), inference.add(key.AutogradCUDA).add(key.ADInplaceOrView).raw_repr()))
+    # ... and what a thread adds to every call when no mode is active (in inference mode, and
+    # otherwise): the Python modes, functorch's transforms, functionalization and tracing add theirs
+    thread_keys = frozenset((
+        key_set(key.BackendSelect).raw_repr(),
+        key_set(key.BackendSelect).add(key.ADInplaceOrView).raw_repr()))
+    state = (torch._C._dispatch_keys, torch._C._dispatch_tls_local_include_set,
+             torch._C._len_torch_function_stack, torch.autograd._profiler_enabled,
+             lambda: _fwd_ad._current_level, tensor_keys, thread_keys)
+    for read in (*state[1:5], lambda: state[0](torch.empty(0)).raw_repr(),
+                 lambda: state[1]().raw_repr()):
+        read()
+    return state
+
+
+try:
+    _STATE = _torch_state()
+except (AttributeError, TypeError, RuntimeError):   # a torch that keeps this elsewhere: every call takes the general route
+    _STATE = None
 
 
 def plain(*args) -> bool:
     """Whether a call on these arguments has nothing to record, trace, transform, wrap or
     profile: then the dispatcher would end in the op's body with the same arguments."""
-    if (torch.compiler.is_compiling() or torch.autograd._profiler_enabled()
-            or torch._C._len_torch_function_stack() != 0
-            or torch._C._dispatch_tls_local_include_set().raw_repr() not in _THREAD_KEYS):
+    if torch.compiler.is_compiling() or _STATE is None:
+        return False
+    keys_of, thread_keys_now, function_modes, profiling, _, tensor_keys, thread_keys = _STATE
+    if (profiling() or function_modes() != 0
+            or thread_keys_now().raw_repr() not in thread_keys):
         return False
     grad = torch.is_grad_enabled()
     for t in args:
         if type(t) in _TYPES:
-            if (torch._C._dispatch_keys(t).raw_repr() not in _TENSOR_KEYS
-                    or (grad and t.requires_grad)):
+            if keys_of(t).raw_repr() not in tensor_keys or (grad and t.requires_grad):
                 return False
         elif hasattr(type(t), "__torch_function__"):    # subclasses, proxies
             return False
@@ -83,8 +103,8 @@ def run_in(ctx, op, *args):
 
 def apply(function: type[torch.autograd.Function], *args):
     """``function.apply(*args)``; with gradients off its forward alone."""
-    if (torch.compiler.is_compiling() or torch.is_grad_enabled()
-            or _fwd_ad._current_level >= 0 or not plain(*args)):
+    if (torch.compiler.is_compiling() or torch.is_grad_enabled() or not plain(*args)
+            or _STATE[4]() >= 0):
         return function.apply(*args)
     out = function.forward(NoGraph(), *args)
     # (an input that comes back as an output is a view of it, as from apply)
