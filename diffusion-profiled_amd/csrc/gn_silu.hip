@@ -1244,6 +1244,14 @@ struct GnSlab {
   }
 };
 
+// Whether a lane's u-th pixel lies past the image in every lane (workgroup-uniform): its turn in
+// a pass is left out. All of them are loaded (the ones past the end load the last pixel again, from
+// the L1), so that every load is in flight before the first is waited for.
+template <int PLN>
+__device__ __forceinline__ bool res_past(const GnArgs& p, int u) {
+  return u > 0 && u * PLN >= p.HW;
+}
+
 // v unchanged, but opaque to the optimiser (no value numbering across this point)
 __device__ __forceinline__ void opaque_u4(uint4& v) {
   asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
@@ -1391,7 +1399,11 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
   uint4 mask[kEarly ? U : 1];
   if constexpr (kEarly) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) mask[u] = mask_of(u);
+    for (int u0 = 0; u0 < U; u0 += 4) {  // (four at a time, for the arithmetic in between)
+      if (U >= 16 && res_past<PLN>(p, u0)) continue;
+#pragma unroll
+      for (int u = u0; u < u0 + 4; ++u) mask[u] = mask_of(u);
+    }
     __builtin_amdgcn_sched_barrier(0);
   }
   float sm[2] = {0.f, 0.f};
@@ -1462,13 +1474,14 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
   asm volatile("" : "+v"(pl2));
 #pragma unroll
   for (int u = 0; u < U; ++u) {
+    if (U >= 16 && !kCat && res_past<PLN>(p, u)) continue;
     reopen(u);
-    float f[8];
-    unpack_x<kF32>(v, u, f);
     const int px = pl2 + u * PLN;
-    const uint4 o = fwd_out8<kDrop>(f, A, B, kEarly ? mask[kEarly ? u : 0] : mask_of(u),
-                                    p.drop_scale);
     if (px < p.HW) {
+      float f[8];
+      unpack_x<kF32>(v, u, f);
+      const uint4 o = fwd_out8<kDrop>(f, A, B, kEarly ? mask[kEarly ? u : 0] : mask_of(u),
+                                      p.drop_scale);
       if (p.q)
         qo.put(p, ((int64_t)n * p.HW + px) * p.C + ch, o);
       else
@@ -1531,6 +1544,7 @@ __global__ __launch_bounds__(NG * PLN) void gn_res_bwd_kernel(const GnArgs p) {
   v4f* gl = reinterpret_cast<v4f*>(gls) + threadIdx.x;  // pixel u < kGL: entries 2u, 2u + 1
 #pragma unroll
   for (int u = 0; u < U; ++u) {
+    if (!kCat && res_past<PLN>(p, u)) continue;
     float f[8], d[8], xh[8], g[8];
     unpack_x<kF32>(v, u, f);
     bwd_dout<kDrop>(v[in.kN - 1][u], z0 + (uint64_t)u * zs, p, d);
@@ -1715,6 +1729,7 @@ __global__ __launch_bounds__(NG * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     asm volatile("" : "+v"(pl2));
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      if (res_past<PLN>(p, u)) continue;
       float t[8];
       pixel_dx(u, t);
       auto dx = [&](int e) __attribute__((always_inline)) { return t[e]; };

@@ -594,3 +594,21 @@ def test_thin_resident_slabs_vs_single_images(G, n, c, groups, h, w, film, f32, 
         assert torch.equal(x16, x.to(torch.bfloat16))
         (qa, sa), (qb, sb) = K.quantize_fp8_from_producer(x16, x16), K.quantize_fp8(x16)
         assert torch.equal(sa, sb) and torch.equal(qa.view(torch.uint8), qb.view(torch.uint8))
+
+# images that fill their workgroup's pixels in part: one pixel, one more than a lane's first, half
+# and most of the room, at every pixel count per lane
+PART_CASES = [("bf16", 1, 128, 1, 1, True), ("bf16", 2, 256, 3, 11, False),
+              ("bf16", 1, 128, 3, 43, True), ("bf16", 2, 128, 1, 193, False),
+              ("bf16", 1, 128, 1, 257, True), ("bf16", 1, 128, 25, 40, False),
+              ("f32", 1, 128, 1, 257, False), ("f32", 1, 256, 31, 33, False),
+              ("f32", 2, 128, 3, 11, True), ("f32", 1, 128, 3, 43, False),
+              ("drop", 1, 128, 1, 257, False), ("drop", 1, 128, 3, 43, True),
+              ("drop", 1, 256, 25, 40, True), ("drop", 2, 128, 3, 11, False)]
+
+
+@pytest.mark.parametrize("kind,n,c,h,w,flag", PART_CASES, ids=str)
+def test_images_that_fill_their_workgroups_in_part(G, kind, n, c, h, w, flag):
+    """Pixels past the image are left out of every pass: the oracle's tests at such sizes."""
+    print("part", kind, n, c, h, w, flag, flush=True)
+    {"bf16": test_gn_silu_fwd_bwd_vs_oracle, "f32": test_gn_silu_fp32_input_vs_oracle,
+     "drop": test_gn_silu_film_dropout_vs_oracle}[kind](G, n, c, h, w, flag)
