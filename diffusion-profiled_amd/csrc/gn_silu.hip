@@ -1388,9 +1388,9 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
       if (p.xb_part) finish_xb_amax(p, xacc, qred, sl.blk());
     }
   }
-  // the dropout masks, hashed while the loads are in flight (beside 128 registers of fp32 x: at
-  // their use)
-  constexpr bool kEarly = kDrop && !(kF32 && U >= 16);
+  // the dropout masks, hashed while the loads are in flight (beside 128 registers of fp32 x, and
+  // at four pixels per lane, where they cost a wave per SIMD: at their use)
+  constexpr bool kEarly = kDrop && U >= 8 && !(kF32 && U >= 16);
   const uint64_t z0 = kDrop ? drop_z(seed, ((int64_t)n * p.HW + pl) * p.C + ch) : 0;
   const uint64_t zs = (uint64_t)(PLN * p.C / 4) * kDropGolden;  // per pixel of the lane
   auto mask_of = [&](int u) __attribute__((always_inline)) {
@@ -1497,11 +1497,13 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
 // and the dropout hash are its largest costs and run once. At 16 pixels per lane, whose x and
 // g take 192 registers (fp32 x: 256), the first few pixels' g lie in LDS. 128 images of 32x32 x
 // 128 bf16 with FiLM and dropout: 41.3 us with g formed in both passes and dout in LDS, 33.2 so.
+// At four pixels per lane many workgroups share a CU, so the bf16 form is held to four waves per
+// SIMD: 128 images of 4x4 x 512 with FiLM 15.2 us at three, 11.4 at four (with g formed twice 11.4).
 template <int U, bool kFilm, bool kF32, bool kCat>
 constexpr int kGnResLdsG = U < 16 ? 0 : (kF32 ? 9 : (kCat ? 8 : (kFilm ? 6 : 3)));
 
 template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8>
-__global__ __launch_bounds__(NG * PLN) void gn_res_bwd_kernel(const GnArgs p) {
+__global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_kernel(const GnArgs p) {
   static_assert(!kCat || (!kF32 && PLN == 64 && U == 16) || (kF32 && PLN == 32 && U == 8),
                 "32x32 images (bf16 sources) or 16x16 (cat_h bf16 or fp32)");
   constexpr int kGL = kGnResLdsG<U, kFilm, kF32, kCat>;
@@ -1567,9 +1569,13 @@ __global__ __launch_bounds__(NG * PLN) void gn_res_bwd_kernel(const GnArgs p) {
     // before the next pixel's are formed (else the interleaved pixels exceed the registers)
     __builtin_amdgcn_sched_barrier(0);
   }
-  const GnChan<kFilm, true> kc2(p, n, ch);  // (again, not kept across the pixels)
-  slab_reduce<16, PLN, NG>(acc, red);
-  gn_bwd_setup<kFilm>(p, kc2, st);
+  if constexpr (U >= 16) {
+    const GnChan<kFilm, true> kc2(p, n, ch);  // (again, not kept across the pixels)
+    slab_reduce<16, PLN, NG>(acc, red);
+    gn_bwd_setup<kFilm>(p, kc2, st);
+  } else {
+    slab_reduce<16, PLN, NG>(acc, red);
+  }
   if (pl == 0) {
     const int64_t nc = (int64_t)p.N * p.C;
     float h1[2] = {0.f, 0.f}, h2[2] = {0.f, 0.f};
