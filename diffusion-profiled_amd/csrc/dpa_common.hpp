@@ -353,6 +353,9 @@ inline int launch_status() {
   return e == hipSuccess ? DPA_OK : (int)e;
 }
 
+// CUs of the device (256 where there is none to ask)
+int num_cus();
+
 inline bool aligned(const void* p, uintptr_t a) { return ((uintptr_t)p % a) == 0; }
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -1570,8 +1570,16 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
 template <int U, bool kFilm, bool kF32, bool kCat>
 constexpr int kGnResLdsG = U < 16 ? 0 : (kF32 ? 9 : (kCat ? 8 : (kFilm ? 6 : 3)));
 
-template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8>
+//
+// kAgain (below 16 pixels per lane): g formed again in the second pass, for fp32 x of 8 pixels per
+// lane without FiLM and dropout where a CU holds several workgroups: what they load and store is
+// then the longer part, and a second pass with arithmetic between its stores the shorter whole
+// (images of 16x16, us, g kept / again: 128 x 256 channels 22.4 / 18.9, 64 x 512 22.6 / 21.1, 128 x
+// 512 36.8 / 35.0; 16 x 256, one workgroup per CU, 9.9 / 11.6).
+template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8,
+          bool kAgain = false>
 __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_kernel(const GnArgs p) {
+  static_assert(!kAgain || (U < 16 && !kCat), "g is kept");
   static_assert(!kCat || (!kF32 && PLN == 64 && U == 16) || (kF32 && PLN == 32 && U == 8),
                 "32x32 images (bf16 sources) or 16x16 (cat_h bf16 or fp32)");
   constexpr int kGL = kGnResLdsG<U, kFilm, kF32, kCat>;
@@ -1634,7 +1642,8 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
         acc[8 + e] += g[e] * xh[e];
       }
     }
-    if (u < kGL) {
+    if (kAgain) {
+    } else if (u < kGL) {
       gl[(2 * u) * NG * PLN] = v4f{g[0], g[1], g[2], g[3]};
       gl[(2 * u + 1) * NG * PLN] = v4f{g[4], g[5], g[6], g[7]};
     } else {
@@ -1695,14 +1704,19 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
   // across the reduction (8 registers per pixel more)
   auto pixel_dx = [&](int u, float (&t)[8]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int l = 0; l < in.kX; ++l) opaque_u4(v[l][u]);
-    float f[8];
+    for (int l = 0; l < (kAgain ? in.kN : in.kX); ++l) opaque_u4(v[l][u]);
+    float f[8], ga[8];
     unpack_x<kF32>(v, u, f);
+    if constexpr (kAgain) {
+      float d[8], xh[8];
+      bwd_dout<kDrop>(v[in.kN - 1][u], z0 + (uint64_t)u * zs, p, d);
+      bwd_terms<kFilm>(f, d, st, xh, ga);
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int h = e >> 2;
       const float xh = __builtin_fmaf(f[e], st.rs[h], st.nmr[h]);
-      const float g = u < kGL ? gl[(2 * u + h) * NG * PLN][e & 3] : gk[u][e];
+      const float g = kAgain ? ga[e] : u < kGL ? gl[(2 * u + h) * NG * PLN][e & 3] : gk[u][e];
       t[e] = st.rs[h] * __builtin_fmaf(-xh, m2[h], g * st.gC[e] - m1[h]);
     }
   };
@@ -2224,11 +2238,17 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
     dispatch3(film, x_f32, a.drop_seed != nullptr, [&](auto FILM, auto F32, auto DROP) {
       constexpr bool kF = decltype(FILM)::value, k3 = decltype(F32)::value,
                      kD = decltype(DROP)::value;
-      if (rs.u == 4)
+      if (rs.u == 4) {
         gn_res_bwd_kernel<32, 4, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
-      else if (rs.u == 8)
+      } else if (rs.u == 8) {
+        if constexpr (k3 && !kF && !kD) {
+          if ((int64_t)(C / kSlab) * N >= 2 * num_cus()) {
+            gn_res_bwd_kernel<32, 8, false, true, false, false, 8, true><<<rgrid, 8 * 32, 0, s>>>(a);
+            return;
+          }
+        }
         gn_res_bwd_kernel<32, 8, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
-      else if constexpr (!k3 || (!kF && !kD)) {  // (gn_res_bwd_ok)
+      } else if constexpr (!k3 || (!kF && !kD)) {  // (gn_res_bwd_ok)
         if (rs.ng == 8)
           gn_res_bwd_kernel<64, 16, kF, k3, kD><<<rgrid, 8 * 64, 0, s>>>(a);
         else if (rs.ng == 4)

@@ -630,7 +630,7 @@ __global__ __launch_bounds__(256) void igemm_split_reduce_kernel(const IgemmArgs
 
 static int g_num_cus = 0;
 
-static int num_cus() {
+int num_cus() {
   if (g_num_cus == 0) {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) == hipSuccess &&

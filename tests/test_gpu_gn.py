@@ -612,3 +612,25 @@ def test_images_that_fill_their_workgroups_in_part(G, kind, n, c, h, w, flag):
     print("part", kind, n, c, h, w, flag, flush=True)
     {"bf16": test_gn_silu_fwd_bwd_vs_oracle, "f32": test_gn_silu_fp32_input_vs_oracle,
      "drop": test_gn_silu_film_dropout_vs_oracle}[kind](G, n, c, h, w, flag)
+
+
+@pytest.mark.parametrize("h,w", [(16, 16), (12, 13)], ids=str)
+def test_fp32_backward_of_many_images_equals_few(G, h, w):
+    """Launches of two and more workgroups per CU form g twice instead of keeping it: the same
+    bits as in launches of fewer (129 to 256 pixels, fp32 x, no FiLM, no dropout)."""
+    n, c = 130, 256                                    # 520 workgroups, and 260 each half
+    g = torch.Generator(device="cuda").manual_seed(h)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x = (rnd(n, c, h, w) * 1.5 + 0.3).contiguous(memory_format=torch.channels_last)
+    dout = (rnd(n, c, h, w) * 1e-2).to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    gamma, beta = 1.0 + 0.3 * rnd(c), 0.3 * rnd(c)
+    _, mean, rstd = G.gn_silu_fwd(x, gamma, beta, GROUPS, 1e-5)
+    whole = G.gn_silu_bwd(x, dout, gamma, beta, mean, rstd, GROUPS)
+    halves = [G.gn_silu_bwd(x[s], dout[s], gamma, beta, mean.view(n, -1)[s].reshape(-1),
+                            rstd.view(n, -1)[s].reshape(-1), GROUPS)
+              for s in (slice(0, n // 2), slice(n // 2, n))]
+    assert torch.equal(whole[0], torch.cat([t[0] for t in halves]))
+    for k in (1, 2):
+        ref = halves[0][k].double() + halves[1][k].double()
+        # the sums over images in fp32, in slices of another length: 2^-20 of their size
+        assert float((whole[k].double() - ref).norm() / ref.norm()) < 2**-20
