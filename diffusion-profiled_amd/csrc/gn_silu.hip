@@ -54,7 +54,8 @@ struct GnArgs {
   const void* dx_add;  // bwd: a gradient added to dx (chunked and small forms), or null
   int dx_add_bf16;     // bwd: dx_add is bf16 while x and dx are fp32
   uint16_t* x_bf16;    // fwd: fp32 x also written as bf16 here (chunked and small forms), or null
-  uint32_t* xb_part;   // fwd: with x_bf16, one amax partial of its bf16 values per workgroup
+  uint32_t* xb_part;   // fwd: with x_bf16, one amax partial of its bf16 values per workgroup,
+  uint32_t xb_room;    //   and zeros in the rest of the room
   // Two-source x (a decoder stage's first GroupNorm with the upsample-and-concatenate before
   // it, diffusion/unet.py:379-382): channels [0, cat_ca) are the 2x nearest upsampling of
   // cat_a ([N][H/2][W/2][cat_ca], bf16), the others cat_h ([N][H][W][C - cat_ca], bf16 or
@@ -768,6 +769,9 @@ __device__ __forceinline__ uint4 store_x_bf16(const GnArgs& p, int64_t off, cons
 __device__ __forceinline__ void finish_xb_amax(const GnArgs& p, us2 acc, uint32_t* red,
                                                GnBlk b = GnBlk()) {
   store_amax_partial(acc, red, p.xb_part, nullptr, b.blk, b.count);
+  // (its reader takes the whole room, of which the thin slabs use a part)
+  if (threadIdx.x == 0)
+    for (uint32_t i = b.blk + b.count; i < p.xb_room; i += b.count) p.xb_part[i] = 0;
 }
 
 // The channel constants of this thread's 8 channels (gamma, beta, FiLM) and, for the backward,
@@ -1840,41 +1844,58 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
   if (p.q) qo.finish(p, qred, sl.blk());
 }
 
-// Resident-form geometry for an image of HW pixels: pixel lanes, pixels per lane and granules
-// of a slab, or zeros where none is taken. Above kResMaxHW pixels a slab has fewer channels,
-// which have to be whole groups, and a workgroup takes about 12 us (forward) and 19 us
-// (backward) however few there are, so the chunked form's two passes over memory stay the
-// better choice where the launch leaves half of the register room of its rounds unused; for
-// the forward on 16-channel slabs, whose one round ends with the SiLU's arithmetic and nothing
-// under it, an eighth. Forward / backward, us, chunked -> resident, bf16 unless said:
-//   32 images of 64x64 x 128 (all of the room)   21.3 / 42.6 -> 19.6 / 29.0 (fp32: 33.8 / 51.7
-//                                                -> 23.1 / 37.3)
-//   50 of 64x64 x 128 (two rounds, 78 %)         34.1 / 58.0 -> 26.1 / 47.4
-//   30 of 3000 pixels x 128 (69 %)               14.1 / 30.2 -> 15.2 / 25.0
-//   64 of 2048 pixels x 128                      17.8 / 39.0 -> 15.6 / 27.2
-//   40 of 36x36 x 256 (40 %)                     14.1 / 34.1 -> 18.6 / 35.8
-//   1 of 64x64 x 128                              9.6 / 12.4 -> 12.1 / 18.5
+// Resident-form geometry of a launch: pixels per lane and granules of a slab, or zeros where the
+// resident form is not taken. Above kResMaxHW pixels a slab has 32 channels (up to 2048 pixels) or
+// 16 (up to 4096), which have to be whole groups, and the chunked form is there too, whose time
+// grows with the bytes alone. A thin slab's workgroup takes about the same time however few there
+// are, so what decides is how full its rounds are: one workgroup per CU (two in the bf16 forward
+// without dropout, whose loads then run under the other's arithmetic, but not before both are
+// there). gn_thin_pays has the lines, each drawn so that no launch of 1025 to 4096 pixels at 128,
+// 256 or 512 channels takes more than a few hundredths above the chunked form's time, on one set of
+// buffers or on three in turn. us on three in turn, chunked -> resident, images of 128 channels:
+//   2048 pixels, FiLM and dropout, forward / backward: 128 slabs 14.9 / 24.1 -> 16.8 / 28.5, 192
+//     18.3 / 34.0 -> 17.6 / 30.2, 256 23.1 / 41.8 -> 19.9 / 35.5, 288 26.9 / 46.2 -> 33.1 / 59.2, 512
+//     42.4 / 76.0 -> 35.9 / 73.8
+//   4096 pixels: 256 slabs 21.3 / 41.1 -> 18.5 / 31.4 (with FiLM 23.2 / 37.7 -> 19.0 / 36.5, fp32 33.3 /
+//     54.6 -> 30.0 / 45.9), 288 25.5 / 44.8 -> 24.4 / 53.7, 512 40.4 / 74.9 -> 39.8 / 65.2 (with FiLM
+//     42.3 / 69.4 -> 40.4 / 74.2)
 struct GnRes {
-  int pln, u, ng;
+  int u, ng;
 };
-static GnRes gn_res_shape(int N, int HW, int C, int G, bool bwd) {
-  if (HW <= 128) return {32, 4, 8};
-  if (HW <= 256) return {32, 8, 8};
-  if (HW <= kResMaxHW) return {64, 16, 8};
-  const int ng = HW <= 2 * kResMaxHW ? 4 : 2;
-  if (HW > 4 * kResMaxHW || (8 * ng) % (C / G) != 0) return {0, 0, 0};
-  const int64_t slabs = (int64_t)(C / (8 * ng)) * N;
-  const int64_t room = ceil_div(slabs, 256) * 256 * (512 * 16 * 8);  // 512 threads of 16 pixels
-  const int64_t used = (int64_t)N * HW * C;
-  const bool strict = !bwd && ng == 2 && slabs <= 256;
-  if (strict ? 8 * used < 7 * room : 2 * used < room) return {0, 0, 0};
-  return {512 / ng, 16, ng};
+struct GnForm {
+  bool bwd, f32, film, drop;
+};
+static bool gn_thin_pays(int64_t slabs, int64_t per_image, int HW, const GnForm& f) {
+  const bool wide = HW <= 2 * kResMaxHW;
+  const int64_t cus = num_cus(), k = ceil_div(slabs, cus);
+  // share of the CUs that the last round of one workgroup per CU uses, in sixteenths
+  const int64_t last = 16 * (slabs - (k - 1) * cus) / cus;
+  if (f.bwd) {
+    if (f.f32) return last >= 12 && (wide || k == 1);
+    // (an image's lines in more than 16 pieces: 8 images of 64x64 x 512 40.9 -> 44.1 us)
+    if (f.film) return wide ? k <= 2 && last >= 12 : k == 1 && last >= 14 && per_image <= 16;
+    return k <= 2 && last >= 12;
+  }
+  // the fp32 forward's chunked form reads 8 B per element twice: its pixels count too
+  if (f.f32 && k == 1)
+    return last >= 12 && 16 * slabs * HW >= 9 * cus * (wide ? 2 : 4) * kResMaxHW;
+  if (f.f32) return k == 2 && wide && !f.drop && last >= 12;
+  if (!wide) return k == 1 && last >= 15 && HW >= 7 * kResMaxHW / 2;
+  if (f.drop) return k == 1 && last >= 12;
+  return k == 1 ? last >= 12 : (k > 2 || last >= 8);
 }
-// The backward with an fp32 x holds 2 x 16 B of x per pixel in registers: that fits at 16 pixels
-// per lane without FiLM and dropout (their per-channel terms and keep bits are the registers
-// that do not fit); with them, images above 256 pixels take the chunked form.
-static bool gn_res_bwd_ok(const GnRes& rs, bool x_f32, bool film, bool drop) {
-  return rs.ng > 0 && (!x_f32 || rs.u < 16 || (!film && !drop));
+static GnRes gn_res_shape(int N, int HW, int C, int G, const GnForm& f) {
+  // The backward with an fp32 x holds 2 x 16 B of x per pixel in registers: that fits at 16
+  // pixels per lane without FiLM and dropout (their per-channel terms and masks are the
+  // registers that do not fit); with them, images above 256 pixels take the chunked form.
+  if (HW > 256 && f.bwd && f.f32 && (f.film || f.drop)) return {0, 0};
+  if (HW <= 128) return {4, 8};
+  if (HW <= 256) return {8, 8};
+  if (HW <= kResMaxHW) return {16, 8};
+  const int ng = HW <= 2 * kResMaxHW ? 4 : 2;
+  if (HW > 4 * kResMaxHW || (8 * ng) % (C / G) != 0) return {0, 0};
+  const int64_t per_image = C / (8 * ng);
+  return gn_thin_pays(per_image * N, per_image, HW, f) ? GnRes{16, ng} : GnRes{0, 0};
 }
 
 static int gn_chunks(int HW) {
@@ -1928,14 +1949,14 @@ struct GnQOut {
   uint32_t* count;
 };
 
-// Workgroups of the launch that writes the output (one amax partial each), 0 for the form
-// without the fused cast (HW > 8192 pixels). The forward's; the backward never has more (it takes
-// the resident form wherever the forward does, and a slab is more than its chunks).
-static int64_t gn_q_blocks(int N, int HW, int C, int G) {
-  const GnRes rs = gn_res_shape(N, HW, C, G, false);
-  if (rs.ng > 0) return (int64_t)(C / (8 * rs.ng)) * N;
+// Room for the amax partials of the launch that writes the output, 0 for the form without the
+// fused cast (HW > 8192 pixels): one per workgroup of the resident form up to kResMaxHW pixels and
+// of the chunked form above, which has more of them than the thin slabs (HW / 128 chunks of 64
+// channels against two slabs of 32, or four of 16 above 2048 pixels).
+static int64_t gn_q_blocks(int N, int HW, int C) {
   const int nchunk = gn_chunks(HW);
-  return nchunk > 0 ? (int64_t)(C / kSlab) * N * nchunk : 0;
+  const int64_t slabs = (int64_t)(C / kSlab) * N;
+  return HW <= kResMaxHW ? slabs : slabs * nchunk;
 }
 
 // Launch grid of a resident kernel (GnSlab)
@@ -2001,7 +2022,8 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
   a.rstd = rstd;
   a.N = N; a.HW = HW; a.C = C; a.G = G; a.cpg = C / G; a.eps = eps;
   const int nchunk = gn_chunks(HW);
-  const GnRes rs = gn_res_shape(N, HW, C, G, false);
+  const GnRes rs = gn_res_shape(
+      N, HW, C, G, {false, x_f32, film_scale || film_wb, drop_seed != nullptr});
   const bool ws_ok = nchunk > 0 && workspace && workspace_bytes >= gn_fwd_workspace(N, HW, G) &&
                      aligned(workspace, 8);
   // (above kResMaxHW a call without the chunked form's workspace keeps its one-launch form)
@@ -2018,15 +2040,16 @@ static int gn_fwd(const void* x, const float* gamma, const float* beta, const fl
     // the chunked form's apply launch)
     if (!x_bf16) return DPA_ERR_NULL;
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    if (xb_part_cap < gn_q_blocks(N, HW, C, G)) return DPA_ERR_WORKSPACE;
+    if (xb_part_cap < gn_q_blocks(N, HW, C)) return DPA_ERR_WORKSPACE;
     if (!aligned(xb_part, 4)) return DPA_ERR_ALIGN;
     a.xb_part = xb_part;
+    a.xb_room = (uint32_t)gn_q_blocks(N, HW, C);
   }
   const int dst = gn_set_dropout(a, drop_seed, drop_p);
   if (dst != DPA_OK) return dst;
   if (qo) {
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C, G));
+    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C));
     if (qst != DPA_OK) return qst;
     a.out = qo->q;  // not written: the kernels store through a.q
   }
@@ -2196,12 +2219,11 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
   a.N = N; a.HW = HW; a.C = C; a.G = G; a.cpg = C / G; a.eps = 0.f;
   hipStream_t s = (hipStream_t)stream;
   const int nchunk = gn_chunks(HW);
-  const GnRes rs = gn_res_shape(N, HW, C, G, true);
+  const GnRes rs = gn_res_shape(
+      N, HW, C, G, {true, x_f32, film_scale || film_wb, drop_seed != nullptr});
   const bool ws_ok = nchunk > 0 && workspace_bytes >= gn_bwd_workspace(N, HW, C) &&
                      aligned(workspace, 16);
-  const bool resident =
-      gn_res_bwd_ok(rs, x_f32, film_scale || film_wb, drop_seed != nullptr) &&
-      (HW <= kResMaxHW || ws_ok);
+  const bool resident = rs.ng > 0 && (HW <= kResMaxHW || ws_ok);
   const bool chunked = !resident && ws_ok;
   if ((x_f32 || drop_seed || dx_add) && !chunked && !resident)
     return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
@@ -2213,7 +2235,7 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
   if (qo) {
     if (x_f32 || dx_add) return DPA_ERR_SHAPE;  // e4m3 of a bf16 dx, nothing added
     if (!chunked && !resident) return nchunk > 0 ? DPA_ERR_WORKSPACE : DPA_ERR_SHAPE;
-    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C, G));
+    const int qst = gn_set_q(a, qo, gn_q_blocks(N, HW, C));
     if (qst != DPA_OK) return qst;
   }
   const bool film = a.fs || a.wb;
@@ -2248,7 +2270,7 @@ static int gn_bwd(const void* x, const void* dout, const float* gamma, const flo
           }
         }
         gn_res_bwd_kernel<32, 8, kF, k3, kD><<<rgrid, 8 * 32, 0, s>>>(a);
-      } else if constexpr (!k3 || (!kF && !kD)) {  // (gn_res_bwd_ok)
+      } else if constexpr (!k3 || (!kF && !kD)) {  // (gn_res_shape)
         if (rs.ng == 8)
           gn_res_bwd_kernel<64, 16, kF, k3, kD><<<rgrid, 8 * 64, 0, s>>>(a);
         else if (rs.ng == 4)
@@ -2321,7 +2343,7 @@ extern "C" int dpa_gn_silu_bwd_ex(const void* x, int x_dtype, const void* dout, 
 
 extern "C" int dpa_gn_silu_fp8_partials(int N, int HW, int C, int G) {
   if (!gn_shape_ok(N, HW, C, G)) return 0;
-  const int64_t nb = gn_q_blocks(N, HW, C, G);
+  const int64_t nb = gn_q_blocks(N, HW, C);
   return nb <= INT32_MAX ? (int)nb : 0;
 }
 
@@ -2436,7 +2458,7 @@ extern "C" int dpa_upcat_gn_silu_fwd(const void* a, const void* h, int h_dtype, 
   g.rstd = rstd;
   g.x_bf16 = (uint16_t*)x_bf16;
   g.N = N; g.HW = HW; g.C = C; g.G = G; g.cpg = C / G; g.eps = eps;
-  const int64_t nblk = gn_q_blocks(N, HW, C, G);
+  const int64_t nblk = gn_q_blocks(N, HW, C);
   if (xb_partials) {
     if (xb_partials_cap < nblk) return DPA_ERR_WORKSPACE;
     g.xb_part = xb_partials;

@@ -374,8 +374,8 @@ int dpa_gn_silu_bwd_ex(const void* x, int x_dtype, const void* dout, const float
  * (bf16 entry, then the deferred cast). Arguments otherwise as dpa_gn_silu_fwd_ex /
  * dpa_gn_silu_bwd_ex; the backward takes bf16 x and no dx_add. The resident form (images of
  * up to 1024 pixels, one partial per (image, slab)) and the forms of larger images (up to
- * 8192 pixels with the workspace, one partial per 128-pixel chunk of each slab, or per slab
- * where the resident form runs) cast; larger
+ * 8192 pixels with the workspace: one partial per 128-pixel chunk of each slab, or, where the
+ * resident form runs, fewer) cast, and *q_count says how many partials they left; larger
  * images return DPA_ERR_SHAPE, a chunked-size image without the workspace
  * DPA_ERR_WORKSPACE. q_partials_cap < dpa_gn_silu_fp8_partials(...) returns
  * DPA_ERR_WORKSPACE. */
@@ -389,7 +389,8 @@ int dpa_gn_silu_fwd_fp8(const void* x, int x_dtype, const float* gamma, const fl
 
 /* dpa_gn_silu_fwd_ex / dpa_gn_silu_fwd_fp8 that also leave, with x_bf16 (fp32 x), one amax
  * partial of the bf16 copy of x per workgroup of the launch that writes it (u32 bf16
- * magnitude bits; count dpa_gn_silu_fp8_partials(N, HW, C, G)): the copy is the input of the
+ * magnitude bits; dpa_gn_silu_fp8_partials(N, HW, C, G) of them, zeros where the launch has
+ * fewer workgroups): the copy is the input of the
  * residual block's 1x1 skip conv (diffusion/unet.py:137-139, :161), which quantizes it with
  * current scaling, and dpa_quantize_fp8_bf16_from_partials takes these partials in place of
  * its amax pass (partial_amax_kernel, diffusion/fp8_kernels.py:54-64). Resident and chunked

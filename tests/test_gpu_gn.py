@@ -634,3 +634,103 @@ def test_fp32_backward_of_many_images_equals_few(G, h, w):
         ref = halves[0][k].double() + halves[1][k].double()
         # the sums over images in fp32, in slices of another length: 2^-20 of their size
         assert float((whole[k].double() - ref).norm() / ref.norm()) < 2**-20
+
+
+# (n, c, h, w, film, f32, p_drop, forward on thin slabs, backward on thin slabs): full and nearly
+# full rounds of workgroups take them, launches that leave a round mostly empty the chunked form
+THIN_LINES = [(32, 128, 64, 64, False, False, 0.0, True, True),
+              (36, 128, 64, 64, False, False, 0.0, False, False),
+              (64, 128, 64, 64, False, False, 0.0, False, True),
+              (64, 128, 64, 64, True, False, 0.0, False, False),
+              (8, 512, 64, 64, True, False, 0.2, True, False),
+              (32, 128, 33, 32, False, False, 0.0, False, False),
+              (48, 128, 33, 32, True, False, 0.0, True, True),
+              (72, 128, 33, 32, False, False, 0.0, False, False),
+              (96, 128, 33, 32, False, False, 0.0, True, False),
+              (144, 128, 33, 32, False, False, 0.0, True, False),
+              (112, 128, 33, 32, True, False, 0.2, False, True),
+              (16, 512, 33, 32, False, True, 0.0, False, None),
+              (16, 512, 36, 37, True, True, 0.2, True, None),
+              (32, 512, 33, 32, False, True, 0.0, True, None),
+              (32, 512, 33, 32, True, True, 0.2, False, None)]
+
+
+@pytest.mark.parametrize("n,c,h,w,film,f32,p_drop,fwd_thin,bwd_thin", THIN_LINES, ids=str)
+def test_thin_slab_lines_and_fused_casts(G, n, c, h, w, film, f32, p_drop, fwd_thin, bwd_thin):
+    """Which form a launch of 1025 to 4096 pixels takes (a launch that casts counts its
+    workgroups), and its casts: the e4m3 output and bf16 dx are the deferred casts of the plain
+    ones, with the same maximum over the partials counted and nothing written behind them, and the
+    partials of an fp32 x's bf16 copy fill their room, zeros where no workgroup wrote."""
+    print("lines", n, c, h, w, film, f32, p_drop, flush=True)
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines below are those of 256 CUs")
+    L, K = dpa_mod("_lib"), dpa_mod("fp8_kernels")
+    hw, st = h * w, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device="cuda").manual_seed(n + c + h)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    p = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    x = (rnd(n, c, h, w) * 1.5 + 0.3).contiguous(memory_format=torch.channels_last)
+    x = x if f32 else x.to(torch.bfloat16)
+    gamma, beta = 1.0 + 0.3 * rnd(c), 0.3 * rnd(c)
+    wb = (0.3 * rnd(n, 2 * c)).to(torch.bfloat16) if film else None
+    seed = torch.tensor([24681357], dtype=torch.int64, device="cuda") if p_drop else None
+    mean, rstd = torch.empty(n * GROUPS, device="cuda"), torch.empty(n * GROUPS, device="cuda")
+    slab = 32 if hw <= 2048 else 16
+    blocks = {True: n * c // slab, False: n * c // 64 * -(-hw // 128)}
+    room = L.query("dpa_gn_silu_fp8_partials", n, hw, c, GROUPS)
+    assert room == blocks[False]
+    poison = 0x7F7F7F7F
+
+    def hand():
+        return K.Fp8Handoff(torch.tensor(0.01, device="cuda"),
+                            torch.full((room + 64,), poison, device="cuda", dtype=torch.int32),
+                            torch.zeros(1, device="cuda", dtype=torch.int32))
+
+    def check_cast(hd, plain, thin):
+        count = int(hd.count)
+        assert count == blocks[thin]
+        assert bool((hd.partials[count:] == poison).all())
+        part = [torch.zeros(1 << 16, device="cuda", dtype=torch.int32),
+                torch.zeros(1, device="cuda", dtype=torch.int32)]
+        q = K.quantize_fp8_delayed_deferred(plain, hd.scale, *part)
+        assert torch.equal(hd.q.view(torch.uint8), q.view(torch.uint8))
+        assert int(hd.partials[:count].max()) == int(part[0][:int(part[1])].max())
+
+    out = torch.empty_like(x, dtype=torch.bfloat16)
+    ws_bytes = L.query("dpa_gn_silu_fwd_workspace_bytes", n, hw, c, GROUPS)
+    ws = torch.empty(ws_bytes, device="cuda", dtype=torch.uint8)
+    x16 = torch.empty_like(x, dtype=torch.bfloat16) if f32 else None
+    args = (x.data_ptr(), int(f32), gamma.data_ptr(), beta.data_ptr(), None, None, p(wb),
+            out.data_ptr(), mean.data_ptr(), rstd.data_ptr(), ws.data_ptr(), ws_bytes, n, hw, c,
+            GROUPS, 1e-5, p(seed), p_drop, p(x16))
+    if f32:
+        xbp = torch.full((room + 64,), poison, device="cuda", dtype=torch.int32)
+        L.call("dpa_gn_silu_fwd_ex_amax", *args, xbp.data_ptr(), room, st)
+        assert bool((xbp[room:] == poison).all()) and bool((xbp[blocks[fwd_thin]:room] == 0).all())
+        assert torch.equal(x16, x.to(torch.bfloat16))
+        assert int(xbp[:room].max()) == int(x16.abs().max().view(torch.int16))
+    else:
+        L.call("dpa_gn_silu_fwd_ex", *args, st)
+    fwd = hand()
+    G._fwd_fp8_call(x, gamma, beta, wb, fwd, mean, rstd, GROUPS, 1e-5, seed, p_drop)
+    check_cast(fwd, out, fwd_thin)
+    if f32:
+        return                                      # (the backward casts a bf16 dx)
+    dout = (rnd(n, c, h, w) * 1e-2).to(torch.bfloat16).contiguous(memory_format=torch.channels_last)
+    dx = torch.empty_like(x)
+    grads = [torch.empty(c, device="cuda") for _ in range(2)]
+    dwb = None if wb is None else torch.empty_like(wb)
+    ws_bytes = L.query("dpa_gn_silu_bwd_workspace_bytes", n, hw, c, GROUPS)
+    ws = torch.empty(ws_bytes, device="cuda", dtype=torch.uint8)
+    L.call("dpa_gn_silu_bwd_ex", x.data_ptr(), 0, dout.data_ptr(), gamma.data_ptr(), beta.data_ptr(),
+           None, None, p(wb), mean.data_ptr(), rstd.data_ptr(), dx.data_ptr(), None, 0,
+           grads[0].data_ptr(), grads[1].data_ptr(), None, None, p(dwb), ws.data_ptr(), ws_bytes,
+           n, hw, c, GROUPS, p(seed), p_drop, st)
+    bwd = hand()
+    bwd.q = torch.empty_like(x, dtype=torch.float8_e4m3fn)
+    L.call("dpa_gn_silu_bwd_fp8", x.data_ptr(), dout.data_ptr(), gamma.data_ptr(), beta.data_ptr(),
+           None, None, p(wb), mean.data_ptr(), rstd.data_ptr(), bwd.q.data_ptr(),
+           bwd.scale.data_ptr(), bwd.partials.data_ptr(), room, bwd.count.data_ptr(),
+           grads[0].data_ptr(), grads[1].data_ptr(), None, None, p(dwb), ws.data_ptr(), ws_bytes,
+           n, hw, c, GROUPS, p(seed), p_drop, st)
+    check_cast(bwd, dx, bwd_thin)
