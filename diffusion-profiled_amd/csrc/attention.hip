@@ -116,10 +116,9 @@ __device__ __forceinline__ uint2 att_pack4(float a, float b, float c, float d, u
 }
 
 // The workgroup's max of what it stored, for the consumer's current-scaling cast; every
-// thread calls it (uniform), NW waves.
+// thread calls it (uniform), NW waves; red: LDS room for NW numbers that nothing else uses.
 template <int NW>
-__device__ __forceinline__ void att_store_partial(us2 am, uint32_t* part) {
-  __shared__ uint32_t red[NW];
+__device__ __forceinline__ void att_store_partial(us2 am, uint32_t* part, uint32_t* red) {
   uint32_t m = am.x > am.y ? am.x : am.y;
   m = wave_max_u32(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -148,7 +147,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
   constexpr int NKB = LP / 16;    // key blocks
   __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t vs[LP * 64];
-  __shared__ __attribute__((aligned(1024))) uint16_t q1[64 * 64];  // the first block of each wave
+  // A head of up to 32 keys passes through registers, its first queries straight into them: there
+  // is little to start on before V is there (128 images of 8 heads of 16 tokens 3.8 us by DMA, 3.5
+  // so; of 64 tokens neither is the faster at every count: 4 heads 4.5 and 4.7, 8 heads 7.2 and
+  // 6.5). Above, the waves' first queries pass through q1. At LP = 128 the three arrays are 40 KB,
+  // four workgroups per CU.
+  constexpr bool kReg = LP <= 32;
+  __shared__ __attribute__((aligned(1024))) uint16_t q1[kReg ? 8 : 64 * 64];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -163,22 +168,48 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
 
   // the waves' first queries, K, then V (padded rows zero)
   constexpr int NF = LP * 8 / 256;  // transfers per wave of K, of V
+  uint4 qf0 = {0u, 0u, 0u, 0u}, qf1 = {0u, 0u, 0u, 0u};
+  if constexpr (kReg) {
+    uint4 kv[NF], vv[NF];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) att_dma(qg, S3, tid + 256 * r, L, LDS_ADDR(q1));
+    for (int r = 0; r < NF; ++r) {
+      const int c = tid + 256 * r, j = c >> 3, g = c & 7;
+      kv[r] = vv[r] = uint4{0u, 0u, 0u, 0u};
+      if (j < L) {
+        kv[r] = ld16(kg + j * S3 + 8 * g);
+        vv[r] = ld16(vg + j * S3 + 8 * g);
+      }
+    }
+    if (wave * 16 < L) {
+      const uint16_t* qr = qg + (wave * 16 + frow) * S3 + 8 * fq;
+      qf0 = ld16(qr);
+      qf1 = ld16(qr + 32);
+    }
 #pragma unroll
-  for (int r = 0; r < NF; ++r) att_dma(kg, S3, tid + 256 * r, L, LDS_ADDR(ks));
+    for (int r = 0; r < NF; ++r) {
+      const int c = tid + 256 * r, j = c >> 3, g = c & 7;
+      *reinterpret_cast<uint4*>(ks + att_off(j, g)) = kv[r];
+      *reinterpret_cast<uint4*>(vs + att_off(j, g)) = vv[r];
+    }
+    wait_lgkmcnt0();
+  } else {
 #pragma unroll
-  for (int r = 0; r < NF; ++r) att_dma(vg, S3, tid + 256 * r, L, LDS_ADDR(vs));
-  wait_vmcnt<NF>();  // queries and K
+    for (int r = 0; r < 2; ++r) att_dma(qg, S3, tid + 256 * r, L, LDS_ADDR(q1));
+#pragma unroll
+    for (int r = 0; r < NF; ++r) att_dma(kg, S3, tid + 256 * r, L, LDS_ADDR(ks));
+#pragma unroll
+    for (int r = 0; r < NF; ++r) att_dma(vg, S3, tid + 256 * r, L, LDS_ADDR(vs));
+    wait_vmcnt<NF>();  // queries and K
+  }
   lds_barrier();
-  uint4 qf0, qf1;
-  {
+  if constexpr (!kReg) {
     const int row = wave * 16 + frow;
     qf0 = ld16(q1 + att_off(row, fq));
     qf1 = ld16(q1 + att_off(row, 4 + fq));
   }
   // V complete; every wave passes this once
   auto wait_v = [&]() __attribute__((always_inline)) {
+    if (kReg) return;
     wait_vmcnt<0>();
     lds_barrier();
   };
@@ -257,7 +288,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
     qf1 = nq1;
   }
   if (wave * 16 >= L) wait_v();  // a wave without queries
-  if (p.amax_part) att_store_partial<4>(am, p.amax_part);
+  // (every wave is past its reads of q1)
+  if (p.amax_part) att_store_partial<4>(am, p.amax_part, reinterpret_cast<uint32_t*>(q1));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -285,13 +317,18 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   constexpr int NCH = LP * 8;            // 16-B chunks of a rows array
   constexpr int NF = (NCH + 511) / 512;  // its transfers per wave, and the parts
   constexpr int OB = NF < 3 ? NF : 3;    // O parts in flight (a fourth reuses the first's room)
+  // A head of up to 32 tokens has nothing to start on early: its rows pass through registers, where D is
+  // formed from them, and K's and V's fragments come from memory (128 images of 4 heads, us: 16
+  // tokens 4.6 by DMA, 4.4 so; 64 10.4 and 10.9)
+  constexpr bool kReg = LP <= 32;
   __shared__ __attribute__((aligned(1024))) uint16_t qs[LP * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t gs[LP * 64];
-  __shared__ __attribute__((aligned(1024))) uint16_t os[OB][64 * 64];
+  __shared__ __attribute__((aligned(1024))) uint16_t os[OB][kReg ? 8 : 64 * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t dsb[2][32 * TP];
   __shared__ __attribute__((aligned(256))) float lse_s[LP < 64 ? 64 : LP];
   __shared__ float dd_s[LP];
+  __shared__ uint32_t red[8];
   static_assert(2 * 32 * TP >= LP * 64, "V fits the dS buffers");
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -319,11 +356,49 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     // part r's 64 rows at os[r % OB]: as rows 0 .. 63 of its own array
     att_dma(og + (int64_t)64 * r * C, C, tid, L - 64 * r, LDS_ADDR(os[r % OB]));
   };
-  if (wave * 64 < LP) {
+  uint4 kf[KB][2], vf[KB][2];
+  if constexpr (kReg) {
+    // every load in flight before the first store
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const int key = kw0 + 16 * kb + frow;
+#pragma unroll
+      for (int hs = 0; hs < 2; ++hs) {
+        kf[kb][hs] = key < L ? ld16(kg + key * S3 + 32 * hs + 8 * fq) : uint4{0u, 0u, 0u, 0u};
+        vf[kb][hs] = key < L ? ld16(vg + key * S3 + 32 * hs + 8 * fq) : uint4{0u, 0u, 0u, 0u};
+      }
+    }
+    const float lse_t = tid < L ? p.lse[(int64_t)bh * L + tid] : __builtin_inff();
+    const int j = tid >> 3, g = tid & 7;
+    uint4 kv = {0u, 0u, 0u, 0u}, qv = kv, ov = kv, gv = kv;
+    if (j < L) {
+      kv = ld16(kg + j * S3 + 8 * g);
+      qv = ld16(qg + j * S3 + 8 * g);
+      ov = ld16(og + j * C + 8 * g);
+      gv = ld16(dg + j * C + 8 * g);
+    }
+    if (has) {
+      *reinterpret_cast<uint4*>(ks + att_off(j, g)) = kv;
+      *reinterpret_cast<uint4*>(qs + att_off(j, g)) = qv;
+      *reinterpret_cast<uint4*>(gs + att_off(j, g)) = gv;
+      float fo[8], fg[8];
+      unpack8_bf16(ov, fo);
+      unpack8_bf16(gv, fg);
+      float dot8 = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot8 += fo[e] * fg[e];
+      dot8 += __shfl_xor(dot8, 1, 64);
+      dot8 += __shfl_xor(dot8, 2, 64);
+      dot8 += __shfl_xor(dot8, 4, 64);
+      if (g == 0) dd_s[j] = dot8;
+    }
+    if (tid < LP) lse_s[tid] = lse_t;
+  }
+  if (!kReg && wave * 64 < LP) {
     const void* a = tid < L ? static_cast<const void*>(p.lse + (int64_t)bh * L + tid) : &att_inf;
     dma4_lds(a, LDS_ADDR(lse_s) + 256 * wave);
   }
-  if (has) {
+  if (!kReg && has) {
 #pragma unroll
     for (int r = 0; r < NF; ++r) att_dma(kg, S3, tid + 512 * r, L, LDS_ADDR(ks));
 #pragma unroll
@@ -357,9 +432,11 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     for (int kb = 0; kb < KB; ++kb) dvt[hb][kb] = dkt[hb][kb] = v4f{0.f, 0.f, 0.f, 0.f};
   // outstanding transfers after K, V and part 0: of parts 1 .. NF - 1
   constexpr int kLater = 2 * (NF - 1) + (OB - 1);
-  wait_vmcnt<kLater>();
-  asm volatile("" ::: "memory");  // (the DMAs' writes are invisible to the compiler)
-  form_d(0);
+  if constexpr (!kReg) {
+    wait_vmcnt<kLater>();
+    asm volatile("" ::: "memory");  // (the DMAs' writes are invisible to the compiler)
+    form_d(0);
+  }
   wait_lgkmcnt0();
   asm volatile("" ::: "memory");
   if (NF > OB && has) dma_o(OB);  // into os[0], whose chunks only their own wave read
@@ -367,24 +444,27 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
 
   // this wave's keys: B fragments of K and V (lane (key frow, k-slice fq): dims 8 fq .. + 7
   // of each 32-wide half)
-  uint4 kf[KB][2], vf[KB][2];
-  const uint16_t* vrow = &dsb[0][0];
+  if constexpr (!kReg) {
+    const uint16_t* vrow = &dsb[0][0];
 #pragma unroll
-  for (int kb = 0; kb < KB; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-    for (int hs = 0; hs < 2; ++hs) {
-      const int o = kact ? att_off(kw0 + 16 * kb + frow, 4 * hs + fq) : 0;
-      kf[kb][hs] = ld16(ks + o);
-      vf[kb][hs] = ld16(vrow + o);
-    }
+      for (int hs = 0; hs < 2; ++hs) {
+        const int o = kact ? att_off(kw0 + 16 * kb + frow, 4 * hs + fq) : 0;
+        kf[kb][hs] = ld16(ks + o);
+        vf[kb][hs] = ld16(vrow + o);
+      }
+  }
   // the K^T operand of this wave's dQ block (dims 16 (wave & 3) ..) over all keys: the same
   // for every query block, so read once
   uint4 ktf[LP / 32];
 #pragma unroll
   for (int kk = 0; kk < LP / 32; ++kk)
     ktf[kk] = frag_tr(ks, 32 * kk + 8 * fq, 32 * kk + 8 * fq + 4, wave & 3, frow);
-  wait_lgkmcnt0();
-  lds_barrier();  // V read: the dS buffers are free
+  if constexpr (!kReg) {
+    wait_lgkmcnt0();
+    lds_barrier();  // V read: the dS buffers are free
+  }
 
   // A fragments of a query block: rows q0 + 16 sub + frow of Q and dO (read one block ahead,
   // during the previous block's dQ products)
@@ -517,7 +597,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
       }
     }
   }
-  if (p.amax_part) att_store_partial<8>(am, p.amax_part);
+  if (p.amax_part) att_store_partial<8>(am, p.amax_part, red);
 }
 
 static int attn_lp(int L) {
