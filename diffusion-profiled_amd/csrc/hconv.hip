@@ -101,7 +101,10 @@ __device__ __forceinline__ v8i hc_gload2(const uint8_t* lo_src, const uint8_t* h
   return v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
 }
 
-template <bool WFRAG>
+// kRows: the tile is whole image rows (W = TC), so a tile's pixels are consecutive and a patch
+// slot's column is in the image or not for every tile (128 images of 32x32, us, checked per tile /
+// so: 128 -> 128 20.1 / 19.8, 256 -> 256 61.3 / 59.8, 512 -> 256 113.1 / 109.7).
+template <bool WFRAG, bool kRows>
 __global__ __launch_bounds__(kHcThreads, 1) void hconv_fp8_kernel(const HconvArgs p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -132,7 +135,7 @@ __global__ __launch_bounds__(kHcThreads, 1) void hconv_fp8_kernel(const HconvArg
     const int px = e / 9, g = e - px * 9;
     const int pr = px / p.PC;  // once per kernel: plain divisions are fine
     const int pc = px - pr * p.PC;
-    const int ok = (g < 8) & (px < patch_px);
+    const int ok = (g < 8) & (px < patch_px) & (!kRows | ((pc >= 1) & (pc <= p.W)));
     prw[d] = pr | (pc << 8) | (ok << 16);
     pxo[d] = ((pr - 1) * p.W + (pc - 1)) * p.C + g * 16;
   }
@@ -151,12 +154,12 @@ __global__ __launch_bounds__(kHcThreads, 1) void hconv_fp8_kernel(const HconvArg
     const int kc = gg - j * p.KC;
     const int tile = t_begin + j * p.wg_per_xcd;
     const int tm = (int)fdiv((uint32_t)tile, p.divTN);
-    const int ty = (int)fdiv((uint32_t)tm, p.divTX);
-    c.x0 = (tm - ty * p.tiles_x) * p.TC;
+    const int ty = kRows ? tm : (int)fdiv((uint32_t)tm, p.divTX);
+    c.x0 = kRows ? 0 : (tm - ty * p.tiles_x) * p.TC;
     c.n0 = (tile - tm * p.tiles_n) * kHcBN;
     const int row0 = ty * p.TR;  // global output row n * H + y0
     c.y0 = row0 - (int)fdiv((uint32_t)row0, p.divH) * p.H;
-    c.m0 = row0 * p.W + c.x0;
+    c.m0 = kRows ? tm * kHcBM : row0 * p.W + c.x0;
     c.pbase = c.m0 * p.C + kc * kHcBK;
     if (WFRAG)  // 2 KB block of (kc, tap 0, this wave's first 16 rows)
       c.wbase = ((kc * 9) * cb16 + (c.n0 >> 4) + wn * (kHcWN / 16)) * 2048 + lane * 16;
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(kHcThreads, 1) void hconv_fp8_kernel(const HconvArg
     const int y_ = (c).y0 + (prw[d] & 0xff) - 1;                                           \
     const int x_ = (c).x0 + ((prw[d] >> 8) & 0xff) - 1;                                    \
     const bool ok_ = (c).live & ((prw[d] >> 16) != 0) & ((unsigned)y_ < (unsigned)p.H) &   \
-                     ((unsigned)x_ < (unsigned)p.W);                                       \
+                     (kRows || (unsigned)x_ < (unsigned)p.W);                              \
     const uint8_t* src_ = ok_ ? p.act + (uint32_t)((c).pbase + pxo[d]) : hc_zero16;        \
     dst = *reinterpret_cast<const uint4*>(src_);                                           \
   }
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(kHcThreads, 1) void hconv_fp8_kernel(const HconvArg
       const int r = pf * 16 + (lane >> 2);
       const uint4 o = *reinterpret_cast<const uint4*>(slot + r * 64 + ((g_rd ^ ((r >> 2) & 3)) * 16));
       const int m = wm * kHcWM + r;
-      const int pix = m0 + (m >> p.tcshift) * p.W + (m & (p.TC - 1));
+      const int pix = kRows ? m0 + m : m0 + (m >> p.tcshift) * p.W + (m & (p.TC - 1));
       st_nt16(p.out + (uint32_t)(pix * p.Cout + n0 + wn * kHcWN + g_rd * 8), o);
     }
   };
@@ -589,7 +592,7 @@ __global__ __launch_bounds__(kHcThreads, 1) void hconv_small_kernel(const HconvA
 #undef HS_STORE_PATCH
 }
 
-// Fragment-native weight layout for hconv_fp8_kernel<true>: 2 KB blocks, block
+// Fragment-native weight layout for hconv_fp8_kernel<true, .>: 2 KB blocks, block
 // (kc * T + t) * (rows / 16) + rb holds, at byte half * 1024 + lane * 16 + b, row
 // 16 rb + (lane & 15), K byte 128 kc + 32 (lane >> 4) + 16 half + b of tap t. The forward
 // weight is read as [rows = Cout][T][K = Cin] (OHWI); the data gradient's as the transpose
@@ -678,10 +681,12 @@ static int hconv_launch(HconvArgs& a, int flip, int wfrag, int num_cus, hipStrea
   a.tcshift = a.TC == 32 ? 5 : 4;
   a.flip = flip;
   const int grid = hconv_grid(a, kHcBM, num_cus);
-  if (wfrag)
-    hconv_fp8_kernel<true><<<(unsigned)grid, kHcThreads, 0, s>>>(a);
+  if (!wfrag)  // (OHWI weights: whole rows, hconv_supported)
+    hconv_fp8_kernel<false, true><<<(unsigned)grid, kHcThreads, 0, s>>>(a);
+  else if (a.TC == a.W)
+    hconv_fp8_kernel<true, true><<<(unsigned)grid, kHcThreads, 0, s>>>(a);
   else
-    hconv_fp8_kernel<false><<<(unsigned)grid, kHcThreads, 0, s>>>(a);
+    hconv_fp8_kernel<true, false><<<(unsigned)grid, kHcThreads, 0, s>>>(a);
   return launch_status();
 }
 
