@@ -603,6 +603,24 @@ extern "C" int dpa_hcp_read(void* dst) {
 """
 
 
+def hconv_stamped_source(src: str) -> str:
+    """csrc/hconv.hip with the stamps in its 256-pixel kernel (the first there)."""
+    at = src.index("void hconv_fp8_kernel(")
+    end = src.index("\n}\n", at)
+    kernel = src[at:end]
+    for old, new, mode in _HCP_PATCHES:
+        if mode == "first":
+            continue
+        if kernel.count(old) != 1:
+            raise RuntimeError(f"hconv_fp8_kernel no longer has the marker {old.strip()[:50]!r}")
+        kernel = kernel.replace(old, new, 1)
+    head = src[:at]
+    for old, new, mode in _HCP_PATCHES:
+        if mode == "first":
+            head = head.replace(old, new, 1)
+    return head + kernel + src[end:] + _HCP_TAIL
+
+
 def hconv_phases_main(args):
     """cfg2 forward and data gradient through a stamped copy of the halo-patch conv, each
     graph-replayed; prints the launch time (HIP events) split into the workgroups' phases."""
@@ -613,12 +631,7 @@ def hconv_phases_main(args):
 
     B = importlib.import_module("diffusion-profiled_amd.build")
     K = importlib.import_module("diffusion-profiled_amd.fp8_kernels")
-    src = open(os.path.join(B.CSRC_DIR, "hconv.hip")).read()
-    for old, new, mode in _HCP_PATCHES:
-        if src.count(old) < 1 or (mode == "once" and src.count(old) != 1):
-            raise RuntimeError(f"hconv.hip no longer has the marker {old.strip()[:50]!r}")
-        src = src.replace(old, new, 1)
-    src += _HCP_TAIL
+    src = hconv_stamped_source(open(os.path.join(B.CSRC_DIR, "hconv.hip")).read())
     tmp = tempfile.mkdtemp(prefix="hcp_")
     gen, lib_path = os.path.join(tmp, "hconv_stamped.hip"), os.path.join(tmp, "libhcp.so")
     with open(gen, "w") as f:
