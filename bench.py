@@ -87,6 +87,13 @@ def seeded(shape, seed, std=1.0, kaiming=False):
     return (torch.randn(shape, generator=g) * std).to(torch.bfloat16)
 
 
+def library_kernels(n, h, w, cin, cout, k, stride, pad):
+    """(forward, data gradient, weight gradient) kernels of a conv into aligned outputs."""
+    lib = importlib.import_module("diffusion-profiled_amd._lib").load()
+    names = (lib.dpa_conv2d_kernel(p, 16, n, h, w, cin, cout, k, k, stride, pad) for p in range(3))
+    return tuple(v.decode() for v in names)
+
+
 class ConvWorkload:
     """One FP8 conv layer fwd + dgrad + wgrad with current scaling."""
 
@@ -168,19 +175,10 @@ class ConvWorkload:
         return 3 * self.flop
 
     def kernel_names(self):
-        """Kernels the library launches for this layer's GEMMs, following its dispatch
-        (csrc/igemm.hip use_hconv and onetap_ok, csrc/wgrad.hip use_hwgrad): 3x3 / stride-1 convs
-        of 16- or 32-wide images go to the halo-patch and three-tap kernels, 1x1 convs that reduce
-        over at most 512 channels to the one-tap kernel."""
-        s1 = self.k == 3 and self.stride == 1 and self.pad == 1 and self.w in (16, 32)
-        conv = "hconv_fp8_kernel" if (s1 and self.h % (256 // self.w) == 0) else "igemm_fp8_kernel"
-        if s1 and self.h % (128 // self.w) == 0 and self.cin % 64 == 0:
-            wg = f"hwgrad_partial_kernel<{self.w}>+wgrad_reduce_kernel"
-        else:
-            wg = "wgrad_partial_kernel+wgrad_reduce_kernel"
-        fwd, dgrad = ("onetap_fp8_kernel" if self.k == 1 and c <= 512 else conv
-                      for c in (self.cin, self.cout))
-        return {"fwd": fwd, "dgrad": dgrad, "wgrad": wg}
+        """Kernels that the library says it launches for this layer's GEMMs."""
+        fwd, dgrad, wg = library_kernels(self.n, self.h, self.w, self.cin, self.cout, self.k,
+                                         self.stride, self.pad)
+        return {"fwd": fwd, "dgrad": dgrad, "wgrad": wg + "+wgrad_reduce_kernel"}
 
     def config(self):
         return {
@@ -221,6 +219,9 @@ class GemmWorkload:
 
     def step_flop(self):
         return self.flop
+
+    def kernel_names(self):
+        return {"fwd": library_kernels(self.m, 1, 1, self.kk, self.nn, 1, 1, 0)[0]}
 
     def config(self):
         return {"workload": self.name, "m": self.m, "n": self.nn, "k": self.kk}
@@ -772,7 +773,7 @@ def main():
     tflops = wl.step_flop() / dt / 1e12
     # dominant kernel = the MFMA kernel with the most device time per step: the conv kernel
     # (one fwd and one dgrad launch) or the weight-gradient pair (partial + split reduce)
-    names = wl.kernel_names() if hasattr(wl, "kernel_names") else {"fwd": "onetap_fp8_kernel"}
+    names = wl.kernel_names()
     conv_launches = [parts[k] for k in ("fwd", "dgrad") if k in parts]
     if "wgrad" in parts and parts["wgrad"] > sum(conv_launches):
         dominant, dom_us, dom_bytes = names["wgrad"], parts["wgrad"], wl.bytes["wgrad"]

@@ -522,6 +522,16 @@ int hwgrad_splits(int N, int H, int W, int Cin, int Cout, int split_k) {
 
 // Launches the partial kernel; the caller has checked hwgrad_supported and the workspace
 // (splits x Cout x 9 x Cin fp32).
+// Name of the instance that hwgrad_partial_run launches.
+const char* hwgrad_name(int H, int W) {
+  const int tw = hwgrad_cols(W);
+  if (hwgrad_whole_rows(H, W))
+    return tw == 32 ? "hwgrad_partial_kernel<32, false>" : "hwgrad_partial_kernel<16, false>";
+  return tw == 32   ? "hwgrad_partial_kernel<32, true>"
+         : tw == 16 ? "hwgrad_partial_kernel<16, true>"
+                    : "hwgrad_partial_kernel<8, true>";
+}
+
 int hwgrad_partial_run(const void* xq, const void* dyq, float* partial, int N, int H, int W,
                        int Cin, int Cout, int splits, hipStream_t s) {
   HwgradArgs a{};

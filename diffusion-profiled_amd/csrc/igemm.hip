@@ -824,6 +824,9 @@ int hconv_frag_run(const void* act, const void* wf, const float* sa, const float
 int weight_frag_run(const void* w, void* out, int rows, int K, int T, int transpose,
                     hipStream_t s);
 
+// the weight gradient's kernel (wgrad.hip)
+const char* wgrad_name(int N, int H, int W, int Cin, int Cout, int R, int S, int stride, int pad);
+
 static bool use_hconv(int N, int H, int W, int C, int Cout, int R, int S, int stride, int pad) {
   return R == 3 && S == 3 && stride == 1 && pad == 1 && hconv_supported(N, H, W, C, Cout);
 }
@@ -990,8 +993,9 @@ extern "C" int dpa_conv2d_fwd_fp8(const void* xq, const void* wq, const float* x
 
 extern "C" const char* dpa_conv2d_kernel(int product, const void* out, int N, int H, int W, int Cin,
                                          int Cout, int R, int S, int stride, int pad) {
+  if (product == 2) return wgrad_name(N, H, W, Cin, Cout, R, S, stride, pad);
   const bool bwd = product == 1;
-  if (product < 0 || product > 1) return nullptr;
+  if (product < 0 || product > 2) return nullptr;
   if (!conv_shape_ok(N, H, W, bwd ? Cout : Cin, bwd ? Cin : Cout, R, S, stride, pad))
     return nullptr;
   if (use_hconv(N, H, W, bwd ? Cout : Cin, bwd ? Cin : Cout, R, S, stride, pad) &&

@@ -370,6 +370,7 @@ static WgradPlan plan_wgrad(int N, int H, int W, int Cin, int Cout, int R, int S
 // of large batches of images a multiple of 8 wide (hwgrad.hip); its partial tiles have the layout wgrad_reduce_kernel sums.
 bool hwgrad_supported(int N, int H, int W, int Cin, int Cout);
 int hwgrad_splits(int N, int H, int W, int Cin, int Cout, int split_k);
+const char* hwgrad_name(int H, int W);
 int hwgrad_partial_run(const void* xq, const void* dyq, float* partial, int N, int H, int W,
                        int Cin, int Cout, int splits, hipStream_t s);
 
@@ -383,6 +384,13 @@ static int wgrad_splits(int N, int H, int W, int Cin, int Cout, int R, int S, in
   if (use_hwgrad(N, H, W, Cin, Cout, R, S, stride, pad))
     return hwgrad_splits(N, H, W, Cin, Cout, split_k);
   return plan_wgrad(N, H, W, Cin, Cout, R, S, stride, pad, split_k).splits;
+}
+
+// dpa_conv2d_kernel's weight gradient (igemm.hip)
+const char* wgrad_name(int N, int H, int W, int Cin, int Cout, int R, int S, int stride, int pad) {
+  if (!wgrad_shape_ok(N, H, W, Cin, Cout, R, S, stride, pad)) return nullptr;
+  return use_hwgrad(N, H, W, Cin, Cout, R, S, stride, pad) ? hwgrad_name(H, W)
+                                                           : "wgrad_partial_kernel";
 }
 
 }  // namespace dpa

@@ -172,7 +172,8 @@ int dpa_conv2d_dgrad_fp8_frag(const void* dyq, const void* wf_dgrad, const float
 
 /* Name of the kernel that forms a product into out: product 0 = forward (dpa_conv2d_fwd_fp8 and
  * its _split form; a linear [M, K] x [N, K]^T is the 1x1 conv N = M, H = W = 1, Cin = K, Cout =
- * N), 1 = data gradient (dpa_conv2d_dgrad_fp8, _wt, _wt_split). Of out only the alignment counts,
+ * N), 1 = data gradient (dpa_conv2d_dgrad_fp8, _wt, _wt_split), 2 = weight gradient's partial
+ * sums (dpa_conv2d_wgrad_fp8; wgrad_reduce_kernel adds them up). Of out only the alignment counts,
  * nothing is launched. NULL: those entries refuse the shape. */
 const char* dpa_conv2d_kernel(int product, const void* out, int N, int H, int W, int Cin, int Cout,
                               int R, int S, int stride, int pad);

@@ -265,4 +265,4 @@ def test_wide_store_kernels_need_an_aligned_output(lib):
         assert kernel(0, out, 4096, 1, 1, 640, 768) == b"igemm_fp8_kernel"
         assert kernel(0, out, 4, 32, 32, 128, 128, 3, 2) == b"igemm_fp8_kernel"
         assert kernel(1, out, 4, 32, 32, 128, 128, 3, 2) == b"igemm_fp8_kernel"
-    assert kernel(0, 0x1000, 4, 32, 32, 96, 128) is None and kernel(2, 0x1000, 4, 1, 1, 128, 128) is None
+    assert kernel(0, 0x1000, 4, 32, 32, 96, 128) is None and kernel(3, 0x1000, 4, 1, 1, 128, 128) is None
