@@ -20,7 +20,7 @@ import torch
 from torch.amp.autocast_mode import custom_bwd, custom_fwd
 
 from . import _lib
-from .eager import apply, run, run_in
+from .eager import NoGraph, apply, run, run_in
 
 # diffusion/fp8_kernels.py:11-12
 FP8_DTYPE = torch.float8_e4m3fn
@@ -142,12 +142,14 @@ def _quantize_impl(tensor: torch.Tensor, prev_scale: torch.Tensor | None) -> tup
     return quantized, scale
 
 
-def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool):
+def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool,
+                               dgrad_copy: bool = True):
     """Both operands of one FP8 product in two launches (dpa_quantize_fp8_bf16_with_weight):
     (x e4m3, x scale, w e4m3, its data-gradient copy, w scale), the bytes and scales of
     quantize_fp8 of x and of the bf16 weight. weight: fp32 or bf16, [Cout, Cin, k, k] or [N, K].
     The weight's copies are the OHWI / [N][K] bytes and their [Cin][k][k][Cout] / [K][N]
-    transpose, or with ``frag`` the halo-patch conv's two fragment layouts (flat uint8)."""
+    transpose, or with ``frag`` the halo-patch conv's two fragment layouts (flat uint8). Without
+    ``dgrad_copy`` the data-gradient copy is not written and comes back empty."""
     assert x.dtype == torch.bfloat16, f"{x.dtype}"
     assert x.is_cuda and weight.device == x.device, f"{x.device} {weight.device}"
     assert weight.ndim in (2, 4) and (weight.ndim == 4 or not frag)
@@ -164,16 +166,18 @@ def _quantize_with_weight_impl(x: torch.Tensor, weight: torch.Tensor, frag: bool
     ws = torch.empty((), device=dev, dtype=torch.float32)
     if frag:
         wq = torch.empty(weight.numel(), device=dev, dtype=torch.uint8)
-        wt = torch.empty(weight.numel(), device=dev, dtype=torch.uint8)
+        wt = torch.empty(weight.numel() if dgrad_copy else 0, device=dev, dtype=torch.uint8)
     else:
         wq = torch.empty(weight.shape, device=dev, dtype=FP8_DTYPE, memory_format=(
             torch.channels_last if weight.ndim == 4 else torch.contiguous_format))
-        wt = torch.empty((cin, *weight.shape[2:], cout), device=dev, dtype=FP8_DTYPE)
+        wt = torch.empty((cin, *weight.shape[2:], cout) if dgrad_copy else 0, device=dev,
+                         dtype=FP8_DTYPE)
     ws_bytes = _lib.query("dpa_quantize_with_weight_workspace_bytes", cout, taps, cin)
     workspace = torch.empty(ws_bytes, device=dev, dtype=torch.uint8)
     flags = (1 if weight.dtype == torch.bfloat16 else 0) | (2 if frag else 0)   # DPA_WP_*
     _lib.call("dpa_quantize_fp8_bf16_with_weight", x.data_ptr(), n, xq.data_ptr(), xs.data_ptr(),
-              weight.data_ptr(), flags, cout, taps, cin, wq.data_ptr(), wt.data_ptr(),
+              weight.data_ptr(), flags, cout, taps, cin, wq.data_ptr(),
+              wt.data_ptr() if dgrad_copy else None,
               ws.data_ptr(), workspace.data_ptr(), ws_bytes, _stream(x))
     return xq, xs, wq, wt, ws
 
@@ -716,14 +720,15 @@ def conv2d_bwd_weight_fp8(x: torch.Tensor, dy: torch.Tensor) -> torch.Tensor:
 def _conv_current_fwd(ctx: Any, x: torch.Tensor, weight: torch.Tensor, stride: int,
                       padding: int) -> torch.Tensor:
     """Current-scaling conv forward of a bf16 channels-last x and an fp32 or bf16 weight, saving
-    e4m3 x and the weight's data-gradient copy."""
+    e4m3 x and the weight's data-gradient copy (which a forward that records nothing leaves out)."""
     assert x.dtype == torch.bfloat16 and x.is_cuda and x.ndim == 4, f"{x.dtype} {x.is_cuda} {x.ndim}"
     assert weight.device == x.device and weight.ndim == 4, f"{weight.device} {x.device} {weight.ndim}"
     batch, cin, height, width = x.shape
     cout, wcin, kh, kw = weight.shape
     assert wcin == cin and kh == kw
     frag = frag_shape(batch, cin, cout, height, width, kh, stride, padding)
-    x_fp8, x_scale, w_fp8, w_t, w_scale = run_in(ctx, _ops.quantize_with_weight, x, weight, frag)
+    x_fp8, x_scale, w_fp8, w_t, w_scale = run_in(ctx, _ops.quantize_with_weight, x, weight, frag,
+                                                 type(ctx) is not NoGraph)
     ctx.save_for_backward(x_fp8, w_t, x_scale, w_scale)
     ctx.geom = (cin, height, width, kh, stride, padding)
     ctx.dw_f32 = weight.dtype == torch.float32
@@ -1032,7 +1037,8 @@ class LinearFP8Function(torch.autograd.Function):
         assert x.shape[-1] == k
         x2 = x.to(torch.bfloat16).reshape(-1, k).contiguous()
         assert x2.is_cuda and weight.device == x2.device, f"{x2.device} {weight.device}"
-        xq, xs, wq, wt, wsc = run_in(ctx, _ops.quantize_with_weight, x2, weight, False)
+        xq, xs, wq, wt, wsc = run_in(ctx, _ops.quantize_with_weight, x2, weight, False,
+                                     type(ctx) is not NoGraph)
         b32 = None if bias is None else bias.detach().float().contiguous()
         y = run_in(ctx, _ops.gemm, xq, wq, xs, wsc, b32)
         ctx.save_for_backward(xq, wt, xs, wsc)

@@ -75,26 +75,28 @@ def _quantize_delayed_fake(tensor, prev_scale):
 
 
 @custom_op("dpa_fp8::quantize_with_weight")
-def quantize_with_weight(x: torch.Tensor, weight: torch.Tensor, frag: bool
+def quantize_with_weight(x: torch.Tensor, weight: torch.Tensor, frag: bool,
+                         dgrad_copy: bool = True
                          ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """(e4m3 x, x scale, e4m3 w, its data-gradient copy, w scale), the weight's copies in the
-    halo-patch conv's fragment layouts (flat uint8) with ``frag``."""
-    return K._quantize_with_weight_impl(x, weight, frag)
+    halo-patch conv's fragment layouts (flat uint8) with ``frag``; the data-gradient copy empty
+    without ``dgrad_copy``."""
+    return K._quantize_with_weight_impl(x, weight, frag, dgrad_copy)
 
 
 @quantize_with_weight.register_fake
-def _quantize_with_weight_fake(x, weight, frag):
+def _quantize_with_weight_fake(x, weight, frag, dgrad_copy=True):
     xq, xs = _quantize_fake(x)
     ws = x.new_empty((), dtype=torch.float32)
     if frag:
         wq = weight.new_empty((weight.numel(),), dtype=torch.uint8)
-        return xq, xs, wq, torch.empty_like(wq), ws
+        return xq, xs, wq, wq.new_empty(wq.numel() if dgrad_copy else 0), ws
     cout, cin = weight.shape[0], weight.shape[1]
     if weight.ndim == 4:
         wq = _empty_cl(weight.shape, weight.device, K.FP8_DTYPE)
     else:
         wq = weight.new_empty((cout, cin), dtype=K.FP8_DTYPE)
-    wt = weight.new_empty((cin, *weight.shape[2:], cout), dtype=K.FP8_DTYPE)
+    wt = weight.new_empty((cin, *weight.shape[2:], cout) if dgrad_copy else (0,), dtype=K.FP8_DTYPE)
     return xq, xs, wq, wt, ws
 
 

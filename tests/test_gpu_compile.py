@@ -175,6 +175,8 @@ def test_ops_are_registered_with_fakes():
     _, _, _, bt, _ = ops.quantize_with_weight(a, b, False)
     checks += [
         (torch.ops.dpa_fp8.quantize_with_weight.default, (a, b.float(), False)),
+        (torch.ops.dpa_fp8.quantize_with_weight.default, (a, b.float(), False, False)),
+        (torch.ops.dpa_fp8.quantize_with_weight.default, (x, w, True, False)),
         (torch.ops.dpa_fp8.gemm_dgrad_wt.default, (cq, bt, cs, bs)),
     ]
     for op, args in checks:

@@ -135,3 +135,36 @@ def test_a_strided_gradient_of_the_linear_is_made_dense(monkeypatch):
     dy, wt = wide[:, :256].as_subclass(_Cuda), tall.t().as_subclass(_Cuda)
     K._linear_dgrad_wt(dy, wt, one, one)
     assert len(seen) == 1 and seen[0][0] != wide.data_ptr() and seen[0][1] != tall.data_ptr()
+
+
+@pytest.mark.parametrize("frag", [True, False])
+def test_forwards_that_record_nothing_leave_the_data_gradient_copy_out(monkeypatch, frag):
+    """A forward called by ``eager.apply`` has no backward: the weight's second copy is neither
+    allocated nor written, while a recorded forward asks for it."""
+    class _Asked(Exception):
+        pass
+
+    def asked(ctx, op, *args):
+        raise _Asked(args[-1])
+    monkeypatch.setattr(K, "run_in", asked)
+    no_graph, recorded = dpa_mod("eager").NoGraph(), object()
+    with FakeTensorMode():
+        x, w = _bf16(2, 128, 8, 8), _bf16(128, 128, 3, 3)
+        for ctx, want in ((no_graph, False), (recorded, True)):
+            with pytest.raises(_Asked, match=str(want)):
+                K._conv_current_fwd(ctx, x, w, 1, 1)
+        with pytest.raises(_Asked, match="False"):
+            K.LinearFP8Function.forward(no_graph, x[:, :, 0, 0], w[:, :, 0, 0])
+
+    calls = []
+    monkeypatch.setattr(K, "_stream", lambda t: 0)
+    monkeypatch.setattr(K._lib, "call", lambda name, *a: calls.append(a))
+
+    class _Cuda(torch.Tensor):
+        is_cuda = True
+    x = torch.empty(16, 128, dtype=torch.bfloat16).as_subclass(_Cuda)
+    w = torch.empty((128, 128, 3, 3) if frag else (256, 128)).as_subclass(_Cuda)
+    for copy in (True, False):
+        wt = K._quantize_with_weight_impl(x, w, frag, copy)[3]
+        assert (wt.numel() == w.numel()) if copy else (wt.numel() == 0)
+        assert (calls[-1][10] is None) == (not copy)
