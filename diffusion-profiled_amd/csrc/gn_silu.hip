@@ -816,10 +816,10 @@ __device__ __forceinline__ void fwd_affine(const GnArgs& p, const GnChan<kFilm, 
   }
 }
 
-// The same constants through LDS, for the forward at 16 pixels per lane: its registers do not hold
-// them through two reductions. Every thread loads those of one channel before its pixels (threads
-// of equal channels the same values), put() stores them, and the affine reads 8 channels' back
-// after the reductions' barriers.
+// The same constants through LDS, for the bf16 forward at 16 pixels per lane without dropout: its
+// 128 registers do not hold them through two reductions. Every thread loads those of one channel
+// before its pixels (threads of equal channels the same values), put() stores them, and the affine
+// reads 8 channels' back after the reductions' barriers.
 template <bool kFilm, int NG>
 struct GnChanLds {
   static constexpr int kFloats = 8 * NG * (kFilm ? 4 : 2);
@@ -1302,8 +1302,9 @@ struct GnSlab {
 };
 
 // Whether a lane's u-th pixel lies past the image in every lane (workgroup-uniform): its turn in
-// a pass is left out. All of them are loaded (the ones past the end load the last pixel again, from
-// the L1), so that every load is in flight before the first is waited for.
+// a pass is left out (in the backward's first pass of 16 pixels per lane four at a time: a branch at
+// each costs a full image 2 % of the backward). All of them are loaded (the ones past the end load
+// the last pixel again, from the L1), so that every load is in flight before the first is waited for.
 template <int PLN>
 __device__ __forceinline__ bool res_past(const GnArgs& p, int u) {
   return u > 0 && u * PLN >= p.HW;
@@ -1411,7 +1412,7 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
   const int gq = threadIdx.x & (NG - 1);
   const int pl = threadIdx.x / NG;
   const int ch = sl.c0 + gq * 8;
-  constexpr bool kChanLds = U >= 16;
+  constexpr bool kChanLds = U >= 16 && !kF32 && !kDrop;  // (the instances held to 128 registers)
   using ChanLds = GnChanLds<kFilm, NG>;
   __shared__ __attribute__((aligned(16))) float chan[kChanLds ? ChanLds::kFloats : 4];
   using Chan = std::conditional_t<kChanLds, ChanLds, GnChan<kFilm, false>>;
@@ -1466,11 +1467,18 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
   };
   uint4 mask[kEarly ? U : 1];
   if constexpr (kEarly) {
+    // (straight through where most pixels are there: in pieces the hash takes 128 images of 32x32 x
+    // 128 from 18.3 us to 18.9; left out past the image it takes 16 of 20x20 x 256 from 11.2 to 9.5)
+    if (U < 16 || p.HW > 12 * PLN) {
 #pragma unroll
-    for (int u0 = 0; u0 < U; u0 += 4) {  // (four at a time, for the arithmetic in between)
-      if (U >= 16 && res_past<PLN>(p, u0)) continue;
+      for (int u = 0; u < U; ++u) mask[u] = mask_of(u);
+    } else {
 #pragma unroll
-      for (int u = u0; u < u0 + 4; ++u) mask[u] = mask_of(u);
+      for (int u0 = 0; u0 < 12; u0 += 4) {
+        if (res_past<PLN>(p, u0)) continue;
+#pragma unroll
+        for (int u = u0; u < u0 + 4; ++u) mask[kEarly && U >= 16 ? u : 0] = mask_of(u);
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -1605,6 +1613,7 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
   const GnChan<kFilm, true> kc(p, n, ch);
   GnQ qo(p);
   const GnSrc<kF32, true> in(p, base);
+  constexpr int kStep = U >= 16 ? 4 : 1;  // pixels per look at res_past
   // fp32 x and dout of 16 pixels are 192 registers: the last four pixels' dout is loaded as the
   // first pixels' dies, or the first pass spills
   constexpr int kLate = kF32 && U >= 16 ? 4 : 0;
@@ -1628,35 +1637,38 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
   float gk[U][8];
   v4f* gl = reinterpret_cast<v4f*>(gls) + threadIdx.x;  // pixel u < kGL: entries 2u, 2u + 1
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (u > 0 && u <= kLate) {
-      const int w = U - kLate + u - 1;
-      v[in.kN - 1][w] = *reinterpret_cast<const uint4*>(in.src[in.kN - 1] +
-                                                        (int64_t)pxs[w] * in.stride[in.kN - 1]);
-    }
-    if (!kCat && res_past<PLN>(p, u)) continue;
-    float f[8], d[8], xh[8], g[8];
-    unpack_x<kF32>(v, u, f);
-    bwd_dout<kDrop>(v[in.kN - 1][u], z0 + (uint64_t)u * zs, p, d);
-    bwd_terms<kFilm>(f, d, st, xh, g);
-    if (ok[u]) {
+  for (int u0 = 0; u0 < U; u0 += kStep) {
+    if (!kCat && res_past<PLN>(p, u0)) continue;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        acc[e] += g[e];
-        acc[8 + e] += g[e] * xh[e];
+    for (int u = u0; u < u0 + kStep; ++u) {
+      if (u > 0 && u <= kLate) {
+        const int w = U - kLate + u - 1;
+        v[in.kN - 1][w] = *reinterpret_cast<const uint4*>(in.src[in.kN - 1] +
+                                                          (int64_t)pxs[w] * in.stride[in.kN - 1]);
       }
-    }
-    if (kAgain) {
-    } else if (u < kGL) {
-      gl[(2 * u) * NG * PLN] = v4f{g[0], g[1], g[2], g[3]};
-      gl[(2 * u + 1) * NG * PLN] = v4f{g[4], g[5], g[6], g[7]};
-    } else {
+      float f[8], d[8], xh[8], g[8];
+      unpack_x<kF32>(v, u, f);
+      bwd_dout<kDrop>(v[in.kN - 1][u], z0 + (uint64_t)u * zs, p, d);
+      bwd_terms<kFilm>(f, d, st, xh, g);
+      if (ok[u]) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) gk[u][e] = g[e];
+        for (int e = 0; e < 8; ++e) {
+          acc[e] += g[e];
+          acc[8 + e] += g[e] * xh[e];
+        }
+      }
+      if (kAgain) {
+      } else if (u < kGL) {
+        gl[(2 * u) * NG * PLN] = v4f{g[0], g[1], g[2], g[3]};
+        gl[(2 * u + 1) * NG * PLN] = v4f{g[4], g[5], g[6], g[7]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) gk[u][e] = g[e];
+      }
+      // one pixel at a time: the packed inputs stay resident, each pixel's unpacked terms die
+      // before the next pixel's are formed (else the interleaved pixels exceed the registers)
+      __builtin_amdgcn_sched_barrier(0);
     }
-    // one pixel at a time: the packed inputs stay resident, each pixel's unpacked terms die
-    // before the next pixel's are formed (else the interleaved pixels exceed the registers)
-    __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (U >= 16) {
     const GnChan<kFilm, true> kc2(p, n, ch);  // (again, not kept across the pixels)
