@@ -298,8 +298,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
 // start: K and V, then Q, dO and O in parts of 64 rows. The first query blocks run on the first
 // part while the others are on their way; part r is awaited, and its D formed, in block 2 r - 1.
 // (V passes through the dS buffers on its way to registers.) Wave w owns KB key blocks (keys
-// kw0 = 16 KB w ..) and keeps their K and V rows as B fragments and the dK^T, dV^T accumulators in registers;
-// query blocks of 32 rows stream through:
+// kw0 = 16 KB w ..) and keeps their K and V rows as B fragments and the dK^T, dV^T accumulators
+// in registers; query blocks of 32 rows stream through:
 //   S = Q K^T and dP = dO V^T (A = Q / dO rows from LDS) in the layout lane (frow, fq) <->
 //   (query 16 sub + 4 fq + t, key frow);  P = 2^(S log2(e)/8 - lse), dS = P (dP - D);
 //   dV^T += dO^T P and dK^T += Q^T dS: B = P / dS straight from those registers (the k-slice
@@ -317,9 +317,9 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   constexpr int NCH = LP * 8;            // 16-B chunks of a rows array
   constexpr int NF = (NCH + 511) / 512;  // its transfers per wave, and the parts
   constexpr int OB = NF < 3 ? NF : 3;    // O parts in flight (a fourth reuses the first's room)
-  // A head of up to 32 tokens has nothing to start on early: its rows pass through registers, where D is
-  // formed from them, and K's and V's fragments come from memory (128 images of 4 heads, us: 16
-  // tokens 4.6 by DMA, 4.4 so; 64 10.4 and 10.9)
+  // A head of up to 32 tokens has nothing to start on early: its rows pass through registers, where
+  // D is formed from them, and K's and V's fragments come from memory (128 images of 4 heads, us:
+  // 16 tokens 4.6 by DMA, 4.4 so; 64 10.4 and 10.9)
   constexpr bool kReg = LP <= 32;
   __shared__ __attribute__((aligned(1024))) uint16_t qs[LP * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];

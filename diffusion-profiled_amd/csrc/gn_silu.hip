@@ -1264,9 +1264,10 @@ __global__ __launch_bounds__(8 * kChPLN) void gn_chunk_bwd_apply_kernel(const Gn
 }
 
 // ---- resident form (HW <= kResMaxHW: the 32x32, 16x16, 8x8 and 4x4 levels; up to four times
-// that on slabs of NG = 4 or 2 granules, see gn_res_shape): one workgroup per (image, slab) of
-// PLN pixel lanes x NG granules holds all of the slab's pixels in registers (U per lane, packed as loaded), so the forward and the backward each read their
-// inputs once and write their outputs once; every pass unpacks from those registers ----
+// that on slabs of NG = 4 or 2 granules in the launches that gn_res_shape names): one workgroup
+// per (image, slab) of PLN pixel lanes x NG granules holds all of the slab's pixels in registers
+// (U per lane, packed as loaded), so the forward and the backward each read their inputs once and
+// write their outputs once; every pass unpacks from those registers ----
 constexpr int kResMaxHW = 1024;
 
 // A workgroup's image and slab of 8 NG channels. 64-channel slabs: grid (C / 64, N). Thinner ones
@@ -1398,7 +1399,7 @@ __device__ __forceinline__ void cat_load(const GnArgs& p, int n, int ch, int pl,
 // the end, so that at 16 pixels per lane of bf16 x two workgroups fit a CU (128 registers) and
 // one's loads run under the other's arithmetic: the two-source form at 32x32 x 512 (2048
 // workgroups) 111 -> 94 us. With dropout the masks hashed under the loads take that room instead
-// (256 workgroups: 22.4 us with two per CU and the hash at the end, 20.4 so).
+// (256 workgroups 18.4 us; with two per CU and the hash at the end a tenth more).
 template <int PLN, int U, bool kFilm, bool kF32, bool kDrop, bool kCat = false, int NG = 8>
 __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void gn_res_fwd_kernel(const GnArgs p) {
   static_assert(!kCat || NG == 8, "64-channel slabs");
@@ -1576,7 +1577,7 @@ __global__ __launch_bounds__(NG * PLN, U >= 16 && !kF32 && !kDrop ? 4 : 1) void 
 // pass as the loads arrive: the sigmoid's exp2 and reciprocal, which issue at a quarter rate,
 // and the dropout hash are its largest costs and run once. At 16 pixels per lane, whose x and
 // g take 192 registers (fp32 x: 256), the first few pixels' g lie in LDS. 128 images of 32x32 x
-// 128 bf16 with FiLM and dropout: 41.3 us with g formed in both passes and dout in LDS, 33.2 so.
+// 128 bf16 with FiLM and dropout: 41.2 us with g formed in both passes and dout in LDS, 30.1 so.
 // At four pixels per lane many workgroups share a CU, so the bf16 form is held to four waves per
 // SIMD: 128 images of 4x4 x 512 with FiLM 15.2 us at three, 11.4 at four (with g formed twice 11.4).
 template <int U, bool kFilm, bool kF32, bool kCat>
@@ -1744,7 +1745,7 @@ __global__ __launch_bounds__(NG * PLN, U == 4 && !kF32 ? 4 : 1) void gn_res_bwd_
     // images are PLN / 2 wide, so pixel pl + PLN u is row 2u + pl / kW, column pl mod kW:
     // window (u, j) holds lanes 2j, 2j + 1 (row 2u) and 2j + kW, 2j + kW + 1 (row 2u + 1). The
     // odd lane's value comes by a shuffle (8 threads on), the lower row's two through LDS
-    // (an exchange buffer), four pixels per exchange.
+    // (an exchange buffer), kXR pixels per exchange.
     constexpr int kW = PLN / 2;
     constexpr int kEnt = (kW / 2) * 8 * 16;  // floats per pixel row pair: (window, granule) x 16
     const bool in_a = ch < p.cat_ca;  // workgroup-uniform

@@ -6,8 +6,8 @@
 //
 // The nine taps of a 3x3 conv read the same input pixels shifted by (dy, dx). An output tile
 // of 256 pixels is TR x TC = 8 x 32 or 16 x 16 pixels of one image, so its input is one
-// (TR + 2) x (TC + 2) pixel patch. Per 128-channel chunk the patch goes into LDS once and the nine K-steps (one
-// per tap) read their pixel fragments from it at offset dy * (W + 2) + dx.
+// (TR + 2) x (TC + 2) pixel patch. Per 128-channel chunk the patch goes into LDS once and the nine
+// K-steps (one per tap) read their pixel fragments from it at offset dy * (TC + 2) + dx.
 //
 // Schedule: persistent, one workgroup of 8 waves per CU, XCD-aware contiguous tile ranges;
 // K-steps are (chunk, tap) with taps inner. Workgroup tile 256 pixels x 128 channels; each
@@ -27,8 +27,9 @@
 // cfg2 launch), which the op-level entry without a weight preparation still accepts.
 // Epilogue: the wave's accumulators go through its 8 KB LDS slot and leave as 16-B
 // nontemporal stores of 64-B channel runs (8-B stores straight from the accumulators,
-// nontemporal or not, were 9-17 us slower per launch; plain 16-B stores 2 us slower). The data gradient is the same kernel
-// on dy with the transposed weight and the taps mirrored (baked into its fragment layout).
+// nontemporal or not, were 9-17 us slower per launch; plain 16-B stores 2 us slower). The data
+// gradient is the same kernel on dy with the transposed weight and the taps mirrored (baked into
+// its fragment layout).
 #include "dpa_common.hpp"
 
 #include <type_traits>
@@ -37,7 +38,7 @@ namespace dpa {
 
 constexpr int kHcThreads = 512;
 constexpr int kHcWaves = kHcThreads / 64;
-constexpr int kHcBM = 256;  // output pixels per tile (TR whole rows)
+constexpr int kHcBM = 256;  // output pixels per tile (a patch of TR rows x TC columns)
 constexpr int kHcBN = 128;  // output channels per tile
 constexpr int kHcBK = 128;  // K bytes per step (MFMA depth)
 constexpr int kHcWM = 128;  // pixels per wave

@@ -682,10 +682,13 @@ static int64_t igemm_workspace(IgemmArgs& a) {
   return bytes;
 }
 
-// Launches of onetap_fp8_kernel: with K <= 256 of any size, with 384 and 512 those whose tiles
-// reach a quarter of the CUs (below, 64 x 32 tiles of the general kernel load fewer weights per
-// workgroup: 128 x 512 -> 512 4.9 us there, 5.1 here; 4096 x 512 -> 128, 64 tiles, 5.5 and 5.4;
-// 10001 x 128 -> 128 5.3 and 3.5). K > 512 would not leave registers for the weights.
+// Launches of onetap_fp8_kernel: with K <= 256 of any size (general kernel / here, us: one row x
+// 128 -> 128 3.4 / 3.0, 64 x 256 -> 768 4.1 / 3.7, 512 x 256 -> 2048 5.7 / 4.1; over 1 to 8192 rows
+// and 128 to 2048 channels 0.63 to 0.97 of the general kernel's time), with 384 and 512 those whose
+// tiles reach a quarter of the CUs (below, 64 x 32 tiles of the general kernel load fewer weights
+// per workgroup: 128 x 512 -> 512 4.9 us there, 5.1 here; 4096 x 512 -> 128, 64 tiles, 5.5 and 5.4).
+// K > 512 would not fit the LDS as it is: two 64-pixel stages at K = 768 and the output block are
+// 112 KB, one workgroup per CU, and the next tile's loads would not run under another's stores.
 static bool onetap_ok(const IgemmArgs& a) {
   if (a.iy_step != 1 || a.ix_step != 1 || a.oy_step != 1 || a.ox_step != 1) return false;
   return a.nk <= 2 || (a.nk <= 4 && ceil_div(a.M, kOtBM) * a.tiles_n * 4 >= num_cus());

@@ -367,7 +367,8 @@ static WgradPlan plan_wgrad(int N, int H, int W, int Cin, int Cout, int R, int S
 }
 
 // Three-tap kernel for 3x3 / stride-1 / pad-1 convolutions of 16- and 32-pixel-wide images and
-// of large batches of images a multiple of 8 wide (hwgrad.hip); its partial tiles have the layout wgrad_reduce_kernel sums.
+// of large batches of images a multiple of 8 wide (hwgrad.hip); its partial tiles have the layout
+// wgrad_reduce_kernel sums.
 bool hwgrad_supported(int N, int H, int W, int Cin, int Cout);
 int hwgrad_splits(int N, int H, int W, int Cin, int Cout, int split_k);
 const char* hwgrad_name(int H, int W);
