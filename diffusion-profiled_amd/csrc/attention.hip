@@ -68,15 +68,31 @@ __device__ __forceinline__ uint2 ld_tr16(const uint16_t* p) {
 // At B = 128, 4 heads, L = 256 (512 workgroups, 268 MB forward and backward), against 144-B
 // rows staged through registers with the whole head awaited before the first product: forward
 // and backward 83.8 -> 80.0 us; both wait for their rows first and then for LDS and latency.
-__device__ __forceinline__ int att_off(int row, int g) { return row * 64 + ((g ^ (row & 7)) << 3); }
+//
+// kReg: rows that come through registers, of heads of up to 64 tokens, keep a pitch of 144 B
+// instead: as free of conflicts, and a fragment's rows are one address and constant offsets (62
+// registers instead of 73 in the forward of 64 tokens).
+template <bool kReg>
+constexpr int kAttPitch = kReg ? 72 : 64;
+template <bool kReg>
+__device__ __forceinline__ int att_off(int row, int g) {
+  return kReg ? row * kAttPitch<true> + g * 8 : row * 64 + ((g ^ (row & 7)) << 3);
+}
 
 // A fragment (rows = dims 16 hb + frow, k-slice fq) of the transpose of such an array x, k
 // running over x's rows: elements 0-3 = x[r1 + t][16 hb + frow] and 4-7 = x[r2 + t][16 hb +
 // frow], t = 0..3 (r1, r2: this lane group's first rows, multiples of 4).
+template <bool kReg>
 __device__ __forceinline__ uint4 frag_tr(const uint16_t* x, int r1, int r2, int hb, int frow) {
+  if constexpr (kReg) {
+    const int off = (frow >> 2) * kAttPitch<true> + 16 * hb + 4 * (frow & 3);
+    const uint2 lo = ld_tr16(x + r1 * kAttPitch<true> + off);
+    const uint2 hi = ld_tr16(x + r2 * kAttPitch<true> + off);
+    return uint4{lo.x, lo.y, hi.x, hi.y};
+  }
   const int rr = frow >> 2, g = 2 * hb + ((frow & 3) >> 1), half = 4 * (frow & 1);
-  const uint2 lo = ld_tr16(x + att_off(r1 + rr, g) + half);
-  const uint2 hi = ld_tr16(x + att_off(r2 + rr, g) + half);
+  const uint2 lo = ld_tr16(x + att_off<false>(r1 + rr, g) + half);
+  const uint2 hi = ld_tr16(x + att_off<false>(r2 + rr, g) + half);
   return uint4{lo.x, lo.y, hi.x, hi.y};
 }
 
@@ -145,14 +161,15 @@ __device__ __forceinline__ void att_store_partial(us2 am, uint32_t* part, uint32
 template <int LP>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
   constexpr int NKB = LP / 16;    // key blocks
-  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
-  __shared__ __attribute__((aligned(1024))) uint16_t vs[LP * 64];
-  // A head of up to 32 keys passes through registers, its first queries straight into them: there
-  // is little to start on before V is there (128 images of 8 heads of 16 tokens 3.8 us by DMA, 3.5
-  // so; of 64 tokens neither is the faster at every count: 4 heads 4.5 and 4.7, 8 heads 7.2 and
-  // 6.5). Above, the waves' first queries pass through q1. At LP = 128 the three arrays are 40 KB,
-  // four workgroups per CU.
-  constexpr bool kReg = LP <= 32;
+  // A head of up to 64 keys passes through registers, its first queries straight into them after
+  // the rows' stores: there is little to start on before V is there (128 images of 8 heads, us by
+  // DMA and so: 16 tokens 3.8 and 3.45, 64 tokens 7.2 and 6.5; 4 heads of 64 tokens 4.5 and 4.45).
+  // Above, the waves' first queries pass through q1. At LP = 128 the three arrays are 40 KB, four
+  // workgroups per CU.
+  constexpr bool kReg = LP <= 64;
+  constexpr int RP = kAttPitch<kReg>;
+  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * RP];
+  __shared__ __attribute__((aligned(1024))) uint16_t vs[LP * RP];
   __shared__ __attribute__((aligned(1024))) uint16_t q1[kReg ? 8 : 64 * 64];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -180,16 +197,16 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
         vv[r] = ld16(vg + j * S3 + 8 * g);
       }
     }
+#pragma unroll
+    for (int r = 0; r < NF; ++r) {
+      const int c = tid + 256 * r, j = c >> 3, g = c & 7;
+      *reinterpret_cast<uint4*>(ks + att_off<kReg>(j, g)) = kv[r];
+      *reinterpret_cast<uint4*>(vs + att_off<kReg>(j, g)) = vv[r];
+    }
     if (wave * 16 < L) {
       const uint16_t* qr = qg + (wave * 16 + frow) * S3 + 8 * fq;
       qf0 = ld16(qr);
       qf1 = ld16(qr + 32);
-    }
-#pragma unroll
-    for (int r = 0; r < NF; ++r) {
-      const int c = tid + 256 * r, j = c >> 3, g = c & 7;
-      *reinterpret_cast<uint4*>(ks + att_off(j, g)) = kv[r];
-      *reinterpret_cast<uint4*>(vs + att_off(j, g)) = vv[r];
     }
     wait_lgkmcnt0();
   } else {
@@ -204,8 +221,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
   lds_barrier();
   if constexpr (!kReg) {
     const int row = wave * 16 + frow;
-    qf0 = ld16(q1 + att_off(row, fq));
-    qf1 = ld16(q1 + att_off(row, 4 + fq));
+    qf0 = ld16(q1 + att_off<kReg>(row, fq));
+    qf1 = ld16(q1 + att_off<kReg>(row, 4 + fq));
   }
   // V complete; every wave passes this once
   auto wait_v = [&]() __attribute__((always_inline)) {
@@ -226,8 +243,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
       const int row = 16 * kb + frow;
-      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off(row, fq)), qf0, v4f{0.f, 0.f, 0.f, 0.f});
-      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off(row, 4 + fq)), qf1, s[kb]);
+      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off<kReg>(row, fq)), qf0, v4f{0.f, 0.f, 0.f, 0.f});
+      s[kb] = mfma16x16x32_bf16(ld16(ks + att_off<kReg>(row, 4 + fq)), qf1, s[kb]);
     }
     if (L < LP) {
 #pragma unroll
@@ -273,8 +290,8 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
       const uint4 pf = {pk[2 * kk][0], pk[2 * kk][1], pk[2 * kk + 1][0], pk[2 * kk + 1][1]};
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb)
-        o[hb] = mfma16x16x32_bf16(frag_tr(vs, 32 * kk + 4 * fq, 32 * kk + 16 + 4 * fq, hb, frow),
-                                  pf, o[hb]);
+        o[hb] = mfma16x16x32_bf16(
+            frag_tr<kReg>(vs, 32 * kk + 4 * fq, 32 * kk + 16 + 4 * fq, hb, frow), pf, o[hb]);
       if (kk % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
     const float il = 1.0f / l;
@@ -313,26 +330,29 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(const AttnArgs p) {
 template <int LP>
 __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   constexpr int KB = LP >= 256 ? 2 : 1;  // key blocks per wave
-  constexpr int TP = LP + 16;            // dS row pitch (LP = 256, 128: rows 2 bank slots apart)
   constexpr int NCH = LP * 8;            // 16-B chunks of a rows array
   constexpr int NF = (NCH + 511) / 512;  // its transfers per wave, and the parts
   constexpr int OB = NF < 3 ? NF : 3;    // O parts in flight (a fourth reuses the first's room)
-  // A head of up to 32 tokens has nothing to start on early: its rows pass through registers, where
-  // D is formed from them, and K's and V's fragments come from memory (128 images of 4 heads, us:
-  // 16 tokens 4.6 by DMA, 4.4 so; 64 10.4 and 10.9)
-  constexpr bool kReg = LP <= 32;
-  __shared__ __attribute__((aligned(1024))) uint16_t qs[LP * 64];
-  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * 64];
-  __shared__ __attribute__((aligned(1024))) uint16_t gs[LP * 64];
+  // A head of up to 64 tokens has little to start on early: its rows pass through registers, where
+  // D is formed from them, and K's and V's fragments come from memory (128 images of 4 heads, us by
+  // DMA and so: 16 tokens 4.6 and 4.3, 64 tokens 10.4 and 10.4, on three sets of buffers 12.1 and
+  // 11.7)
+  constexpr bool kReg = LP <= 64;
+  constexpr int RP = kAttPitch<kReg>;
+  constexpr int TP = LP + (kReg ? 8 : 16);  // dS row pitch (LP = 256, 128: rows 2 bank slots apart)
+  __shared__ __attribute__((aligned(1024))) uint16_t qs[LP * RP];
+  __shared__ __attribute__((aligned(1024))) uint16_t ks[LP * RP];
+  __shared__ __attribute__((aligned(1024))) uint16_t gs[LP * RP];
   __shared__ __attribute__((aligned(1024))) uint16_t os[OB][kReg ? 8 : 64 * 64];
   __shared__ __attribute__((aligned(1024))) uint16_t dsb[2][32 * TP];
   __shared__ __attribute__((aligned(256))) float lse_s[LP < 64 ? 64 : LP];
   __shared__ float dd_s[LP];
   __shared__ uint32_t red[8];
-  static_assert(2 * 32 * TP >= LP * 64, "V fits the dS buffers");
+  static_assert(kReg || 2 * 32 * TP >= LP * 64, "V fits the dS buffers");
+  static_assert(!kReg || NF == 1, "a chunk per thread");
 
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = kReg ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   const int frow = lane & 15, fq = lane >> 4;
   const int bh = blockIdx.x;
   const int b = bh / p.heads, h = bh - b * p.heads;
@@ -371,16 +391,16 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     const float lse_t = tid < L ? p.lse[(int64_t)bh * L + tid] : __builtin_inff();
     const int j = tid >> 3, g = tid & 7;
     uint4 kv = {0u, 0u, 0u, 0u}, qv = kv, ov = kv, gv = kv;
-    if (j < L) {
+    if (has && j < L) {
       kv = ld16(kg + j * S3 + 8 * g);
       qv = ld16(qg + j * S3 + 8 * g);
       ov = ld16(og + j * C + 8 * g);
       gv = ld16(dg + j * C + 8 * g);
     }
     if (has) {
-      *reinterpret_cast<uint4*>(ks + att_off(j, g)) = kv;
-      *reinterpret_cast<uint4*>(qs + att_off(j, g)) = qv;
-      *reinterpret_cast<uint4*>(gs + att_off(j, g)) = gv;
+      *reinterpret_cast<uint4*>(ks + att_off<kReg>(j, g)) = kv;
+      *reinterpret_cast<uint4*>(qs + att_off<kReg>(j, g)) = qv;
+      *reinterpret_cast<uint4*>(gs + att_off<kReg>(j, g)) = gv;
       float fo[8], fg[8];
       unpack8_bf16(ov, fo);
       unpack8_bf16(gv, fg);
@@ -436,11 +456,13 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     wait_vmcnt<kLater>();
     asm volatile("" ::: "memory");  // (the DMAs' writes are invisible to the compiler)
     form_d(0);
+    wait_lgkmcnt0();
+    asm volatile("" ::: "memory");
+    if (NF > OB && has) dma_o(OB);  // into os[0], whose chunks only their own wave read
+    lds_barrier();                  // K, V, part 0 and its D, lse
+  } else {
+    __syncthreads();
   }
-  wait_lgkmcnt0();
-  asm volatile("" ::: "memory");
-  if (NF > OB && has) dma_o(OB);  // into os[0], whose chunks only their own wave read
-  lds_barrier();                  // K, V, part 0 and its D, lse
 
   // this wave's keys: B fragments of K and V (lane (key frow, k-slice fq): dims 8 fq .. + 7
   // of each 32-wide half)
@@ -450,7 +472,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int hs = 0; hs < 2; ++hs) {
-        const int o = kact ? att_off(kw0 + 16 * kb + frow, 4 * hs + fq) : 0;
+        const int o = kact ? att_off<kReg>(kw0 + 16 * kb + frow, 4 * hs + fq) : 0;
         kf[kb][hs] = ld16(ks + o);
         vf[kb][hs] = ld16(vrow + o);
       }
@@ -460,7 +482,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
   uint4 ktf[LP / 32];
 #pragma unroll
   for (int kk = 0; kk < LP / 32; ++kk)
-    ktf[kk] = frag_tr(ks, 32 * kk + 8 * fq, 32 * kk + 8 * fq + 4, wave & 3, frow);
+    ktf[kk] = frag_tr<kReg>(ks, 32 * kk + 8 * fq, 32 * kk + 8 * fq + 4, wave & 3, frow);
   if constexpr (!kReg) {
     wait_lgkmcnt0();
     lds_barrier();  // V read: the dS buffers are free
@@ -474,7 +496,7 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
     for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
       for (int hs = 0; hs < 2; ++hs) {
-        const int o = att_off(q0 + 16 * sub + frow, 4 * hs + fq);
+        const int o = att_off<kReg>(q0 + 16 * sub + frow, 4 * hs + fq);
         qa[sub][hs] = ld16(qs + o);
         da[sub][hs] = ld16(gs + o);
       }
@@ -542,8 +564,8 @@ __global__ __launch_bounds__(512, 1) void attn_bwd_kernel(const AttnArgs p) {
       const int r1 = q0 + 4 * fq, r2 = q0 + 16 + 4 * fq;
 #pragma unroll
       for (int hb = 0; hb < 4; ++hb) {
-        const uint4 da4 = frag_tr(gs, r1, r2, hb, frow);
-        const uint4 qa4 = frag_tr(qs, r1, r2, hb, frow);
+        const uint4 da4 = frag_tr<kReg>(gs, r1, r2, hb, frow);
+        const uint4 qa4 = frag_tr<kReg>(qs, r1, r2, hb, frow);
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
           dvt[hb][kb] = mfma16x16x32_bf16(da4, pb[kb], dvt[hb][kb]);
